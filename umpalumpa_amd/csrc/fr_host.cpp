@@ -240,7 +240,9 @@ bool box_can_shift(const umpa_fr_settings &s, uint64_t sliceX, uint64_t sliceY)
   const int nb = lookup ? footprint(s) : 4;
   // positions below 8192 round qx - r and qx + r by at most 2^-11 together, inside the
   // 1e-3 margin of `need`, so the bounding box never has more than `need` columns or rows
-  return need <= nb && sliceX >= (uint64_t)nb && sliceY >= (uint64_t)nb && sliceX <= 8192 &&
+  // (radii below 0.5: the box's first column can lie past the voxel by more than the float
+  // difference holds exactly, see gather_box)
+  return need <= nb && s.blobRadius >= 0.5f && sliceX >= (uint64_t)nb && sliceY >= (uint64_t)nb && sliceX <= 8192 &&
          sliceY <= 8192;
 }
 

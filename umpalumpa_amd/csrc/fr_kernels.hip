@@ -24,7 +24,7 @@
 // fr_insert_kernel covers every mode, precision and strategy; fr_insert_staged_kernel, for the
 // exact FP32 lookup strategy, gathers the predicate's hits of several spaces together (see
 // there).
-#include "fr_device.hpp"
+#include "fr_gather.hpp"
 
 namespace umpa {
 
@@ -39,472 +39,6 @@ __host__ __device__ constexpr int fr_waves(int mode, bool half, bool fastMath)
 }
 constexpr int kEdge = 8;             // brick edge: a wave owns 8 x 8 x 8 voxels, a z column per lane
 constexpr int kVox = kEdge * kEdge * kEdge;
-constexpr uint32_t kOutOfRange = 0x7ffff000u;  // buffer offset past every slice: loads read 0
-constexpr uint32_t kBufferConfig = 0x00020000u; // raw buffer descriptor word 3 on gfx9
-
-__device__ __forceinline__ void wave_sync()
-{
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ __forceinline__ unsigned lanes_below(unsigned long long mask)
-{
-  return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
-}
-
-// Raw buffer loads through the LLVM intrinsics.  (The clang builtin for the 64-bit raw buffer
-// load, __builtin_amdgcn_raw_buffer_load_b64, lowers to a single 32-bit load in this toolchain
-// and returns that dword for both halves, so the vector forms are declared directly.)  Every
-// byte offset travels in the vector offset, which the hardware range-checks together with the
-// instruction's immediate offset; the scalar offset is not range-checked, and loads that
-// differed only in it were observed to be merged into one by this compiler, so it stays 0.
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-__device__ f32x2_t raw_buffer_load_f32x2(__amdgpu_buffer_rsrc_t rsrc, uint32_t voffset,
-                                        uint32_t soffset,
-                                        int aux) __asm("llvm.amdgcn.raw.ptr.buffer.load.v2f32");
-__device__ uint32_t raw_buffer_load_u32(__amdgpu_buffer_rsrc_t rsrc, uint32_t voffset,
-                                        uint32_t soffset,
-                                        int aux) __asm("llvm.amdgcn.raw.ptr.buffer.load.i32");
-__device__ f32x4_t raw_buffer_load_f32x4(__amdgpu_buffer_rsrc_t rsrc, uint32_t voffset,
-                                        uint32_t soffset,
-                                        int aux) __asm("llvm.amdgcn.raw.ptr.buffer.load.v4f32");
-__device__ u32x4_t raw_buffer_load_u32x4(__amdgpu_buffer_rsrc_t rsrc, uint32_t voffset,
-                                        uint32_t soffset,
-                                        int aux) __asm("llvm.amdgcn.raw.ptr.buffer.load.v4i32");
-
-// Slice pixel at byte offset `byteOffset` through a bounds-checked buffer resource: offsets at
-// or past the slice end return zero instead of faulting.
-template <bool kHalf>
-__device__ __forceinline__ float2 load_pixel(__amdgpu_buffer_rsrc_t rsrc, uint32_t byteOffset)
-{
-  if constexpr (kHalf) {
-    const uint32_t v = raw_buffer_load_u32(rsrc, byteOffset, 0, 0);
-    return __half22float2(__builtin_bit_cast(__half2, v));
-  } else {
-    const f32x2_t v = raw_buffer_load_f32x2(rsrc, byteOffset, 0, 0);
-    return make_float2(v.x, v.y);
-  }
-}
-
-// A slice pixel as loaded: complex float, or complex half packed in one dword (converted at
-// the multiply-add, which the compiler fuses into a mixed-precision FMA).
-template <bool kHalf> struct Pixel;
-template <> struct Pixel<false> {
-  float2 v;
-  __device__ __forceinline__ float re() const { return v.x; }
-  __device__ __forceinline__ float im() const { return v.y; }
-};
-template <> struct Pixel<true> {
-  uint32_t v;
-  __device__ __forceinline__ float re() const
-  {
-    return __half2float(__builtin_bit_cast(__half, (uint16_t)(v & 0xffffu)));
-  }
-  __device__ __forceinline__ float im() const
-  {
-    return __half2float(__builtin_bit_cast(__half, (uint16_t)(v >> 16)));
-  }
-};
-
-template <bool kHalf>
-__device__ __forceinline__ Pixel<kHalf> load_pixel_raw(__amdgpu_buffer_rsrc_t rsrc,
-                                                       uint32_t byteOffset)
-{
-  Pixel<kHalf> p;
-  if constexpr (kHalf) {
-    p.v = raw_buffer_load_u32(rsrc, byteOffset, 0, 0);
-  } else {
-    const f32x2_t v = raw_buffer_load_f32x2(rsrc, byteOffset, 0, 0);
-    p.v = make_float2(v.x, v.y);
-  }
-  return p;
-}
-
-// kNB consecutive pixels of a slice row starting at byte `voff`, with 16-byte loads (4 FP16 or
-// 2 FP32 pixels each).  Dwords past the slice end read zero.  A load on the slice's last row
-// can straddle the end; the raw buffer's range check then still returns its in-range dwords
-// (the reference's 3 x 6 plane cases, where every last-row load straddles, are bit-exact).
-template <bool kHalf, int kNB>
-__device__ __forceinline__ void load_row(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff,
-                                         Pixel<kHalf> (&px)[kNB])
-{
-  constexpr int kPix = kHalf ? 4 : 8;
-  constexpr int kPer = 16 / kPix;                  // pixels per 16-byte load
-  constexpr int kLoads = (kNB + kPer - 1) / kPer;
-  // (vector elements are named, never indexed by a loop variable: this compiler folded
-  // v[e] in an unrolled loop over e to v[0] for every e, in the 16-byte loads here)
-#pragma unroll
-  for (int q = 0; q < kLoads; ++q) {
-    if constexpr (kHalf) {
-      const u32x4_t v = raw_buffer_load_u32x4(rsrc, voff + (uint32_t)(q * 16), 0, 0);
-      const uint32_t w[4] = { v.x, v.y, v.z, v.w };
-#pragma unroll
-      for (int e = 0; e < kPer; ++e) {
-        const int j = q * kPer + e;
-        if (j < kNB) px[j].v = w[e];
-      }
-    } else {
-      const f32x4_t v = raw_buffer_load_f32x4(rsrc, voff + (uint32_t)(q * 16), 0, 0);
-      const float w[4] = { v.x, v.y, v.z, v.w };
-#pragma unroll
-      for (int e = 0; e < kPer; ++e) {
-        const int j = q * kPer + e;
-        if (j < kNB) px[j].v = make_float2(w[2 * e], w[2 * e + 1]);
-      }
-    }
-  }
-}
-
-// Blob weight of one candidate pixel (kDynamic modes; kLookup reads the LDS table inline).
-template <int kMode, int kOrder>
-__device__ __forceinline__ float blob_weight(float d2, const umpa_fr_constants &c)
-{
-  if constexpr (kMode == kModeFastKaiser) {
-    return kaiser_value_fast(d2, c);
-  } else {
-    return kaiser_value<kOrder>(sqrtf(d2), c.cBlobRadius, c) * c.cIw0;
-  }
-}
-
-struct Contribution {
-  float re, im, w;
-};
-
-// Reference-ordered gather of one voxel-update with generic loops (rows i ascending, columns j
-// ascending, ProcessVoxelBlob fr_cpu_kernels.hpp:104-147).  Used for footprints wider than the
-// unrolled NB x NB box, which only rounding at the blob edge can produce.
-template <int kMode, int kOrder, bool kHalf, bool kFastMath>
-__device__ Contribution gather_generic(const FrJob &a, int nTable, __amdgpu_buffer_rsrc_t rsrc,
-                                       const float *tbl, float qx, float qy, float zSqr, float dw,
-                                       uint32_t sliceOff = 0)
-{
-  const umpa_fr_constants &c = a.c;
-  const float r = c.cBlobRadius, r2 = r * r;
-  int minX = (int)ceilf(qx - r), maxX = (int)floorf(qx + r);
-  int minY = (int)ceilf(qy - r), maxY = (int)floorf(qy + r);
-  minX = minX < 0 ? 0 : minX;
-  minY = minY < 0 ? 0 : minY;
-  maxX = maxX > a.xSize - 1 ? a.xSize - 1 : maxX;
-  maxY = maxY > a.ySize - 1 ? a.ySize - 1 : maxY;
-  Contribution o{ 0.f, 0.f, 0.f };
-  for (int i = minY; i <= maxY; ++i) {
-    float dy = qy - (float)i;
-    float yz = dy * dy + zSqr;
-    if (yz > r2) continue;
-    for (int j = minX; j <= maxX; ++j) {
-      float xD = qx - (float)j;
-      float d2 = xD * xD + yz;
-      if (d2 > r2) continue;
-      float wb;
-      if constexpr (kMode == kModeLookup) {
-        int aux = kFastMath ? (int)__builtin_fmaf(d2, c.cIDeltaSqrt, 0.5f)
-                            : (int)(d2 * c.cIDeltaSqrt + 0.5f);
-        aux = aux > nTable - 1 ? nTable - 1 : aux;
-        wb = tbl[aux];
-      } else {
-        wb = blob_weight<kMode, kOrder>(d2, c);
-      }
-      float weight = wb * dw;
-      float2 f = load_pixel<kHalf>(rsrc, sliceOff + (uint32_t)((i * a.xSize + j) * (kHalf ? 4 : 8)));
-      o.w += weight;
-      if constexpr (kFastMath) {
-        o.re = __builtin_fmaf(f.x, weight, o.re);
-        o.im = __builtin_fmaf(f.y, weight, o.im);
-      } else {
-        o.re += f.x * weight;
-        o.im += f.y * weight;
-      }
-    }
-  }
-  return o;
-}
-
-// load_row for the exact FP32 Kaiser-mode kernels: a row whose 16-byte loads straddle the slice
-// end (byte `sliceBytes` of the resource) is read pixel by pixel.  This compiler merges those
-// pixel loads back into the same 16-byte loads, so both sides load alike; the branch only
-// splits the rows into scheduling regions, the form these kernels were measured and kept in.
-template <bool kHalf, int kNB>
-__device__ __forceinline__ void load_row_regions(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff,
-                                                 uint32_t sliceBytes, Pixel<kHalf> (&px)[kNB])
-{
-  constexpr int kPix = kHalf ? 4 : 8;
-  constexpr int kLoads = (kNB * kPix + 15) / 16;
-  if (voff < sliceBytes && voff + (uint32_t)(kLoads * 16) > sliceBytes) {
-#pragma unroll
-    for (int j = 0; j < kNB; ++j) px[j] = load_pixel_raw<kHalf>(rsrc, voff + (uint32_t)(j * kPix));
-    return;
-  }
-  load_row<kHalf, kNB>(rsrc, voff, px);
-}
-
-// Blob weight of one candidate at squared distance d2, 0 for a candidate the reference skips
-// (d2 > r^2, and d2 = +inf for box positions outside the slice).  Exact strategy: the
-// reference's table position (int)(d2 * cIDeltaSqrt + 0.5); skipped candidates read the LDS
-// copy's zero entry nTable.  Fast math with the table in LDS: a fused position, clamped into
-// the zero entry, so +inf and every d2 past the blob edge weigh 0 without a test.
-template <int kMode, int kOrder, bool kFastMath, bool kTableLds>
-__device__ __forceinline__ float candidate_weight(float d2, float r2, int nTable, const float *tbl,
-                                                  const umpa_fr_constants &c)
-{
-  if constexpr (kFastMath && kMode == kModeLookup && kTableLds) {
-    // The reference's position (int)(d2 * cIDeltaSqrt + 0.5f): the product rounded to float,
-    // then floor(t + 0.5), which v_cvt_rpi_i32_f32 computes in one instruction from the exact
-    // sum; the reference's rounded sum truncates to the same integer for every t >= 0 outside
-    // (0.5 - 2^-25, 0.5) (on the GPU: 2.16 M values, ties k + 0.5 and their neighbours).
-    // Rounding the fused product to the nearest entry instead (one instruction less) moves
-    // entries at rounding boundaries: 4.2e-5 rel-L2 from FRCPU at box 384 with 64 spaces,
-    // whose central voxels carry most of the volume's norm.  Positions past the table and
-    // +inf (saturated to INT_MAX) are clamped into the zero entry nTable, so candidates
-    // outside the blob weigh 0 without a test.
-    const float t = d2 * c.cIDeltaSqrt;
-    int pos;
-    asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(pos) : "v"(t));
-    const uint32_t aux = (uint32_t)pos;
-    typedef __attribute__((address_space(3))) const float lds_float;
-    return ((lds_float *)tbl)[aux < (uint32_t)nTable ? aux : (uint32_t)nTable];
-  } else {
-    const bool in = d2 <= r2;
-    if constexpr (kMode == kModeLookup) {
-      int aux = kFastMath ? (int)__builtin_fmaf(d2, c.cIDeltaSqrt, 0.5f)
-                          : (int)(d2 * c.cIDeltaSqrt + 0.5f);
-      if constexpr (kTableLds) {
-        return tbl[in ? aux : nTable];  // entry nTable of the LDS copy is 0
-      } else {
-        aux = aux > nTable - 1 ? nTable - 1 : aux;
-        return in ? tbl[aux] : 0.f;
-      }
-    } else {
-      return in ? blob_weight<kMode, kOrder>(d2, c) : 0.f;
-    }
-  }
-}
-
-// Branch-free gather of one voxel-update over the NB x NB candidate box around (qx, qy).
-//
-// Exact strategy: candidates the reference skips (outside the blob, outside the slice) read
-// table[nTable] = 0, so with finite slice values they add +-0; the running sums start at +0
-// and never hold -0, so the float results equal the reference's (footprints wider than 4 read
-// skipped pixels past the buffer end, as zeros).  Fast-math strategy (finite slice values):
-// the table index is clamped into the zero entry, so out-of-blob candidates weigh 0 without a
-// test.  Rows are read whole; pixels past the slice end read 0 through the bounds-checked
-// buffer.  With kShift (the caller's instantiation for jobs with FrJob::shiftBox) the box slides
-// inside the slice (see below).
-// Returns false when the footprint is wider than NB.
-template <int kMode, int kOrder, int kNB, bool kHalf, bool kFastMath, bool kUnitWeight, bool kTableLds,
-          bool kShift>
-__device__ __forceinline__ bool gather_box(const FrJob &a, int nTable,
-                                           __amdgpu_buffer_rsrc_t rsrc, const float *tbl,
-                                           float qx, float qy, float zSqr, float dw,
-                                           Contribution &o, uint32_t sliceOff = 0)
-{
-  const umpa_fr_constants &c = a.c;
-  const float r = c.cBlobRadius, r2 = r * r;
-  const float inf = __builtin_inff();
-  int minX = (int)ceilf(qx - r);
-  int minY = (int)ceilf(qy - r);
-  minX = minX < 0 ? 0 : minX;
-  minY = minY < 0 ? 0 : minY;
-  constexpr int kPix = kHalf ? 4 : 8;
-  bool fits = true;
-  float xd2[kNB], yz[kNB];
-  if constexpr (kShift) {
-    // The box slides inside the slice (slices of at least kNB x kNB pixels): it covers the
-    // reference's bounding box [minX, maxX] x [minY, maxY] whenever that has at most kNB
-    // columns and rows (the host sets shiftBox only where floor(2r) + 1 <= kNB), and every
-    // other candidate in it lies farther than r from q, so it weighs 0 (the table's zero
-    // entry; fast math: the clamp, or the last entry within 0.5 / cIDeltaSqrt of r^2), with no
-    // per-candidate masking.
-    minX = minX < a.xSize - kNB ? minX : a.xSize - kNB;
-    minY = minY < a.ySize - kNB ? minY : a.ySize - kNB;
-    const float fx0 = (float)minX, fy0 = (float)minY;
-#pragma unroll
-    for (int jj = 0; jj < kNB; ++jj) {
-      const float xD = qx - (fx0 + (float)jj);
-      xd2[jj] = xD * xD;
-    }
-#pragma unroll
-    for (int ii = 0; ii < kNB; ++ii) {
-      const float dy = qy - (fy0 + (float)ii);
-      yz[ii] = dy * dy + zSqr;
-    }
-  } else {
-    int maxX = (int)floorf(qx + r), maxY = (int)floorf(qy + r);
-    maxX = maxX > a.xSize - 1 ? a.xSize - 1 : maxX;
-    maxY = maxY > a.ySize - 1 ? a.ySize - 1 : maxY;
-    const int nx = maxX - minX, ny = maxY - minY;
-    fits = (nx < kNB) && (ny < kNB);
-    // (float)j == (float)minX + jj exactly for slice indices
-    const float fx0 = (float)minX, fy0 = (float)minY;
-#pragma unroll
-    for (int jj = 0; jj < kNB; ++jj) {
-      const float xD = qx - (fx0 + (float)jj);
-      xd2[jj] = (jj <= nx) ? xD * xD : inf;
-    }
-#pragma unroll
-    for (int ii = 0; ii < kNB; ++ii) {
-      const float dy = qy - (fy0 + (float)ii);
-      yz[ii] = (ii <= ny) ? dy * dy + zSqr : inf;
-    }
-  }
-  const uint32_t rowStride = (uint32_t)(a.xSize * kPix);
-  // sliceOff: the slice's byte offset within the buffer resource (0 when the resource covers
-  // the slice alone)
-  const uint32_t base = sliceOff + (uint32_t)(minY * a.xSize + minX) * kPix;
-  const uint32_t sliceEnd = sliceOff + (uint32_t)(a.sliceElems * kPix);
-  float w = 0.f, vr = 0.f, vi = 0.f;
-  if constexpr (kNB <= 4) {
-    // Whole candidate rows, summed in the reference's order (rows, then columns).  Candidates
-    // outside the blob or the slice weigh exactly 0 (the table's zero entry), so with finite
-    // slice values they add +-0, which changes no running sum (the sums start at +0 and are
-    // never -0): the result equals the reference's skip-the-pixel loop bit for bit.
-    // The exact FP32 lookup kernel issues each row's table reads in a scheduling region of
-    // its own, all four rows before the sums: left to itself this compiler waited on every
-    // table read in turn there (2.70 ms per 1,000-slice chunk at box 256 instead of 1.94 ms).
-    // The fast-math and FP16 kernels run faster with the compiler's own order (1.49 / 1.42 ms
-    // instead of 1.53 / 1.46 ms with such regions).
-    constexpr bool kRegions = !kHalf && !kFastMath && kMode == kModeLookup;
-    float wr[kNB][kNB];
-    if constexpr (kRegions) {
-#pragma unroll
-      for (int ii = 0; ii < kNB; ++ii) {
-#pragma unroll
-        for (int jj = 0; jj < kNB; ++jj)
-          wr[ii][jj] = candidate_weight<kMode, kOrder, kFastMath, kTableLds>(
-            xd2[jj] + yz[ii], r2, nTable, tbl, c);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-#pragma unroll
-    for (int ii = 0; ii < kNB; ++ii) {
-      Pixel<kHalf> px[kNB];
-      // fast-math FP32: a row wholly outside the blob (every candidate weighs 0) reads zeros
-      // from past the slice end instead of its pixels, a quarter of the rows at r = 1.9
-      // (1.480 -> 1.458 ms per 1,000-slice chunk at box 256; the exact kernel's schedule
-      // degrades with it, 1.94 -> 2.11 ms, and FP16 rows gain nothing)
-      constexpr bool kSkipRows = kFastMath && !kHalf;
-      const uint32_t rowOff =
-        (!kSkipRows || yz[ii] <= r2) ? base + ii * rowStride : kOutOfRange;
-      if constexpr (kRegions) {
-        load_row<kHalf, kNB>(rsrc, rowOff, px);
-      } else if constexpr (!kHalf && !kFastMath) {
-        load_row_regions<kHalf, kNB>(rsrc, rowOff, sliceEnd, px);
-      } else {
-        load_row<kHalf, kNB>(rsrc, rowOff, px);
-      }
-#pragma unroll
-      for (int jj = 0; jj < kNB; ++jj) {
-        const float wb = kRegions ? wr[ii][jj]
-                                  : candidate_weight<kMode, kOrder, kFastMath, kTableLds>(
-                                      xd2[jj] + yz[ii], r2, nTable, tbl, c);
-        const float weight = kUnitWeight ? wb : wb * dw;
-        w += weight;
-        if constexpr (kFastMath) {
-          vr = __builtin_fmaf(px[jj].re(), weight, vr);
-          vi = __builtin_fmaf(px[jj].im(), weight, vi);
-        } else {
-          vr += px[jj].re() * weight;
-          vi += px[jj].im() * weight;
-        }
-      }
-    }
-  } else {
-    // footprints wider than 4 keep one load per candidate (whole rows of a 5- or 6-wide box
-    // would not fit the register budget of 16 wavefronts per CU); skipped candidates read past
-    // the slice end (zero) and are masked, except under fast math with the table in LDS, where
-    // their weight is the zero entry
-#pragma unroll
-    for (int ii = 0; ii < kNB; ++ii) {
-#pragma unroll
-      for (int jj = 0; jj < kNB; ++jj) {
-        const float d2 = xd2[jj] + yz[ii];
-        constexpr bool kZeroEntry = kFastMath && kMode == kModeLookup && kTableLds;
-        const bool inb = kZeroEntry ? true : d2 <= r2;
-        const Pixel<kHalf> pix = load_pixel_raw<kHalf>(
-          rsrc, inb ? base + ii * rowStride + (uint32_t)(jj * kPix) : kOutOfRange);
-        float fre = pix.re(), fim = pix.im();
-        const float wb = candidate_weight<kMode, kOrder, kFastMath, kTableLds>(d2, r2, nTable,
-                                                                                 tbl, c);
-        if constexpr (!kZeroEntry) {
-          const bool in = d2 <= r2;
-          fre = in ? fre : 0.f;
-          fim = in ? fim : 0.f;
-        }
-        const float weight = kUnitWeight ? wb : wb * dw;
-        w += weight;
-        if constexpr (kFastMath) {
-          vr = __builtin_fmaf(fre, weight, vr);
-          vi = __builtin_fmaf(fim, weight, vi);
-        } else {
-          vr += fre * weight;
-          vi += fim * weight;
-        }
-      }
-    }
-  }
-  o.re = vr;
-  o.im = vi;
-  o.w = w;
-  return fits;
-}
-
-// The reference's per-voxel predicate for one (voxel, space) pair in blob mode
-// (ProcessVoxelBlob, fr_cpu_kernels.hpp:83-102) plus membership in the reference traversal of
-// the space.  (qx, qy, zSqr) are returned for the gather, qy already shifted to slice rows.
-// With kFma the rotation is evaluated with fused multiply-adds (fewer instructions; q moves by
-// an ulp, which changes which nearly-zero-weight candidates at the blob edge are counted).  The
-// kernels use the reference's separate products: fused, the weights of small volumes drift to
-// about 1e-5 of FRCPU's, the edge of the fast-math strategy's tolerance.
-template <bool kFma>
-__device__ __forceinline__ bool blob_predicate(const umpa_traverse_space &s, const umpa_fr_constants &c,
-                                               int x, int y, int z, float px, float py, float pz,
-                                               bool brickInside, float &qx, float &qy,
-                                               float &zSqr)
-{
-  const float r = c.cBlobRadius;
-  const float(*t)[3] = s.transformInv;
-  float qz;
-  if constexpr (kFma) {
-    qx = __builtin_fmaf(t[0][2], pz, __builtin_fmaf(t[0][1], py, t[0][0] * px));
-    qy = __builtin_fmaf(t[1][2], pz, __builtin_fmaf(t[1][1], py, t[1][0] * px));
-    qz = __builtin_fmaf(t[2][2], pz, __builtin_fmaf(t[2][1], py, t[2][0] * px));
-  } else {
-    qx = t[0][0] * px + t[0][1] * py + t[0][2] * pz;
-    qy = t[1][0] * px + t[1][1] * py + t[1][2] * pz;
-    qz = t[2][0] * px + t[2][1] * py + t[2][2] * pz;
-  }
-  zSqr = qz * qz;
-  // & rather than &&: every test is evaluated, so the record's fields load together
-  bool pass = !(qx < -r) & !(zSqr > r * r);
-  qy += (float)(c.cMaxVolumeIndexYZ / 2);
-  if (!brickInside) {
-    // the sphere test, and the traversal: the column must lie in the AABB's plane orthogonal
-    // to `dir` (both hold for every voxel of a brick that lies inside them: brick_inside)
-    const float dsq = px * px + py * py + pz * pz;
-    pass = pass & !(dsq > s.maxDistanceSqr);
-    if (s.dir == 0) {
-      pass = pass & (x >= s.minX) & (x <= s.maxX) & (y >= s.minY) & (y <= s.maxY);
-    } else if (s.dir == 1) {
-      pass = pass & (x >= s.minX) & (x <= s.maxX) & (z >= s.minZ) & (z <= s.maxZ);
-    } else {
-      pass = pass & (y >= s.minY) & (y <= s.maxY) & (z >= s.minZ) & (z <= s.maxZ);
-    }
-  }
-  // ... and the voxel must lie in the column's slab between the two bounding planes.  A voxel
-  // whose |qz| is at least 0.001 inside the blob radius is between the planes by at least that
-  // much along the column (the axis of the normal's largest component), five times the float
-  // error of the plane evaluation (about 2e-4 at coordinates up to 256), so the floor/ceil
-  // range holds it; only voxels nearer the slab faces take the reference's exact test, whose
-  // two IEEE divisions a wave runs whenever one lane needs it (a band of 0.01 sent about a
-  // quarter of the batches there).
-  if (pass && !(fabsf(qz) <= r - 0.001f)) {
-    pass = visited_blob(s, x, y, z, c.cMaxVolumeIndexX, c.cMaxVolumeIndexYZ);
-  }
-  return pass;
-}
 
 // Per-wave LDS state: running sums of the wave's 8 x 8 x 8 brick and the queue of voxels that
 // pass the slab test for the current space.
@@ -514,21 +48,6 @@ struct WaveScratch {
   float accW[kVox];
   uint16_t queue[kVox];
 };
-
-// Copies a wave-uniform value into scalar registers, dword by dword: a job record read from
-// memory at a uniform address then lives in SGPRs like a kernel argument.
-template <typename T>
-__device__ __forceinline__ T make_uniform(const T &v)
-{
-  static_assert(sizeof(T) % 4 == 0, "dword-sized records only");
-  int w[sizeof(T) / 4];
-  __builtin_memcpy(w, &v, sizeof(T));
-#pragma unroll
-  for (int i = 0; i < (int)(sizeof(T) / 4); ++i) w[i] = __builtin_amdgcn_readfirstlane(w[i]);
-  T out;
-  __builtin_memcpy(&out, w, sizeof(T));
-  return out;
-}
 
 // Element `index` (wave-uniform) of a buffer the kernels only read, through the constant
 // address space: the compiler then reads it with scalar loads into SGPRs instead of 16-byte
@@ -552,6 +71,8 @@ __device__ __forceinline__ T uniform_load(const T *p, int index)
 
 // ---- the brick's steps shared by the insertion kernels ----------------------------------------
 constexpr float kHalfEdge = 0.5f * (kEdge - 1);
+// |qz| <= r (1 + 1e-6) holds wherever the float qz * qz is at most the float r * r
+constexpr float kSlabMargin = 1.f + 1e-6f;
 
 // Brick of the work item and the lane's column of it.
 struct BrickCtx {
@@ -608,24 +129,37 @@ __device__ __forceinline__ bool brick_inside(const BrickCtx &b, const umpa_trave
   return __builtin_amdgcn_readfirstlane((int)(sphere && box)) != 0;
 }
 
-// The brick's running sums start from the volume (or from zero for a split part).
+// The brick's running sums start from the volume (or from zero for a split part).  Levels go
+// four at a time, all their loads in flight before the first is written to LDS.
 template <typename Scratch>
 __device__ __forceinline__ void load_brick(Scratch &ws, const FrJob &a, const BrickCtx &b,
                                            int lane, bool fromZero)
 {
-  for (int k = 0; k < b.nz; ++k) {
-    const int li = k * 64 + lane;
-    float vr = 0.f, vi = 0.f, vw = 0.f;
-    if (!fromZero && b.colIn) {
-      const int64_t gi = ((int64_t)(b.z0 + k) * a.vy + b.y) * a.vx + b.x;
-      const float2 t = reinterpret_cast<const float2 *>(a.volume)[gi];
-      vr = t.x;
-      vi = t.y;
-      vw = a.weights[gi];
+  const int64_t plane = (int64_t)a.vy * a.vx;
+  const int64_t g0 = ((int64_t)b.z0 * a.vy + b.y) * a.vx + b.x;
+  const float2 *vol = reinterpret_cast<const float2 *>(a.volume);
+  const bool read = !fromZero && b.colIn;
+  for (int k0 = 0; k0 < b.nz; k0 += 4) {
+    float2 v[4];
+    float w[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[k] = make_float2(0.f, 0.f);
+      w[k] = 0.f;
+      if (read && k0 + k < b.nz) {
+        v[k] = vol[g0 + (k0 + k) * plane];
+        w[k] = a.weights[g0 + (k0 + k) * plane];
+      }
     }
-    ws.accR[li] = vr;
-    ws.accI[li] = vi;
-    ws.accW[li] = vw;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int li = (k0 + k) * 64 + lane;
+      if (k0 + k < b.nz) {
+        ws.accR[li] = v[k].x;
+        ws.accI[li] = v[k].y;
+        ws.accW[li] = w[k];
+      }
+    }
   }
   wave_sync();
 }
@@ -635,10 +169,12 @@ template <typename Scratch>
 __device__ __forceinline__ void store_brick(const Scratch &ws, const FrJob &a,
                                             const BrickCtx &b, int lane, bool split)
 {
-  for (int k = 0; k < b.nz; ++k) {
-    if (b.colIn) {
+  const int64_t plane = (int64_t)a.vy * a.vx;
+  const int64_t g0 = ((int64_t)b.z0 * a.vy + b.y) * a.vx + b.x;
+  if (b.colIn) {
+    for (int k = 0; k < b.nz; ++k) {
       const int li = k * 64 + lane;
-      const int64_t gi = ((int64_t)(b.z0 + k) * a.vy + b.y) * a.vx + b.x;
+      const int64_t gi = g0 + k * plane;
       if (split) {
         float *vol = reinterpret_cast<float *>(a.volume);
         if (ws.accW[li] != 0.f || ws.accR[li] != 0.f || ws.accI[li] != 0.f) {
@@ -683,31 +219,34 @@ __device__ __forceinline__ bool cull_space(const FrJob &a, const BrickCtx &b, in
          (dir >= 0) & (dir <= 2);
 }
 
-// Phase 1: the slab test q.z^2 <= slab2 of the column's nz voxels; the voxels that pass go to
-// the wave's queue (index k * 64 + lane), their number is returned.  qz = (t20 px + t21 py) +
-// t22 pz is the reference's left-to-right sum, so the shared partial sum changes no bit.
-__device__ __forceinline__ int slab_queue(WaveScratch &ws, const FrJob &a, const BrickCtx &b,
-                                          const umpa_traverse_space &sp, float slab2, int lane)
+// Phase 1: the slab test of the column's nz voxels; the voxels that pass go to the wave's queue
+// behind `pending` entries (index k * 64 + lane, plus `tag`), their number is returned.
+// qz = (t20 px + t21 py) + t22 pz is the reference's left-to-right sum.  `slabR` is a little
+// above the slab's half width, so that |qz| <= slabR holds for every voxel that passes the
+// reference's rounded q.z^2 <= r^2, which phase 2 tests: one compare per level, whose lane mask
+// is the ballot.  (A column outside the volume compares against -1, which nothing passes.)
+template <typename Scratch>
+__device__ __forceinline__ int slab_queue(Scratch &ws, const FrJob &a, const BrickCtx &b,
+                                          const umpa_traverse_space &sp, float slabR, int lane,
+                                          int pending = 0, uint32_t tag = 0)
 {
   const int cyi = a.c.cMaxVolumeIndexYZ / 2;
   const float t20 = sp.transformInv[2][0], t21 = sp.transformInv[2][1],
               t22 = sp.transformInv[2][2];
   const float cz = t20 * b.px + t21 * b.py;
-  // a column outside the volume compares against -1, which no square passes: the test is one
-  // compare whose lane mask is the ballot (with the column flag and-ed in, this compiler turned
-  // the mask into a 0/1 value and back, two more instructions per level: 1.227 -> 1.205 ms per
-  // box-256 chunk under fast math)
-  const float lim = b.colIn ? slab2 : -1.f;
-  int cnt = 0;
+  const float lim = b.colIn ? slabR : -1.f;
+  uint32_t entry = (uint32_t)lane | tag;
+  int end = pending;
   for (int k = 0; k < b.nz; ++k) {
     const float pz = (float)(b.z0 + k - cyi);
     const float qz = cz + t22 * pz;
-    const bool ok = !(qz * qz > lim);
+    const bool ok = !(fabsf(qz) > lim);
     const unsigned long long m = __ballot(ok);
-    if (ok) ws.queue[cnt + (int)lanes_below(m)] = (uint16_t)(k * 64 + lane);
-    cnt += __popcll(m);
+    if (ok) ws.queue[lanes_below(m, (unsigned)end)] = (uint16_t)entry;
+    end += __popcll(m);
+    entry += 64;
   }
-  return cnt;
+  return end - pending;
 }
 
 template <int kMode, int kOrder, int kNB, bool kHalf, bool kFastMath, bool kCount, bool kTableLds,
@@ -758,16 +297,15 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
     const int sEnd = split ? s0 + (int)((int64_t)(s1 - s0) * (part + 1) / parts) : s1;
     const umpa_fr_constants &c = a.c;
     const int cxi = c.cMaxVolumeIndexX / 2, cyi = c.cMaxVolumeIndexYZ / 2;
-    const float r = c.cBlobRadius;
-    const float r2 = r * r;
-    // phase-1 filter on the squared slab coordinate: the reference's own test for blobs; for
-    // the nearest-neighbour traversal the visited voxel lies within 1.5 of the plane
-    const float slab2 = kMode == kModeNearest ? 2.56f : r2;
+    // phase-1 filter on the slab coordinate: the reference's own test for blobs; for the
+    // nearest-neighbour traversal the visited voxel lies within 1.5 of the plane
+    const float slabR = (kMode == kModeNearest ? 1.6f : c.cBlobRadius) * kSlabMargin;
     if (heavy) __builtin_amdgcn_s_setprio(2);
     // the lane owns the z column (x, y, z0 .. z0 + depth - 1) of the brick
     const BrickCtx bk = make_brick(a, bo, lane);
     const int bz = bk.z0;
-    load_brick(ws, a, bk, lane, split);
+    const float ox = (float)(bo.x - cxi), oy = (float)(bo.y - cyi), oz = (float)(bz - cyi);
+    bool loaded = false;  // the sums are read when the first space reaches the brick
     // wave-uniform: the brick's distance from the centre
     const bool earlyCull = __builtin_amdgcn_readfirstlane((int)(bk.dmin > kEarlyCullRadius)) != 0;
     unsigned long long nupd = 0;
@@ -775,6 +313,10 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
       unsigned long long mask = earlyCull
                                   ? __ballot(cull_space<true>(a, bk, base + lane, sEnd))
                                   : __ballot(cull_space<false>(a, bk, base + lane, sEnd));
+      if (mask && !loaded) {
+        load_brick(ws, a, bk, lane, split);
+        loaded = true;
+      }
       // the space's record goes through the wave's LDS slot: one load of 28 dwords by 28
       // lanes, then broadcast reads, instead of seven 16-byte loads of one address by every
       // lane (its 28 SGPRs would not fit beside this kernel's other scalar state). The next
@@ -801,7 +343,7 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
 
         // phase 1: slab test of the column's nz voxels (nz is wave-uniform: shallow bricks
         // run fewer levels)
-        const int cnt = slab_queue(ws, a, bk, sp, slab2, lane);
+        const int cnt = slab_queue(ws, a, bk, sp, slabR, lane);
         if (cnt == 0) continue;
         wave_sync();
         const bool unit = sp.weight == 1.f;
@@ -814,7 +356,9 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
           const int v = act ? (int)ws.queue[item] : 0;
           const int vl = v & 63, vk = v >> 6;
           const int xv = bo.x + (vl & (kEdge - 1)), yv = bo.y + vl / kEdge, zv = bz + vk;
-          const float pxv = (float)(xv - cxi), pyv = (float)(yv - cyi), pzv = (float)(zv - cyi);
+          // small integers in float: exact however they are summed
+          const float pxv = (float)(vl & (kEdge - 1)) + ox, pyv = (float)(vl / kEdge) + oy,
+                      pzv = (float)vk + oz;
           float qx, qy, zs;
           bool hit;
           if constexpr (kMode == kModeNearest) {
@@ -824,7 +368,7 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
             zs = 0.f;
             hit = act && !(dsq > sp.maxDistanceSqr) && !(qx < 0.f) && visited_nearest(sp, xv, yv, zv);
           } else {
-            hit = act && blob_predicate<false>(sp, c, xv, yv, zv, pxv, pyv, pzv, inside, qx, qy, zs);
+            hit = act && blob_predicate<false>(sp, sp.transformInv, c, xv, yv, zv, pxv, pyv, pzv, inside, qx, qy, zs);
           }
           if (hit) {
             Contribution o;
@@ -846,20 +390,8 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
               o.im = f.y * wgt;
               o.w = wgt;
             } else {
-              bool fits;
-              if (unit) {
-                fits = gather_box<kMode, kOrder, kNB, kHalf, kFastMath, true, kTableLds, kShift>(
-                  a, nTable, rsrc, tbl, qx, qy, zs, sp.weight, o);
-              } else {
-                fits = gather_box<kMode, kOrder, kNB, kHalf, kFastMath, false, kTableLds, kShift>(
-                  a, nTable, rsrc, tbl, qx, qy, zs, sp.weight, o);
-              }
-              if (!fits)
-                o = gather_generic<kMode, kOrder, kHalf, kFastMath>(a, nTable, rsrc, tbl, qx, qy, zs, sp.weight);
-              if constexpr (kHalf) {
-                o.re *= scale;
-                o.im *= scale;
-              }
+              o = gather_update<kMode, kOrder, kNB, kHalf, kFastMath, kTableLds, kShift>(
+                a, nTable, rsrc, tbl, qx, qy, zs, sp.weight, unit, scale);
             }
             // volume += contribution, in space order (one item per voxel per space)
             ws.accR[v] = ws.accR[v] + o.re;
@@ -871,7 +403,7 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
         wave_sync();
       }
     }
-    store_brick(ws, a, bk, lane, split);
+    if (loaded) store_brick(ws, a, bk, lane, split);
     if (heavy) __builtin_amdgcn_s_setprio(0);
     if constexpr (kCount) {
       if (lane == 0 && nupd) atomicAdd(l.updates, nupd);
@@ -913,30 +445,6 @@ struct CarryScratch {
 constexpr int kCarryMaxTable =
   (160 * 1024 - kMaxWaves * (int)(sizeof(CarryScratch) + 2 * sizeof(CarrySlot))) / 4 - 1;
 
-// Slab test of the brick's voxels against `sp`, appended to the queue behind `pending`
-// entries with the space's slot in bit 9; returns the number appended.
-__device__ __forceinline__ int slab_queue_carry(CarryScratch &ws, const FrJob &a,
-                                                const BrickCtx &b, const umpa_traverse_space &sp,
-                                                float slab2, int lane, int pending, int slot)
-{
-  const int cyi = a.c.cMaxVolumeIndexYZ / 2;
-  const float t20 = sp.transformInv[2][0], t21 = sp.transformInv[2][1],
-              t22 = sp.transformInv[2][2];
-  const float cz = t20 * b.px + t21 * b.py;
-  const float lim = b.colIn ? slab2 : -1.f;  // as in slab_queue
-  int cnt = 0;
-  const uint32_t tag = (uint32_t)slot << 9;
-  for (int k = 0; k < b.nz; ++k) {
-    const float pz = (float)(b.z0 + k - cyi);
-    const float qz = cz + t22 * pz;
-    const bool ok = !(qz * qz > lim);
-    const unsigned long long m = __ballot(ok);
-    if (ok) ws.queue[pending + cnt + (int)lanes_below(m)] = (uint16_t)((uint32_t)(k * 64 + lane) | tag);
-    cnt += __popcll(m);
-  }
-  return cnt;
-}
-
 // One batch of `n` (1..64) queue entries from `start`: the rest of the predicate, the gather and
 // the accumulation, space by space.
 template <int kNB, bool kHalf, bool kCount, bool kShift>
@@ -955,29 +463,16 @@ __device__ __forceinline__ void carry_batch(CarryScratch &ws, const CarrySlot *s
   const umpa_traverse_space &sp = slt.rec;
   const int vl = v & 63, vk = v >> 6;
   const int xv = bo.x + (vl & (kEdge - 1)), yv = bo.y + vl / kEdge, zv = bz + vk;
-  const float pxv = (float)(xv - cxi), pyv = (float)(yv - cyi), pzv = (float)(zv - cyi);
+  // small integers in float: exact however they are summed
+  const float pxv = (float)(vl & (kEdge - 1)) + (float)(bo.x - cxi),
+              pyv = (float)(vl / kEdge) + (float)(bo.y - cyi), pzv = (float)vk + (float)(bz - cyi);
   float qx, qy, zs;
   const bool hit =
-    act && blob_predicate<false>(sp, c, xv, yv, zv, pxv, pyv, pzv, slt.inside != 0, qx, qy, zs);
+    act && blob_predicate<false>(sp, sp.transformInv, c, xv, yv, zv, pxv, pyv, pzv, slt.inside != 0, qx, qy, zs);
   Contribution o{ 0.f, 0.f, 0.f };
   if (hit) {
-    const uint32_t sliceOff = slt.sliceOff;
-    const float dw = sp.weight;
-    bool fits;
-    if (__all(!hit || dw == 1.f)) {
-      fits = gather_box<kModeLookup, 0, kNB, kHalf, true, true, true, kShift>(a, nTable, rsrc, tbl, qx,
-                                                                       qy, zs, dw, o, sliceOff);
-    } else {
-      fits = gather_box<kModeLookup, 0, kNB, kHalf, true, false, true, kShift>(a, nTable, rsrc, tbl, qx,
-                                                                        qy, zs, dw, o, sliceOff);
-    }
-    if (!fits)
-      o = gather_generic<kModeLookup, 0, kHalf, true>(a, nTable, rsrc, tbl, qx, qy, zs, dw,
-                                                     sliceOff);
-    if constexpr (kHalf) {
-      o.re *= slt.scale;
-      o.im *= slt.scale;
-    }
+    o = gather_update<kModeLookup, 0, kNB, kHalf, true, true, kShift>(
+      a, nTable, rsrc, tbl, qx, qy, zs, sp.weight, false, slt.scale, slt.sliceOff);
   }
   // lane 0 holds the batch's oldest entry: its space is added first
   const int first = __builtin_amdgcn_readfirstlane(tag);
@@ -1036,13 +531,13 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fr_insert_carry_kernel(FrJob j
     const bool split = parts > 1;
     const int sBegin = split ? s0 + (int)((int64_t)(s1 - s0) * part / parts) : s0;
     const int sEnd = split ? s0 + (int)((int64_t)(s1 - s0) * (part + 1) / parts) : s1;
-    const float r = a.c.cBlobRadius;
-    const float slab2 = r * r;
+    const float slabR = a.c.cBlobRadius * kSlabMargin;
     const int cxi = a.c.cMaxVolumeIndexX / 2, cyi = a.c.cMaxVolumeIndexYZ / 2;
     if (heavy) __builtin_amdgcn_s_setprio(2);
     const BrickCtx bk = make_brick(a, bo, lane);
     const int bz = bk.z0;
     load_brick(ws, a, bk, lane, split);
+    bool loaded = false;
     const uint32_t sliceBytes = (uint32_t)(a.sliceElems * kPix);
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
       (void *)a.fft, 0, (int)((uint32_t)a.nProj * sliceBytes), kBufferConfig);
@@ -1055,6 +550,9 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fr_insert_carry_kernel(FrJob j
       unsigned long long mask = earlyCull
                                   ? __ballot(cull_space<true>(a, bk, base + lane, sEnd))
                                   : __ballot(cull_space<false>(a, bk, base + lane, sEnd));
+      if (mask && !loaded) {
+        loaded = true;
+      }
       constexpr int kRecDwords = (int)(sizeof(umpa_traverse_space) / 4);
       const bool recLane = lane < kRecDwords;
       int rec = 0;
@@ -1082,7 +580,8 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fr_insert_carry_kernel(FrJob j
             a.spaces + __builtin_amdgcn_readfirstlane(base + __builtin_ctzll(mask)))[lane];
         const bool ins = brick_inside(bk, slots[slot].rec, cxi, cyi);
         if (lane == 0) slots[slot].inside = ins ? 1 : 0;
-        const int cnt = slab_queue_carry(ws, a, bk, slots[slot].rec, slab2, lane, pending, slot);
+        const int cnt =
+          slab_queue(ws, a, bk, slots[slot].rec, slabR, lane, pending, (uint32_t)slot << 9);
         if (cnt == 0) continue;  // the slot stays free for the next space
         pending += cnt;
         ++pendSpaces;
@@ -1109,7 +608,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fr_insert_carry_kernel(FrJob j
                                       nupd);
       wave_sync();
     }
-    store_brick(ws, a, bk, lane, split);
+    if (loaded) store_brick(ws, a, bk, lane, split);
     if (heavy) __builtin_amdgcn_s_setprio(0);
     if constexpr (kCount) {
       if (lane == 0 && nupd) atomicAdd(l.updates, nupd);
@@ -1152,18 +651,8 @@ __device__ __forceinline__ void staged_gather(const FrJob &a, int nTable,
   const uint32_t off = act ? st.off[e] : 0u, key = act ? st.key[e] : 0u;
   Contribution o{ 0.f, 0.f, 0.f };
   if (act) {
-    // a weight of 1 multiplies nothing; with another weight the product wb * dw is the
-    // reference's, and wb * 1 = wb, so the choice per batch changes no bit
-    bool fits;
-    if (__all(dw == 1.f)) {
-      fits = gather_box<kModeLookup, 0, kNB, false, false, true, true, kShift>(a, nTable, rsrc, tbl, qx,
-                                                                       qy, zs, dw, o, off);
-    } else {
-      fits = gather_box<kModeLookup, 0, kNB, false, false, false, true, kShift>(a, nTable, rsrc, tbl, qx,
-                                                                        qy, zs, dw, o, off);
-    }
-    if (!fits)
-      o = gather_generic<kModeLookup, 0, false, false>(a, nTable, rsrc, tbl, qx, qy, zs, dw, off);
+    o = gather_update<kModeLookup, 0, kNB, false, false, true, kShift>(
+      a, nTable, rsrc, tbl, qx, qy, zs, dw, __all(dw == 1.f), 1.f, off);
   }
   // add space by space (the lowest remaining lane holds the earliest space): within a space
   // every voxel appears once
@@ -1210,7 +699,7 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
     (void *)a.fft, 0, (int)((uint32_t)a.nProj * sliceBytes), kBufferConfig);
   const umpa_fr_constants &c = a.c;
   const int cxi = c.cMaxVolumeIndexX / 2, cyi = c.cMaxVolumeIndexYZ / 2;
-  const float r2 = c.cBlobRadius * c.cBlobRadius;
+  const float slabR = c.cBlobRadius * kSlabMargin;
 
   for (;;) {
     int b = 0;
@@ -1225,7 +714,8 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
     if (heavy) __builtin_amdgcn_s_setprio(2);
     const BrickCtx bk = make_brick(a, bo, lane);
     const int bz = bk.z0;
-    load_brick(ws, a, bk, lane, false);
+    const float ox = (float)(bo.x - cxi), oy = (float)(bo.y - cyi), oz = (float)(bz - cyi);
+    bool loaded = false;  // the sums are read when the first space reaches the brick
     // wave-uniform: the brick's distance from the centre
     const bool earlyCull = __builtin_amdgcn_readfirstlane((int)(bk.dmin > kEarlyCullRadius)) != 0;
     int head = 0, waiting = 0;  // the ring's oldest entry and its number of entries
@@ -1234,6 +724,10 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
       unsigned long long mask = earlyCull
                                   ? __ballot(cull_space<true>(a, bk, base + lane, sEnd))
                                   : __ballot(cull_space<false>(a, bk, base + lane, sEnd));
+      if (mask && !loaded) {
+        load_brick(ws, a, bk, lane, false);
+        loaded = true;
+      }
       while (mask) {
         const int k0 = __builtin_ctzll(mask);
         mask &= mask - 1;
@@ -1242,7 +736,7 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
         const uint32_t sliceOff =
           (uint32_t)__builtin_amdgcn_readfirstlane(sp.projectionIndex) * sliceBytes;
         // phase 1: the slab test, as in fr_insert_kernel
-        const int cnt = slab_queue(ws, a, bk, sp, r2, lane);
+        const int cnt = slab_queue(ws, a, bk, sp, slabR, lane);
         if (cnt == 0) continue;
         wave_sync();
         const bool inside = brick_inside(bk, sp, cxi, cyi);
@@ -1253,10 +747,12 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
           const int v = act ? (int)ws.queue[item] : 0;
           const int vl = v & 63, vk = v >> 6;
           const int xv = bo.x + (vl & (kEdge - 1)), yv = bo.y + vl / kEdge, zv = bz + vk;
-          const float pxv = (float)(xv - cxi), pyv = (float)(yv - cyi), pzv = (float)(zv - cyi);
+          // small integers in float: exact however they are summed
+          const float pxv = (float)(vl & (kEdge - 1)) + ox, pyv = (float)(vl / kEdge) + oy,
+                      pzv = (float)vk + oz;
           float qx, qy, zs;
           const bool hit =
-            act && blob_predicate<false>(sp, c, xv, yv, zv, pxv, pyv, pzv, inside, qx, qy, zs);
+            act && blob_predicate<false>(sp, sp.transformInv, c, xv, yv, zv, pxv, pyv, pzv, inside, qx, qy, zs);
           const unsigned long long hm = __ballot(hit);
           if (hit) {
             const int e = (head + waiting + (int)lanes_below(hm)) & (kStage - 1);
@@ -1285,7 +781,7 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
       staged_gather<kNB, kShift>(a, nTable, rsrc, tbl, ws, st, lane, head, waiting);
       wave_sync();
     }
-    store_brick(ws, a, bk, lane, false);
+    if (loaded) store_brick(ws, a, bk, lane, false);
     if (heavy) __builtin_amdgcn_s_setprio(0);
   }
 }

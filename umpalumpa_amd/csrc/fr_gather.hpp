@@ -265,7 +265,8 @@ __device__ __forceinline__ bool gather_box(const FrJob &a, int nTable,
   if constexpr (kShift) {
     // The box slides inside the slice (slices of at least kNB x kNB pixels): it covers the
     // reference's bounding box [minX, maxX] x [minY, maxY] whenever that has at most kNB
-    // columns and rows (the host sets shiftBox only where floor(2r) + 1 <= kNB), and every
+    // columns and rows (the host sets shiftBox only where floor(2r) + 1 <= kNB, or 2r = kNB for
+    // the widths that test for one column more), and every
     // other candidate in it lies farther than r from q, so it weighs 0 (the table's zero
     // entry; fast math: the clamp, or the last entry within 0.5 / cIDeltaSqrt of r^2), with no
     // per-candidate masking.
@@ -275,6 +276,12 @@ __device__ __forceinline__ bool gather_box(const FrJob &a, int nTable,
     // the host slides boxes for (r >= 0.5, box_can_shift): it is a multiple of q's last place
     // no larger than q, so (q - minX) - jj rounds once, to the same float.
     const float fx = qx - (float)minX, fy = qy - (float)minY;
+    if constexpr (kNB == 3 || kNB == 5) {
+      // where 2r = kNB: column (row) kNB of the box, if the slice has it, lies at distance
+      // kNB - fx, beyond r unless fx >= kNB - r (= r: both edges exactly at distance r)
+      const float edge = (float)kNB - r;
+      fits = (fx < edge || minX >= a.xSize - kNB) & (fy < edge || minY >= a.ySize - kNB);
+    }
 #pragma unroll
     for (int jj = 0; jj < kNB; ++jj) {
       const float xD = fx - (float)jj;

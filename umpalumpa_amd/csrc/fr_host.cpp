@@ -225,15 +225,33 @@ void compute_traverse_space(uint32_t imgSizeX, uint32_t imgSizeY, const float tr
   space.weight = weight;
 }
 
+namespace {
+
+// Columns (and rows) of the blob's bounding box that the kernels' box has to hold: floor(2r) + 1,
+// with a margin for rounding at the edge.  Where 2r is 3 or 5 a voxel has that one more column
+// only if both its outermost pixels lie at distance r to the last bit; the 3- and 5-wide boxes
+// test for that and leave such voxels to the general loop, so 2r columns do (9 candidates
+// instead of 16 at r = 1.5, 25 instead of 36 at r = 2.5: box 384, 256 FP16 slices under D2 at
+// r = 2.5, 4.88 -> 3.98 ms; box 100, 251 slices under C4 at r = 1.5, 1.04 -> 0.99 ms).
+int box_columns(const umpa_fr_settings &s)
+{
+  const double d = 2.0 * (double)s.blobRadius;
+  for (int odd : { 3, 5 })
+    if (std::fabs(d - odd) <= 1e-6) return odd;
+  return (int)std::floor(d + 1e-3) + 1;
+}
+
+}  // namespace
+
 int footprint(const umpa_fr_settings &s)
 {
-  const int nb = (int)std::floor(2.0 * (double)s.blobRadius + 1e-3) + 1;
+  const int nb = box_columns(s);
   return nb < 3 ? 3 : (nb > 6 ? 6 : nb);
 }
 
 bool box_can_shift(const umpa_fr_settings &s, uint64_t sliceX, uint64_t sliceY)
 {
-  const int need = (int)std::floor(2.0 * (double)s.blobRadius + 1e-3) + 1;
+  const int need = box_columns(s);
   // the box width the kernel runs with: the footprint for table lookups, 4 for the other
   // blob modes (which fall back to the general gather past it)
   const bool lookup = s.type != UMPA_FR_FAST && s.interpolation == UMPA_FR_LOOKUP;
@@ -242,8 +260,8 @@ bool box_can_shift(const umpa_fr_settings &s, uint64_t sliceX, uint64_t sliceY)
   // 1e-3 margin of `need`, so the bounding box never has more than `need` columns or rows
   // (radii below 0.5: the box's first column can lie past the voxel by more than the float
   // difference holds exactly, see gather_box)
-  return need <= nb && s.blobRadius >= 0.5f && sliceX >= (uint64_t)nb && sliceY >= (uint64_t)nb && sliceX <= 8192 &&
-         sliceY <= 8192;
+  return need <= nb && s.blobRadius >= 0.5f && sliceX >= (uint64_t)nb &&
+         sliceY >= (uint64_t)nb && sliceX <= 8192 && sliceY <= 8192;
 }
 
 std::vector<BrickCand> brick_candidates(int vx, int vy, int vz, float depthScale)

@@ -24,8 +24,8 @@ void compute_traverse_space(uint32_t imgSizeX, uint32_t imgSizeY, const float tr
                             float weight);
 
 // Width of the unrolled candidate box for blob radius r: floor(2r) + 1 columns (with a margin
-// for rounding at the blob edge), clamped to the kernels' widths 3..6; wider footprints take
-// the generic gather.
+// for rounding at the blob edge; 2r where that is 3 or 5), clamped to the kernels' widths 3..6;
+// wider footprints take the generic gather.
 int footprint(const umpa_fr_settings &s);
 
 // May the candidate box slide inside the slice (no per-candidate masking)?  Slices of at least

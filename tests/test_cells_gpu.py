@@ -1,0 +1,78 @@
+"""The small-problem insertion kernel (cells of 2 x 2 x 2 voxels, eight spaces at a time) where it
+can go wrong: volumes at and around the edges of its cells, blocks and size rule, numbers of
+spaces around its steps of 8, its queue entries of 64 and its tiles of 1,024, every mode and
+footprint.  Exact strategy: bit-identical to the oracle; fast math and FP16: 1e-5 relative L2."""
+import numpy as np
+import pytest
+
+import pyoracle
+from frtools import (problem, quantize_f16, rel_l2, run_hip, run_oracle, settings,
+                     synthetic_slices)
+from umpalumpa_amd import fr as F
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("box,n", [(2, 3), (6, 1), (8, 7), (14, 8), (16, 9), (30, 64), (34, 65),
+                                   (22, 1023), (20, 1025), (12, 2100), (116, 12), (118, 12)])
+def test_sizes(box, n):
+    s = settings()
+    fft, spaces, desc, table = problem(box, n, s, seed=box + n)
+    ov, ow, _ = run_oracle(s, fft, spaces, table, box)
+    v, w, _ = run_hip(s, fft, spaces, desc, table, box)
+    assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()
+    v, w, _ = run_hip(s, fft, spaces, desc, table, box, strategy=F.FR_FAST_MATH)
+    assert rel_l2(v, ov) <= 1e-5 and rel_l2(w, ow) <= 1e-5
+    h, scales, deq = quantize_f16(fft)
+    ov, ow, _ = run_oracle(s, deq, spaces, table, box)
+    v, w, _ = run_hip(s, fft, spaces, desc, table, box, half=(h, scales))
+    assert rel_l2(v, ov) <= 1e-5 and rel_l2(w, ow) <= 1e-5
+
+
+@pytest.mark.parametrize("box,n", [(128, 256), (144, 256)])
+def test_many_spaces_rule(box, n):
+    s = settings(radius=1.2)
+    fft, spaces, desc, table = problem(box, n, s, seed=4)
+    ov, ow, _ = run_oracle(s, fft, spaces, table, box)
+    v, w, _ = run_hip(s, fft, spaces, desc, table, box)
+    assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()
+
+
+@pytest.mark.parametrize("interp,typ,alpha,radius", [
+    (F.FR_LOOKUP, F.FR_PRECISE, 15.0, 0.4), (F.FR_LOOKUP, F.FR_PRECISE, 15.0, 1.0),
+    (F.FR_LOOKUP, F.FR_PRECISE, 15.0, 2.2), (F.FR_LOOKUP, F.FR_PRECISE, 15.0, 2.5),
+    (F.FR_LOOKUP, F.FR_PRECISE, 15.0, 2.9), (F.FR_LOOKUP, F.FR_PRECISE, 15.0, 3.2),
+    (F.FR_DYNAMIC, F.FR_PRECISE, 15.0, 1.9), (F.FR_DYNAMIC, F.FR_PRECISE, 12.0, 2.5),
+    (F.FR_DYNAMIC, F.FR_FAST, 15.0, 1.9)])
+@pytest.mark.parametrize("box", [10, 42])
+def test_modes_and_radii(box, interp, typ, alpha, radius):
+    s = settings(interp, typ, alpha, radius)
+    sym = [np.eye(3), np.diag([-1.0, -1.0, 1.0])]
+    fft, spaces, desc, table = problem(box, 21, s, seed=8, symmetries=sym)
+    spaces["weight"][::3] = 0.5
+    ov, ow, _ = run_oracle(s, fft, spaces, table, box)
+    v, w, _ = run_hip(s, fft, spaces, desc, table, box)
+    assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()
+
+
+def test_accumulates_in_order_and_leaves_the_rest():
+    """Chunks into a volume that holds values, -0 among them: touched voxels take the oracle's
+    bits, the others keep their own; slices of another size than the volume's half plane, a
+    space naming no slice."""
+    box, n = 26, 40
+    s = settings()
+    fft = synthetic_slices(box, n, 3)[:, :, :9]
+    spaces = F.traverse_spaces(pyoracle.uniform_rotations(n, 6), box, s)
+    spaces["projectionIndex"][5] = n + 3
+    desc = F.fr_desc(9, box, n, box + 1, n, 10000)
+    table = F.fill_blob_table(10000, desc, s)
+    rng = np.random.default_rng(1)
+    v0 = rng.standard_normal((box + 1,) * 3 + (2,)).astype(np.float32)
+    v0[rng.random(v0.shape) < 0.3] = -0.0
+    v0 = np.ascontiguousarray(v0).view(np.complex64)[..., 0]
+    w0 = rng.random((box + 1,) * 3).astype(np.float32)
+    keep = np.delete(np.arange(n), 5)
+    ov, ow, _ = run_oracle(s, fft, np.ascontiguousarray(spaces[keep]), table, box, v0, w0)
+    v, w, _ = run_hip(s, np.ascontiguousarray(fft), spaces, desc, table, box, chunks=3, volume=v0,
+                      weights=w0)
+    assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()

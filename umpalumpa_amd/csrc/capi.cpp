@@ -49,8 +49,11 @@ struct umpa_fr_op {
   int nBricks = 0;
   int *dBricksSplit = nullptr; // fast-math schedule: central bricks split over wavefronts
   int nBricksSplit = 0;
-  int *dCounter = nullptr;
+  int *dState = nullptr;       // owns the following:
+  int *dCounter = nullptr;     //   work counter of the brick kernels, then the cell kernel's
   unsigned long long *dUpdates = nullptr;
+  int *dCells = nullptr;       //   small volumes: the blocks of the small-problem kernel
+  int nCells = 0;
   int nb = 0;
   umpa::host::SchedParams params[2];  // schedule knobs: exact / fast-math schedules
 
@@ -58,11 +61,13 @@ struct umpa_fr_op {
   {
     if (dBricks) (void)hipFree(dBricks);
     if (dBricksSplit) (void)hipFree(dBricksSplit);
-    if (dCounter) (void)hipFree(dCounter);
-    if (dUpdates) (void)hipFree(dUpdates);
+    if (dState) (void)hipFree(dState);
+    dState = nullptr;
     dBricks = nullptr;
     dBricksSplit = nullptr;
     nBricksSplit = 0;
+    dCells = nullptr;
+    nCells = 0;
     dCounter = nullptr;
     dUpdates = nullptr;
     nBricks = 0;
@@ -170,16 +175,32 @@ int umpa_fr_init(umpa_fr_op *op, const umpa_fr_desc *desc, const umpa_fr_setting
     op->constants = umpa::host::create_constants(desc->volume.x, desc->volume.y,
                                                  desc->blobTable, *s);
     const int vx = (int)desc->volume.x, vy = (int)desc->volume.y, vz = (int)desc->volume.z;
-    auto bricks = umpa::host::make_brick_schedule(vx, vy, vz, false, op->params[0]);
-    auto split = umpa::host::make_brick_schedule(vx, vy, vz, true, op->params[1]);
+    // both schedules order the same bricks unless their depths were set apart
+    using umpa::host::JobWork;
+    const auto set = umpa::host::make_brick_set(vx, vy, vz, op->params[0].depthScale);
+    const auto bricks = umpa::host::make_schedule({ JobWork{ &set, 0, 1.0 } }, false, op->params[0]);
+    const auto split = op->params[1].depthScale == op->params[0].depthScale
+                         ? umpa::host::make_schedule({ JobWork{ &set, 0, 1.0 } }, true, op->params[1])
+                         : umpa::host::make_brick_schedule(vx, vy, vz, true, op->params[1]);
+    // the counters (work items, blocks, updates; zero) and the blocks of a small volume
+    std::vector<int> state(16, 0);
+    if (umpa::cells_possible(vx, vy, vz)) {
+      const auto cells = umpa::host::make_cell_blocks(vx, vy, vz);
+      op->nCells = (int)(cells.size() / 2);
+      state.insert(state.end(), cells.begin(), cells.end());
+    }
     hipError_t e = upload_bricks(bricks, &op->dBricks);
     if (e == hipSuccess) e = upload_bricks(split, &op->dBricksSplit);
-    if (e == hipSuccess) e = hipMalloc(&op->dCounter, sizeof(int));
-    if (e == hipSuccess) e = hipMalloc(&op->dUpdates, sizeof(unsigned long long));
+    if (e == hipSuccess) e = hipMalloc(&op->dState, state.size() * sizeof(int));
+    if (e == hipSuccess)
+      e = hipMemcpy(op->dState, state.data(), state.size() * sizeof(int), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
       op->release();
       return from_hip(e);
     }
+    op->dCounter = op->dState;
+    op->dUpdates = reinterpret_cast<unsigned long long *>(op->dState + 2);
+    op->dCells = op->nCells > 0 ? op->dState + 16 : nullptr;
     op->nBricksSplit = (int)split.size();
     op->nBricks = (int)bricks.size();
     op->nb = fr_footprint(*s);
@@ -324,13 +345,16 @@ static int fr_execute_impl(umpa_fr_op *op, const void *fft, const float *scales,
   umpa::FrLaunch l{};
   l.items = v.fastMath ? op->dBricksSplit : op->dBricks;
   l.nItems = v.fastMath ? op->nBricksSplit : op->nBricks;
+  l.cells = op->dCells;
+  l.nCells = op->nCells;
+  l.cellCounter = op->dCounter + 1;
   l.counter = op->dCounter;
   l.updates = op->dUpdates;
   l.table = table;
   l.nTable = (int)op->desc.blobTable;
   hipError_t e = hipSuccess;
   if (v.count) e = hipMemsetAsync(op->dUpdates, 0, sizeof(unsigned long long), op->stream);
-  if (e == hipSuccess) e = umpa::prepare_fr_insert(v, l.nTable);
+  if (e == hipSuccess && !umpa::use_cells(a, l, v)) e = umpa::prepare_fr_insert(v, l.nTable);
   if (e == hipSuccess) e = umpa::launch_fr_insert(a, l, v, op->numCUs, op->stream);
   if (e == hipSuccess && v.count) {
     e = hipMemcpyAsync(&op->lastUpdates, op->dUpdates, sizeof(unsigned long long),
@@ -465,6 +489,9 @@ static int fr_autotune_impl(umpa_fr_op *op, const void *fft, const float *scales
       umpa::FrLaunch l{};
       l.items = items;
       l.nItems = (int)bricks.size();
+      l.cells = op->dCells;
+      l.nCells = op->nCells;
+      l.cellCounter = op->dCounter + 1;
       l.counter = op->dCounter;
       l.updates = op->dUpdates;
       l.table = table;
@@ -485,6 +512,12 @@ static int fr_autotune_impl(umpa_fr_op *op, const void *fft, const float *scales
       }
     };
     try {
+      // the default choice where it may be the small-problem kernel, which no knob names
+      if (op->nCells > 0) {
+        umpa::host::SchedParams def;
+        if (!v.fastMath) def.maxParts = 1;
+        time_candidate(def);
+      }
       // schedules (exact: with every kernel knob), then the kernel knobs over the best one
       for (const auto &cand : umpa::host::tuning_candidates(v.fastMath))
         if (e == hipSuccess) time_candidate(cand);

@@ -246,7 +246,7 @@ __device__ __forceinline__ float candidate_weight(float d2, float r2, int nTable
 // inside the slice (see below).
 // Returns false when the footprint is wider than NB.
 template <int kMode, int kOrder, int kNB, bool kHalf, bool kFastMath, bool kUnitWeight, bool kTableLds,
-          bool kShift>
+          bool kShift, int kRows = 0>
 __device__ __forceinline__ bool gather_box(const FrJob &a, int nTable,
                                            __amdgpu_buffer_rsrc_t rsrc, const float *tbl,
                                            float qx, float qy, float zSqr, float dw,
@@ -326,13 +326,13 @@ __device__ __forceinline__ bool gather_box(const FrJob &a, int nTable,
   // values they add +-0, which changes no running sum (the sums start at +0 and are never -0):
   // the result equals the reference's skip-the-pixel loop bit for bit.
   //
-  // The rows go in groups of kGroup: all of a group's pixel loads are issued, then its table
+  // The rows go in groups of kGroup (kRows, or what the brick kernels' registers hold): all of a group's pixel loads are issued, then its table
   // reads, then its sums, each in a scheduling region of its own.  Left to itself this compiler
   // orders the same code by what else the kernel holds in registers: a change elsewhere could
   // make it wait for every row before loading the next (1.42 -> 1.84 ms per 1,000-slice chunk
   // at box 256 under the exact strategy).
   constexpr int kVecs = (kNB * kPix + 15) / 16;          // 16-byte loads per row
-  constexpr int kGroup = kVecs == 1 ? kNB : kVecs == 2 ? (kNB <= 4 ? kNB : 3) : 2;
+  constexpr int kGroup = kRows ? kRows : kVecs == 1 ? kNB : kVecs == 2 ? (kNB <= 4 ? kNB : 3) : 2;
   // wider boxes under the exact strategy mask skipped pixels, whatever their value
   constexpr bool kMask = kNB > 4 && !(kFastMath && kMode == kModeLookup && kTableLds);
 #pragma unroll
@@ -392,7 +392,8 @@ __device__ __forceinline__ bool gather_box(const FrJob &a, int nTable,
 // general loop where the footprint is wider.  The exact strategy multiplies every candidate's
 // weight by dw as the reference does (`unit`, wave-uniform: all weights are 1, which multiply
 // nothing); fast math sums with unit weights and scales the three sums.
-template <int kMode, int kOrder, int kNB, bool kHalf, bool kFastMath, bool kTableLds, bool kShift>
+template <int kMode, int kOrder, int kNB, bool kHalf, bool kFastMath, bool kTableLds, bool kShift,
+          int kRows = 0>
 __device__ __forceinline__ Contribution gather_update(const FrJob &a, int nTable,
                                                       __amdgpu_buffer_rsrc_t rsrc,
                                                       const float *tbl, float qx, float qy,
@@ -401,7 +402,7 @@ __device__ __forceinline__ Contribution gather_update(const FrJob &a, int nTable
 {
   Contribution o;
   if constexpr (kFastMath) {
-    if (!gather_box<kMode, kOrder, kNB, kHalf, kFastMath, true, kTableLds, kShift>(
+    if (!gather_box<kMode, kOrder, kNB, kHalf, kFastMath, true, kTableLds, kShift, kRows>(
           a, nTable, rsrc, tbl, qx, qy, zSqr, 1.f, o, sliceOff))
       o = gather_generic<kMode, kOrder, kHalf, kFastMath>(a, nTable, rsrc, tbl, qx, qy, zSqr, 1.f,
                                                           sliceOff);
@@ -412,10 +413,10 @@ __device__ __forceinline__ Contribution gather_update(const FrJob &a, int nTable
   } else {
     bool fits;
     if (unit) {
-      fits = gather_box<kMode, kOrder, kNB, kHalf, kFastMath, true, kTableLds, kShift>(
+      fits = gather_box<kMode, kOrder, kNB, kHalf, kFastMath, true, kTableLds, kShift, kRows>(
         a, nTable, rsrc, tbl, qx, qy, zSqr, dw, o, sliceOff);
     } else {
-      fits = gather_box<kMode, kOrder, kNB, kHalf, kFastMath, false, kTableLds, kShift>(
+      fits = gather_box<kMode, kOrder, kNB, kHalf, kFastMath, false, kTableLds, kShift, kRows>(
         a, nTable, rsrc, tbl, qx, qy, zSqr, dw, o, sliceOff);
     }
     if (!fits)
@@ -423,6 +424,27 @@ __device__ __forceinline__ Contribution gather_update(const FrJob &a, int nTable
                                                           sliceOff);
   }
   return o;
+}
+
+// ProcessVoxel (fr_cpu_kernels.hpp:50-67): the nearest pixel, weight = space weight.
+template <bool kHalf>
+__device__ __forceinline__ Contribution gather_nearest(const FrJob &a, __amdgpu_buffer_rsrc_t rsrc,
+                                                       float qx, float qy, float dw, float scale,
+                                                       uint32_t sliceOff = 0)
+{
+  int ix = (int)(qx + 0.5f);
+  ix = ix > a.xSize - 1 ? a.xSize - 1 : ix;
+  ix = ix < 0 ? 0 : ix;
+  int iy = (int)(qy + 0.5f + (float)(a.c.cMaxVolumeIndexYZ / 2));
+  iy = iy > a.ySize - 1 ? a.ySize - 1 : iy;
+  iy = iy < 0 ? 0 : iy;
+  const float wgt = 1.f * dw;
+  float2 f = load_pixel<kHalf>(rsrc, sliceOff + (uint32_t)((iy * a.xSize + ix) * (kHalf ? 4 : 8)));
+  if constexpr (kHalf) {
+    f.x *= scale;
+    f.y *= scale;
+  }
+  return { f.x * wgt, f.y * wgt, wgt };
 }
 
 // The reference's per-voxel predicate for one (voxel, space) pair in blob mode
@@ -478,6 +500,23 @@ __device__ __forceinline__ bool blob_predicate(const umpa_traverse_space &s, con
     pass = visited_blob(s, x, y, z, c.cMaxVolumeIndexX, c.cMaxVolumeIndexYZ);
   }
   return pass;
+}
+
+// The blob table and its zero entry into LDS, eight loads of a thread in flight at a time (one
+// at a time, a workgroup's 40 KB took as many round trips to L2 as it has rounds).
+template <int kThreads>
+__device__ __forceinline__ void stage_table(float *dst, const float *__restrict__ src, int n)
+{
+  for (int i0 = threadIdx.x; i0 < n; i0 += 8 * kThreads) {
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = i0 + k * kThreads < n ? src[i0 + k * kThreads] : 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (i0 + k * kThreads < n) dst[i0 + k * kThreads] = v[k];
+  }
+  if (threadIdx.x == 0) dst[n] = 0.f;
+  __syncthreads();
 }
 
 // Copies a wave-uniform value into scalar registers, dword by dword: a job record read from

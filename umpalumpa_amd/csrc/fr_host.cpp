@@ -458,6 +458,48 @@ std::vector<BrickOrigin> make_brick_schedule(int vx, int vy, int vz, bool splitH
   return make_schedule({ JobWork{ &set, 0, 1.0 } }, splitHeavy, sp);
 }
 
+std::vector<int> make_cell_blocks(int vx, int vy, int vz)
+{
+  const int cx = (vx - 1) / 2, cy = (vy - 1) / 2;
+  // a wavefront's steps per space and block: a random plane passes within w of a point at
+  // distance R with probability ~w/R, times the wavefront's cells
+  auto cost = [&](int x, int y, int z, int e) {
+    const float h = 0.5f * (float)(e - 1);
+    const float dx = x + h - cx, dy = y + h - cy, dz = z + h - cy;
+    const float R = std::sqrt(dx * dx + dy * dy + dz * dz), w = 3.f;
+    return (e == 4 ? 1.f : 8.f) * w / std::max(R, w);
+  };
+  struct Block {
+    int x, y, z, e, bin;
+  };
+  std::vector<Block> blocks;
+  constexpr int kBins = 256;  // a counting sort by cost
+  std::vector<uint32_t> start(kBins + 1, 0);
+  auto add = [&](int x, int y, int z, int e) {
+    if (x >= vx || y >= vy || z >= vz) return;
+    const int bin = kBins - 1 - std::min(kBins - 1, (int)(cost(x, y, z, e) * (kBins - 1)));
+    blocks.push_back({ x, y, z, e, bin });
+    ++start[(size_t)bin + 1];
+  };
+  for (int z = 0; z < vz; z += 8)
+    for (int y = 0; y < vy; y += 8)
+      for (int x = 0; x < vx; x += 8) {
+        if (cost(x, y, z, 8) <= 0.7f) {
+          add(x, y, z, 8);
+          continue;
+        }
+        for (int i = 0; i < 8; ++i) add(x + 4 * (i & 1), y + 4 * ((i >> 1) & 1), z + 4 * (i >> 2), 4);
+      }
+  for (int i = 0; i < kBins; ++i) start[(size_t)i + 1] += start[(size_t)i];
+  std::vector<int> out(2 * blocks.size());
+  for (const Block &b : blocks) {
+    const size_t i = start[(size_t)b.bin]++;
+    out[2 * i] = b.x | b.y << 16;
+    out[2 * i + 1] = b.z | b.e << 16;
+  }
+  return out;
+}
+
 int symmetry_operators(char family, int n, double *out, uint32_t cap, uint32_t *count)
 {
   // C_n: rotations by 2 pi k / n about z.  D_n: C_n and the n two-fold rotations about the

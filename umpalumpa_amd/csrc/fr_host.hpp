@@ -91,6 +91,10 @@ void make_schedule(const std::vector<JobWork> &jobs, bool splitHeavy, const Sche
 std::vector<BrickOrigin> make_brick_schedule(int vx, int vy, int vz, bool splitHeavy,
                                              const SchedParams &sp = SchedParams());
 
+// The 4 x 4 x 4 blocks covering a volume, nearest to the centre first, two ints each: x | y << 16
+// and z (the small-problem kernel's work items).
+std::vector<int> make_cell_blocks(int vx, int vy, int vz);
+
 // Persisted tuning results: one "key depthScale priority maxParts splitAt kernel tableGlobal
 // boxFixed ms" line per key in $UMPA_TUNING_DIR/fr_tuning.txt (default
 // $HOME/.cache/umpalumpa_amd); keys carry a format tag, so lines of another format are skipped.

@@ -21,6 +21,8 @@
 // Workgroups are persistent (one per CU: 16 or 12 wavefronts sharing the blob table in LDS)
 // and take bricks from a counter, most central (heaviest) first.
 //
+// Small volumes take the cell kernel (fr_cells.hip) instead; see use_cells().
+//
 // fr_insert_kernel covers every mode, precision and strategy; fr_insert_staged_kernel, for the
 // exact FP32 lookup strategy, gathers the predicate's hits of several spaces together (see
 // there).
@@ -260,9 +262,7 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
   __shared__ umpa_traverse_space s_space[kWaves];  // the space the wave works on
   const int nTable = l.nTable;
   if constexpr (kMode == kModeLookup && kTableLds) {
-    for (int i = threadIdx.x; i < nTable; i += kThreads) s_table[i] = l.table[i];
-    if (threadIdx.x == 0) s_table[nTable] = 0.f;
-    __syncthreads();
+    stage_table<kThreads>(s_table, l.table, nTable);
   }
   const float *tbl = (kMode == kModeLookup && kTableLds) ? s_table : l.table;
   const int lane = threadIdx.x & 63;
@@ -373,22 +373,7 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
           if (hit) {
             Contribution o;
             if constexpr (kMode == kModeNearest) {
-              // ProcessVoxel (fr_cpu_kernels.hpp:50-67): nearest pixel, weight = space weight
-              int ix = (int)(qx + 0.5f);
-              ix = ix > a.xSize - 1 ? a.xSize - 1 : ix;
-              ix = ix < 0 ? 0 : ix;
-              int iy = (int)(qy + 0.5f + (float)(c.cMaxVolumeIndexYZ / 2));
-              iy = iy > a.ySize - 1 ? a.ySize - 1 : iy;
-              iy = iy < 0 ? 0 : iy;
-              const float wgt = 1.f * sp.weight;
-              float2 f = load_pixel<kHalf>(rsrc, (uint32_t)((iy * a.xSize + ix) * kPix));
-              if constexpr (kHalf) {
-                f.x *= scale;
-                f.y *= scale;
-              }
-              o.re = f.x * wgt;
-              o.im = f.y * wgt;
-              o.w = wgt;
+              o = gather_nearest<kHalf>(a, rsrc, qx, qy, sp.weight, scale);
             } else {
               o = gather_update<kMode, kOrder, kNB, kHalf, kFastMath, kTableLds, kShift>(
                 a, nTable, rsrc, tbl, qx, qy, zs, sp.weight, unit, scale);
@@ -502,9 +487,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fr_insert_carry_kernel(FrJob j
   __shared__ CarryScratch s_wave[kWaves];
   __shared__ CarrySlot s_slot[kWaves][2];
   const int nTable = l.nTable;
-  for (int i = threadIdx.x; i < nTable; i += kThreads) s_table[i] = l.table[i];
-  if (threadIdx.x == 0) s_table[nTable] = 0.f;
-  __syncthreads();
+  stage_table<kThreads>(s_table, l.table, nTable);
   const float *tbl = s_table;
   const int lane = threadIdx.x & 63;
   const int wv = threadIdx.x >> 6;
@@ -685,9 +668,7 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
   __shared__ WaveScratch s_wave[kWaves];
   __shared__ WaveStage s_stage[kWaves];
   const int nTable = l.nTable;
-  for (int i = threadIdx.x; i < nTable; i += kThreads) s_table[i] = l.table[i];
-  if (threadIdx.x == 0) s_table[nTable] = 0.f;
-  __syncthreads();
+  stage_table<kThreads>(s_table, l.table, nTable);
   const float *tbl = s_table;
   const int lane = threadIdx.x & 63;
   WaveScratch &ws = s_wave[threadIdx.x >> 6];
@@ -936,6 +917,29 @@ hipError_t prepare_fr_insert(const FrVariant &v, int nTable)
   return e;
 }
 
+// Does this launch run the small-problem kernel?  The brick kernels take as long as the central
+// brick's chain of spaces (about 1 us each; 2.7 with the blob evaluated) however small the
+// volume, the cell kernel about 0.03 us per space and 1,000 voxels of a plane plus 0.05 us per
+// 1,000 voxels.  Measured (us, bricks / cells, r 1.9): exact, 400 slices: box 40 448 / 85, 64
+// 388 / 106, 100 463 / 187, 128 404 / 283, 144 415 / 357, 160 429 / 442; 100 slices: 100
+// 151 / 96, 112 137 / 122, 128 154 / 161, 144 171 / 210; fast math, whose schedules split the
+// central bricks, 1,500 slices: 80 787 / 402, 100 771 / 554, 112 728 / 655, 128 709 / 828; FP16
+// 112 816 / 614, 128 793 / 775; blob evaluated, 400 slices: 100 1205 / 330, 160 1074 / 759, 200
+// 1223 / 1224, 50 slices: 100 190 / 129, 128 196 / 209; nearest, 400 slices: 128 386 / 263, 160
+// 437 / 427.  So: up to 117^3 voxels always; without fast math, from 256 spaces, up to 145^3
+// (161^3 with the blob evaluated).
+bool use_cells(const FrJob &job, const FrLaunch &l, const FrVariant &v)
+{
+  if (l.nCells <= 0 || v.batched || v.count || v.kernel != kKernelAuto || v.tableGlobal) return false;
+  if (v.mode == kModeLookup && l.nTable > kMaxLdsTable) return false;  // the table stays global
+  if (!carry_fits(job, v.half)) return false;  // the chunk's slices need one buffer resource each
+  const int64_t voxels = (int64_t)job.vx * job.vy * job.vz;
+  auto cube = [](int64_t n) { return n * n * n; };
+  if (voxels <= cube(117)) return true;
+  const bool blob = v.mode == kModeFastKaiser || v.mode == kModePreciseKaiser;
+  return !v.fastMath && job.spaceEnd - job.spaceBegin >= 256 && voxels <= cube(blob ? 161 : 145);
+}
+
 hipError_t launch_fr_insert(const FrJob &job, const FrLaunch &l, const FrVariant &v0, int numCUs,
                             hipStream_t st)
 {
@@ -943,6 +947,7 @@ hipError_t launch_fr_insert(const FrJob &job, const FrLaunch &l, const FrVariant
   // job of the launch does
   FrVariant v = v0;
   if (!v.batched) v.shift = job.shiftBox != 0;
+  if (use_cells(job, l, v)) return launch_fr_cells(job, l, v, numCUs, st);
   const void *k = pick_kernel(v, l.nTable);
   if (!k) return hipErrorInvalidValue;
   const size_t shmem = table_in_lds(v, l.nTable) ? (size_t)(l.nTable + 1) * sizeof(float) : 0;

@@ -43,6 +43,9 @@ struct FrLaunch {
   int nTable;
   int waveItems;        // items per wave before it leaves (0: until the items run out)
   int maxBlocks;        // persistent launches: at most this many workgroups (0: one per CU)
+  const int *cells;     // int2 {x | y << 16, z | edge << 16} per block of the volume, heaviest first
+  int nCells;           // (plain launches whose host keeps the list; 0: none)
+  int *cellCounter;     // blocks claimed so far: zero between launches
 };
 
 // Largest blob table kept in LDS (floats); batches require it there.
@@ -76,6 +79,17 @@ hipError_t prepare_fr_insert(const FrVariant &v, int nTable);
 // Enqueues the counter reset and the insertion kernel on `st`.
 hipError_t launch_fr_insert(const FrJob &job, const FrLaunch &l, const FrVariant &v, int numCUs,
                             hipStream_t st);
+
+// May a volume of these extents run the small-problem kernel (its host then keeps the block list)?
+inline bool cells_possible(int vx, int vy, int vz)
+{
+  return (int64_t)vx * vy * vz <= (int64_t)161 * 161 * 161 && vx < 65536 && vy < 65536 && vz < 32768;
+}
+// Does the launch run the small-problem kernel (which needs no `prepare`)?
+bool use_cells(const FrJob &job, const FrLaunch &l, const FrVariant &v);
+// The small-problem kernel (fr_cells.hip) over l.cells.
+hipError_t launch_fr_cells(const FrJob &job, const FrLaunch &l, const FrVariant &v, int numCUs,
+                           hipStream_t st);
 
 // Allocation-free insertion: the work counter and the work items live in a static device
 // array of kNoAllocScratchBytes per GPU (a 256-byte header, then int4 items).  `items` is the

@@ -50,7 +50,7 @@ struct umpa_fr_op {
   int *dBricksSplit = nullptr; // fast-math schedule: central bricks split over wavefronts
   int nBricksSplit = 0;
   int *dState = nullptr;       // owns the following:
-  int *dCounter = nullptr;     //   work counter of the brick kernels, then the cell kernel's
+  int *dCounter = nullptr;     //   work counter of the brick kernels; the cell kernel's 128 bytes on
   unsigned long long *dUpdates = nullptr;
   int *dCells = nullptr;       //   small volumes: the blocks of the small-problem kernel
   int nCells = 0;
@@ -182,8 +182,9 @@ int umpa_fr_init(umpa_fr_op *op, const umpa_fr_desc *desc, const umpa_fr_setting
     const auto split = op->params[1].depthScale == op->params[0].depthScale
                          ? umpa::host::make_schedule({ JobWork{ &set, 0, 1.0 } }, true, op->params[1])
                          : umpa::host::make_brick_schedule(vx, vy, vz, true, op->params[1]);
-    // the counters (work items, blocks, updates; zero) and the blocks of a small volume
-    std::vector<int> state(16, 0);
+    // the counters (work items, blocks, updates; zero) and the blocks of a small volume, each
+    // counter in 128-byte lines of its own: the blocks beside it made box 32 take 19 us, not 15
+    std::vector<int> state(96, 0);
     if (umpa::cells_possible(vx, vy, vz)) {
       const auto cells = umpa::host::make_cell_blocks(vx, vy, vz);
       op->nCells = (int)(cells.size() / 2);
@@ -199,8 +200,8 @@ int umpa_fr_init(umpa_fr_op *op, const umpa_fr_desc *desc, const umpa_fr_setting
       return from_hip(e);
     }
     op->dCounter = op->dState;
-    op->dUpdates = reinterpret_cast<unsigned long long *>(op->dState + 2);
-    op->dCells = op->nCells > 0 ? op->dState + 16 : nullptr;
+    op->dUpdates = reinterpret_cast<unsigned long long *>(op->dState + 64);
+    op->dCells = op->nCells > 0 ? op->dState + 96 : nullptr;
     op->nBricksSplit = (int)split.size();
     op->nBricks = (int)bricks.size();
     op->nb = fr_footprint(*s);
@@ -347,7 +348,7 @@ static int fr_execute_impl(umpa_fr_op *op, const void *fft, const float *scales,
   l.nItems = v.fastMath ? op->nBricksSplit : op->nBricks;
   l.cells = op->dCells;
   l.nCells = op->nCells;
-  l.cellCounter = op->dCounter + 1;
+  l.cellCounter = op->dCounter + 32;
   l.counter = op->dCounter;
   l.updates = op->dUpdates;
   l.table = table;
@@ -491,7 +492,7 @@ static int fr_autotune_impl(umpa_fr_op *op, const void *fft, const float *scales
       l.nItems = (int)bricks.size();
       l.cells = op->dCells;
       l.nCells = op->nCells;
-      l.cellCounter = op->dCounter + 1;
+      l.cellCounter = op->dCounter + 32;
       l.counter = op->dCounter;
       l.updates = op->dUpdates;
       l.table = table;

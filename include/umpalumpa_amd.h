@@ -265,9 +265,9 @@ typedef struct umpa_fr_sched_params {
 
 enum {
   UMPA_FR_KERNEL_AUTO = 0,   /* staged for UMPA_FR_EXACT, carried for fast-math FP32, else pair;
-                                small volumes of a plain operation (up to 117^3 voxels, more for
-                                exact chunks of 256 spaces and up) run eight spaces at a time in
-                                cells of 2 x 2 x 2 voxels, whatever the schedule knobs */
+                                small volumes of a plain operation (up to 129^3 voxels, by mode
+                                and number of spaces) run eight spaces at a time in cells of
+                                2 x 2 x 2 voxels, whatever the schedule knobs */
   UMPA_FR_KERNEL_PAIR = 1,   /* one queue of slab voxels per (brick, space), 16 or 12 waves */
   UMPA_FR_KERNEL_CARRY = 2,  /* queues carried across spaces (fast math, footprint 3-4) */
   UMPA_FR_KERNEL_STAGED = 3  /* cross-space ring of entries (exact FP32, footprint 3-4) */

@@ -76,3 +76,85 @@ def test_accumulates_in_order_and_leaves_the_rest():
     v, w, _ = run_hip(s, np.ascontiguousarray(fft), spaces, desc, table, box, chunks=3, volume=v0,
                       weights=w0)
     assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()
+
+
+@pytest.mark.parametrize("box", [104, 130, 160, 162, 198, 224, 226])
+@pytest.mark.parametrize("kernel", [F.FR_KERNEL_AUTO, F.FR_KERNEL_PAIR])
+def test_core_of_larger_volumes(box, kernel):
+    """The exact strategy takes the centre of volumes up to 225^3 as cells: both exact kernels,
+    table in LDS and global, the update count, boxes around the lines of the core's radius."""
+    s = settings(radius=1.5 if box % 4 else 1.9)
+    fft, spaces, desc, table = problem(box, 11, s, seed=box)
+    ov, ow, updates = run_oracle(s, fft, spaces, table, box)
+    sched = F.SchedParams(1.0, 1, 1, 0.5, kernel, 1 if box == 162 else 0, 0)
+    for count in (False, True):
+        v, w, n = run_hip(s, fft, spaces, desc, table, box, sched=sched, count=count)
+        assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()
+    assert n == updates
+
+
+@pytest.mark.parametrize("typ", [F.FR_PRECISE, F.FR_FAST])
+def test_core_without_table(typ):
+    s = settings(F.FR_DYNAMIC, typ, 15.0, 1.9)
+    fft, spaces, desc, table = problem(134, 9, s, seed=2)
+    ov, ow, _ = run_oracle(s, fft, spaces, table, 134)
+    v, w, _ = run_hip(s, fft, spaces, desc, table, 134)
+    assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()
+
+
+def test_no_core_where_slices_exceed_one_resource():
+    """A chunk of more than 2 GiB of slices (13,400 of 101 x 200) gives the small chunk's bits."""
+    import torch
+    box = 200
+    s = settings()
+    fft, spaces, _, table = problem(box, 3, s, seed=17)
+    dev = torch.device("cuda:0")
+    d_tab = torch.from_numpy(table).to(dev)
+    d_sp = torch.from_numpy(np.ascontiguousarray(spaces).view(np.uint8)).to(dev)
+    big = torch.zeros((13400,) + fft.shape[1:], dtype=torch.complex64, device=dev)
+    big[:3] = torch.from_numpy(np.ascontiguousarray(fft)).to(dev)
+    out = []
+    for buf in (big[:3], big):
+        desc = F.fr_desc(fft.shape[2], fft.shape[1], buf.shape[0], box + 1, len(spaces), table.size)
+        op = F.FourierReconstruction(0)
+        assert op.init(desc, s)
+        vol = torch.zeros((box + 1,) * 3, dtype=torch.complex64, device=dev)
+        wts = torch.zeros((box + 1,) * 3, dtype=torch.float32, device=dev)
+        assert op.execute(buf, vol, wts, d_sp, d_tab)
+        op.synchronize()
+        out.append((vol.cpu().numpy().tobytes(), wts.cpu().numpy().tobytes()))
+    assert out[0] == out[1]
+
+
+@pytest.mark.parametrize("items", [1, 2, 5, 1000])
+@pytest.mark.parametrize("strategy", [F.FR_EXACT, F.FR_FAST_MATH])
+def test_dealt_items_cover_every_brick(items, strategy):
+    """Bounded launches deal their items out by workgroup: sizes around one group of workgroups,
+    a last group that is short, fewer items than a workgroup's share."""
+    import torch
+    dev = torch.device("cuda:0")
+    s = settings()
+    jobs, ref = [], []
+    for box, n in ((8, 5), (66, 6), (136, 4)):
+        fft, spaces, desc, table = problem(box, n, s, seed=box)
+        jobs.append(F.BatchJob(torch.from_numpy(fft).to(dev),
+                               torch.zeros((box + 1,) * 3, dtype=torch.complex64, device=dev),
+                               torch.zeros((box + 1,) * 3, dtype=torch.float32, device=dev),
+                               torch.from_numpy(spaces.view(np.uint8)).to(dev), s,
+                               torch.from_numpy(table).to(dev)))
+        ref.append(run_oracle(s, fft, spaces, table, box)[:2])
+    for chosen in ([0], [0, 1, 2]):
+        b = F.FRBatch(0)
+        b.set_wave_items(items)
+        for k in chosen:
+            jobs[k].volume.zero_()
+            jobs[k].weights.zero_()
+        part = [jobs[k] for k in chosen]
+        b.step(part, [0] * len(part), [j.n_spaces for j in part], strategy)
+        b.synchronize()
+        for k in chosen:
+            v, w = jobs[k].volume.cpu().numpy(), jobs[k].weights.cpu().numpy()
+            if strategy == F.FR_EXACT:
+                assert v.tobytes() == ref[k][0].tobytes() and w.tobytes() == ref[k][1].tobytes()
+            else:
+                assert rel_l2(v, ref[k][0]) <= 1e-5 and rel_l2(w, ref[k][1]) <= 1e-5

@@ -54,6 +54,8 @@ struct umpa_fr_op {
   unsigned long long *dUpdates = nullptr;
   int *dCells = nullptr;       //   small volumes: the blocks of the small-problem kernel
   int nCells = 0;
+  int *dCore = nullptr;        //   the core's cells (exact launches)
+  int nCore = 0;
   int nb = 0;
   umpa::host::SchedParams params[2];  // schedule knobs: exact / fast-math schedules
 
@@ -68,6 +70,8 @@ struct umpa_fr_op {
     nBricksSplit = 0;
     dCells = nullptr;
     nCells = 0;
+    dCore = nullptr;
+    nCore = 0;
     dCounter = nullptr;
     dUpdates = nullptr;
     nBricks = 0;
@@ -160,6 +164,25 @@ int umpa_fr_create(umpa_fr_op **op, int device, void *stream)
   return UMPA_OK;
 }
 
+// The radius of the core that an operation's exact launches take as cells: none where a chunk's
+// slices do not fit the one buffer resource that cells read them through.
+static float op_core(const umpa_fr_desc &d)
+{
+  if (d.fft.n * d.fft.x * d.fft.y * 8 > 0x7fff0000ull) return 0.f;
+  if (d.volume.x > 65535 || d.volume.y > 32767) return 0.f;
+  return umpa::host::core_radius((int)d.volume.x, (int)d.volume.y, (int)d.volume.z);
+}
+
+// The work items of an initialised operation's launches under knobs `sp`: every brick, split over
+// wavefronts, for fast math; for the exact strategy, the bricks outside the core.
+static std::vector<umpa::host::BrickOrigin> op_schedule(const umpa_fr_op *op, bool split,
+                                                        const umpa::host::SchedParams &sp)
+{
+  const umpa_fr_desc &d = op->desc;
+  return umpa::host::make_brick_schedule((int)d.volume.x, (int)d.volume.y, (int)d.volume.z, split,
+                                         sp, split ? 0.f : op_core(d));
+}
+
 int umpa_fr_init(umpa_fr_op *op, const umpa_fr_desc *desc, const umpa_fr_settings *s)
 {
   if (!op || !desc || !s) return UMPA_ERR_INVALID_ARG;
@@ -175,19 +198,19 @@ int umpa_fr_init(umpa_fr_op *op, const umpa_fr_desc *desc, const umpa_fr_setting
     op->constants = umpa::host::create_constants(desc->volume.x, desc->volume.y,
                                                  desc->blobTable, *s);
     const int vx = (int)desc->volume.x, vy = (int)desc->volume.y, vz = (int)desc->volume.z;
-    // both schedules order the same bricks unless their depths were set apart
-    using umpa::host::JobWork;
-    const auto set = umpa::host::make_brick_set(vx, vy, vz, op->params[0].depthScale);
-    const auto bricks = umpa::host::make_schedule({ JobWork{ &set, 0, 1.0 } }, false, op->params[0]);
-    const auto split = op->params[1].depthScale == op->params[0].depthScale
-                         ? umpa::host::make_schedule({ JobWork{ &set, 0, 1.0 } }, true, op->params[1])
-                         : umpa::host::make_brick_schedule(vx, vy, vz, true, op->params[1]);
+    const auto bricks = op_schedule(op, false, op->params[0]);
+    const auto split = op_schedule(op, true, op->params[1]);
     // the counters (work items, blocks, updates; zero) and the blocks of a small volume, each
     // counter in 128-byte lines of its own: the blocks beside it made box 32 take 19 us, not 15
     std::vector<int> state(96, 0);
     if (umpa::cells_possible(vx, vy, vz)) {
       const auto cells = umpa::host::make_cell_blocks(vx, vy, vz);
       op->nCells = (int)(cells.size() / 2);
+      state.insert(state.end(), cells.begin(), cells.end());
+    }
+    if (const float core = op_core(*desc); core > 0.f) {
+      const auto cells = umpa::host::core_cells(vx, vy, vz, core);
+      op->nCore = (int)(cells.size() / 2);
       state.insert(state.end(), cells.begin(), cells.end());
     }
     hipError_t e = upload_bricks(bricks, &op->dBricks);
@@ -202,6 +225,7 @@ int umpa_fr_init(umpa_fr_op *op, const umpa_fr_desc *desc, const umpa_fr_setting
     op->dCounter = op->dState;
     op->dUpdates = reinterpret_cast<unsigned long long *>(op->dState + 64);
     op->dCells = op->nCells > 0 ? op->dState + 96 : nullptr;
+    op->dCore = op->nCore > 0 ? op->dState + 96 + 2 * op->nCells : nullptr;
     op->nBricksSplit = (int)split.size();
     op->nBricks = (int)bricks.size();
     op->nb = fr_footprint(*s);
@@ -346,6 +370,10 @@ static int fr_execute_impl(umpa_fr_op *op, const void *fft, const float *scales,
   umpa::FrLaunch l{};
   l.items = v.fastMath ? op->dBricksSplit : op->dBricks;
   l.nItems = v.fastMath ? op->nBricksSplit : op->nBricks;
+  if (!v.fastMath) {
+    l.core = op->dCore;
+    l.nCore = op->nCore;
+  }
   l.cells = op->dCells;
   l.nCells = op->nCells;
   l.cellCounter = op->dCounter + 32;
@@ -482,7 +510,7 @@ static int fr_autotune_impl(umpa_fr_op *op, const void *fft, const float *scales
       const umpa::FrJob a =
         fr_job_record(op->desc, op->settings, op->constants, fft, scales, fftCount, vol,
                       static_cast<float *>(wts), spaces, nSpaces, cand.boxFixed);
-      const auto bricks = umpa::host::make_brick_schedule(vx, vy, vz, v.fastMath, cand);
+      const auto bricks = op_schedule(op, v.fastMath, cand);
       if (items) (void)hipFree(items);
       items = nullptr;
       e = upload_bricks(bricks, &items);
@@ -490,6 +518,10 @@ static int fr_autotune_impl(umpa_fr_op *op, const void *fft, const float *scales
       umpa::FrLaunch l{};
       l.items = items;
       l.nItems = (int)bricks.size();
+      if (!v.fastMath) {
+        l.core = op->dCore;
+        l.nCore = op->nCore;
+      }
       l.cells = op->dCells;
       l.nCells = op->nCells;
       l.cellCounter = op->dCounter + 32;
@@ -539,7 +571,7 @@ static int fr_autotune_impl(umpa_fr_op *op, const void *fft, const float *scales
   }
   // rebuild the schedule of this strategy with the chosen knobs
   try {
-    const auto bricks = umpa::host::make_brick_schedule(vx, vy, vz, v.fastMath, best);
+    const auto bricks = op_schedule(op, v.fastMath, best);
     int *items = nullptr;
     e = upload_bricks(bricks, &items);
     if (e != hipSuccess) return from_hip(e);
@@ -598,8 +630,7 @@ int umpa_fr_set_sched_params(umpa_fr_op *op, int strategy, const umpa_fr_sched_p
   DeviceGuard g(op->device);
   if (!g.ok) return UMPA_ERR_DEVICE;
   try {
-    const auto bricks = umpa::host::make_brick_schedule(
-      (int)op->desc.volume.x, (int)op->desc.volume.y, (int)op->desc.volume.z, slot == 1, sp);
+    const auto bricks = op_schedule(op, slot == 1, sp);
     int *items = nullptr;
     hipError_t e = upload_bricks(bricks, &items);
     if (e != hipSuccess) return from_hip(e);

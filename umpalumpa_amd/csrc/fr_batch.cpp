@@ -384,8 +384,7 @@ static int batch_plan_impl(umpa_fr_batch *b, const umpa_fr_job *jobs, uint32_t n
       for (const auto &li : step)
         if (e == hipSuccess) e = umpa::prepare_fr_insert(li.v, li.nTable);
     if (e == hipSuccess && useGraph) {
-      // the chunk loop as one graph: a counter-reset kernel and the persistent launch per
-      // (step, group), in stream order
+      // the chunk loop as one graph: the persistent launch per (step, group), in stream order
       e = hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal);
       hipError_t le = hipSuccess;
       if (e == hipSuccess) {

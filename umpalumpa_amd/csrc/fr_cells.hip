@@ -26,74 +26,13 @@
 // busy 0.35 (box 64, 500 spaces) and 0.8.  us per pass, bricks -> cells: box 32, 16 slices
 // 24.7 -> 15.3; box 64, 500, fast math 510 -> 120; box 100, 251, C4, r 1.5, exact 1004 -> 299;
 // box 128, 300, blob evaluated 831 -> 407.
-#include "fr_gather.hpp"
+#include "fr_cell.hpp"
 
 namespace umpa {
 
 constexpr int kCellWaves = 8;
 constexpr int kCellThreads = 64 * kCellWaves;
 constexpr int kCellTile = 2 * kCellThreads;  // spaces culled together
-constexpr int kCellRing = 128;               // a wavefront's queue: 7 left over + 64 new
-
-// What a lane needs of its space.
-struct CellSpace {
-  float t[3][3];
-  float weight, scale;
-  uint32_t off;  // byte offset of its slice in the chunk
-  int index;
-  bool inside;   // the block lies inside the space's sphere and traversal plane
-};
-
-// Does space `si` reach the block of edge `e` at (x0, y0, z0)?  As cull_space of the brick kernels;
-// `inside` as brick_inside.
-__device__ __forceinline__ bool cull_block(const FrJob &a, int si, int x0, int y0, int z0, int e,
-                                           int cxi, int cyi, bool &inside)
-{
-  const umpa_traverse_space &sp = a.spaces[si];
-  const float(*t)[3] = sp.transformInv;
-  const float half = 0.5f * (float)(e - 1);
-  const float cx = (float)(x0 - cxi) + half, cy = (float)(y0 - cyi) + half,
-              cz = (float)(z0 - cyi) + half;
-  const float norm = sqrtf(cx * cx + cy * cy + cz * cz);
-  const float dmin = fmaxf(norm - 1.7321f * half, 0.f);
-  const float eps = 0.02f + 1e-5f * norm;
-  const float qz = t[2][0] * cx + t[2][1] * cy + t[2][2] * cz;
-  const float ez = half * (fabsf(t[2][0]) + fabsf(t[2][1]) + fabsf(t[2][2]));
-  const float qx = t[0][0] * cx + t[0][1] * cy + t[0][2] * cz;
-  const float ex = half * (fabsf(t[0][0]) + fabsf(t[0][1]) + fabsf(t[0][2]));
-  const float mds = sp.maxDistanceSqr;
-  const int proj = sp.projectionIndex, dir = sp.dir;
-  const int x1 = x0 + e - 1, y1 = y0 + e - 1, z1 = z0 + e - 1;
-  const int mx = max(abs(x0 - cxi), abs(x1 - cxi));
-  const int my = max(abs(y0 - cyi), abs(y1 - cyi));
-  const int mz = max(abs(z0 - cyi), abs(z1 - cyi));
-  const bool inX = (x0 >= sp.minX) & (x1 <= sp.maxX);
-  const bool inY = (y0 >= sp.minY) & (y1 <= sp.maxY);
-  const bool inZ = (z0 >= sp.minZ) & (z1 <= sp.maxZ);
-  inside = ((float)(mx * mx + my * my + mz * mz) <= mds) &
-           (dir == 0 ? (inX & inY) : dir == 1 ? (inX & inZ) : (inY & inZ));
-  return (fabsf(qz) <= a.cullHalfWidth + ez + eps) & (qx >= -a.cullHalfSpace - ex - eps) &
-         (dmin * dmin <= mds * 1.0001f + eps) & (proj >= 0) & (proj < a.nProj) & (dir >= 0) &
-         (dir <= 2);
-}
-
-template <bool kHalf>
-__device__ __forceinline__ CellSpace load_space(const FrJob &a, int index, bool inside,
-                                                uint32_t sliceBytes)
-{
-  CellSpace s;
-  const umpa_traverse_space &sp = a.spaces[index];
-#pragma unroll
-  for (int i = 0; i < 9; ++i) s.t[i / 3][i % 3] = sp.transformInv[i / 3][i % 3];
-  s.weight = sp.weight;
-  const int proj = sp.projectionIndex;
-  s.off = (uint32_t)proj * sliceBytes;
-  s.scale = 1.f;
-  if constexpr (kHalf) s.scale = a.scales[proj];
-  s.index = index;
-  s.inside = inside;
-  return s;
-}
 
 template <int kMode, int kOrder, int kNB, bool kHalf, bool kFastMath, bool kShift>
 __global__ __launch_bounds__(kCellThreads, 4) void fr_insert_cell_kernel(FrJob a, FrLaunch l)
@@ -121,9 +60,7 @@ __global__ __launch_bounds__(kCellThreads, 4) void fr_insert_cell_kernel(FrJob a
   const uint32_t sliceBytes = (uint32_t)(a.sliceElems * kPix);
   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
     (void *)a.fft, 0, (int)((uint32_t)a.nProj * sliceBytes), kBufferConfig);
-  const int s = lane & 7, v = lane >> 3;  // the lane's space of eight and voxel of the cell
-  // lanes 0..23 own a cell's sums: component lane / 8 (re, im, weight) of voxel lane % 8
-  const int av = lane & 7, comp = lane >> 3;
+  unsigned long long nupd = 0;
 
   // Blocks in turn, heaviest first: the first from the grid, the others from the counter.  Every
   // workgroup's last claim finds none; the one that makes the launch's last claim clears the
@@ -172,98 +109,26 @@ __global__ __launch_bounds__(kCellThreads, 4) void fr_insert_cell_kernel(FrJob a
                   cellY = y0 + step0 * ((wave >> 1) & 1) + 2 * ((ci >> 1) & 1),
                   cellZ = z0 + step0 * (wave >> 2) + 2 * (ci >> 2);
         if (cellX >= a.vx || cellY >= a.vy || cellZ >= a.vz) continue;
-        const int x = cellX + (v & 1), y = cellY + ((v >> 1) & 1), z = cellZ + (v >> 2);
-        const bool valid = x < a.vx && y < a.vy && z < a.vz;
-        const float px = (float)(x - cxi), py = (float)(y - cyi), pz = (float)(z - cyi);
-        const float ccx = (float)(cellX - cxi) + 0.5f, ccy = (float)(cellY - cyi) + 0.5f,
-                    ccz = (float)(cellZ - cyi) + 0.5f;
-        const float cellEps =
-          0.02f + 1e-5f * sqrtf(ccx * ccx + ccy * ccy + ccz * ccz) + a.cullHalfWidth;
-        const int ax = cellX + (av & 1), ay = cellY + ((av >> 1) & 1), az = cellZ + (av >> 2);
-        const bool owner = lane < 24 && ax < a.vx && ay < a.vy && az < a.vz;
-        const int64_t gi = ((int64_t)az * a.vy + ay) * a.vx + ax;
-        float *const sum = comp == 2 ? a.weights + gi
-                                     : reinterpret_cast<float *>(a.volume) + 2 * gi + comp;
-        float acc = 0.f;
-        bool loaded = false;
-
+        Cell cell = make_cell(a, cellX, cellY, cellZ, lane);
         int head = 0, pend = 0;
         for (int t0 = 0; t0 < n; t0 += 64) {
           const bool have = t0 + lane < n;
           const uint32_t e = have ? (uint32_t)s_list[t0 + lane] : 0u;
           const float *r2 = a.spaces[base + (int)(e & 0x7fffu)].transformInv[2];
           const float t20 = r2[0], t21 = r2[1], t22 = r2[2];
-          const float qzc = t20 * ccx + t21 * ccy + t22 * ccz;
+          const float qzc = t20 * cell.cx + t21 * cell.cy + t22 * cell.cz;
           const float ez = 0.5f * (fabsf(t20) + fabsf(t21) + fabsf(t22));
-          const unsigned long long keep = __ballot(have && fabsf(qzc) <= cellEps + ez);
+          const unsigned long long keep = __ballot(have && fabsf(qzc) <= cell.reach + ez);
           if ((keep >> lane) & 1ull)
             queue[lanes_below(keep, (unsigned)(head + pend)) & (kCellRing - 1)] = (uint16_t)e;
           pend += __popcll(keep);
           wave_sync();
-          const int least = t0 + 64 < n ? 8 : 1;  // the last entries also make a partial step
-          if (pend < least) continue;
-          // spaces queue[head .. head + k) of the cell, one per lane & 7
-          auto space_at = [&](int from, int k) {
-            const uint32_t q = queue[(from + (s < k ? s : 0)) & (kCellRing - 1)];
-            return load_space<kHalf>(a, base + (int)(q & 0x7fffu), (q & 0x8000u) != 0, sliceBytes);
-          };
-          CellSpace next = space_at(head, pend);
-          do {
-            const CellSpace sp = next;
-            const int k = pend < 8 ? pend : 8;
-            // the next spaces' records load while these are gathered
-            if (pend - k >= least) next = space_at(head + k, pend - k);
-            head = (head + k) & (kCellRing - 1);
-            pend -= k;
-
-            const bool act = valid && s < k;
-            const umpa_traverse_space &rec = a.spaces[sp.index];
-            float qx, qy, zs;
-            bool hit;
-            if constexpr (kMode == kModeNearest) {
-              const float dsq = px * px + py * py + pz * pz;
-              qx = sp.t[0][0] * px + sp.t[0][1] * py + sp.t[0][2] * pz;
-              qy = sp.t[1][0] * px + sp.t[1][1] * py + sp.t[1][2] * pz;
-              zs = 0.f;
-              hit = act && !(dsq > rec.maxDistanceSqr) && !(qx < 0.f) && visited_nearest(rec, x, y, z);
-            } else {
-              hit = act && blob_predicate<false>(rec, sp.t, c, x, y, z, px, py, pz, sp.inside, qx, qy,
-                                                 zs);
-            }
-            if (!__any(hit)) continue;
-            if (!loaded) {
-              if (owner) acc = *sum;
-              loaded = true;
-            }
-            Contribution o{ -0.f, -0.f, -0.f };
-            if (hit) {
-              if constexpr (kMode == kModeNearest) {
-                o = gather_nearest<kHalf>(a, rsrc, qx, qy, sp.weight, sp.scale, sp.off);
-              } else {
-                o = gather_update<kMode, kOrder, kNB, kHalf, kFastMath, kTableLds, kShift, kRows>(
-                  a, nTable, rsrc, tbl, qx, qy, zs, sp.weight, false, sp.scale, sp.off);
-              }
-            }
-            part[lane] = o.re;
-            part[64 + lane] = o.im;
-            part[128 + lane] = o.w;
-            wave_sync();
-            if (lane < 24) {
-              const float4 p = reinterpret_cast<const float4 *>(part)[2 * lane],
-                           q = reinterpret_cast<const float4 *>(part)[2 * lane + 1];
-              acc = acc + p.x;
-              acc = acc + p.y;
-              acc = acc + p.z;
-              acc = acc + p.w;
-              acc = acc + q.x;
-              acc = acc + q.y;
-              acc = acc + q.z;
-              acc = acc + q.w;
-            }
-            wave_sync();
-          } while (pend >= least);
+          // the last entries also make a partial step
+          cell_take<kMode, kOrder, kNB, kHalf, kFastMath, kTableLds, kShift, kRows, false>(
+            cell, a, base, queue, part, head, pend, t0 + 64 < n ? 8 : 1, nTable, rsrc, tbl,
+            sliceBytes, lane, nupd);
         }
-        if (loaded && owner) *sum = acc;
+        if (cell.loaded && cell.owner) *cell.sum = cell.acc;
       }
     }
     b = __builtin_amdgcn_readfirstlane(s_next[turn]);

@@ -6,6 +6,7 @@
 #include "fr_host.hpp"
 
 #include <algorithm>
+#include <array>
 #include <cfloat>
 #include <cmath>
 #include <cstdlib>
@@ -264,7 +265,21 @@ bool box_can_shift(const umpa_fr_settings &s, uint64_t sliceX, uint64_t sliceY)
          sliceY >= (uint64_t)nb && sliceX <= 8192 && sliceY <= 8192;
 }
 
-std::vector<BrickCand> brick_candidates(int vx, int vy, int vz, float depthScale)
+float core_radius(int vx, int vy, int vz)
+{
+  // An exact launch takes at least as long as its heaviest brick's chain of spaces: 1 us a space
+  // at the centre, which every space reaches, against 0.36 us of the GPU's time per space at box
+  // 128, 0.75 at 192 and 1.25 at 256.  Taken as cells, the core's chain is a third as long (us
+  // without / with: box 128, 1,000 slices 926 / 427, 100 slices 123 / 113; 160, 400 404 / 299; 192,
+  // 333 374 / 324, 1,000 966 / 700; 192, 200, blob evaluated 567 / 444); from box 256 on it gains
+  // nothing (1,000 slices 1250 / 1248).  Radii of 9 to 17 measured alike, except box 128: 1,000
+  // slices 466 at 9 to 13, 427 at 17.
+  const int64_t voxels = (int64_t)vx * vy * vz;
+  auto cube = [](int64_t n) { return n * n * n; };
+  return voxels <= cube(161) ? 17.f : voxels <= cube(225) ? 11.f : 0.f;
+}
+
+std::vector<BrickCand> brick_candidates(int vx, int vy, int vz, float depthScale, float core)
 {
   // Bricks are 8 x 8 x D columns, D in {8, 4, 2, 1}.  A voxel at distance R from the centre
   // is crossed by a fraction ~ r/R of random slices, so the work of a brick grows towards the
@@ -280,6 +295,10 @@ std::vector<BrickCand> brick_candidates(int vx, int vy, int vz, float depthScale
   for (int y = 0; y < vy; y += 8)
     for (int x = 0; x < vx; x += 8)
       for (int z = 0; z < vz;) {
+        if (core > 0.f && z % 8 == 0 && radius(x, y, z, 8) <= core) {  // the core: core_cells
+          z += 8;
+          continue;
+        }
         int d = 8;
         while (d > 1 && depth_for(radius(x, y, z, d)) < d) d /= 2;
         const float R = radius(x, y, z, d);
@@ -297,10 +316,36 @@ std::vector<BrickCand> brick_candidates(int vx, int vy, int vz, float depthScale
   return cand;
 }
 
-BrickSet make_brick_set(int vx, int vy, int vz, float depthScale)
+std::vector<int> core_cells(int vx, int vy, int vz, float core)
+{
+  std::vector<int> out;
+  const float cx = static_cast<float>((vx - 1) / 2), cy = static_cast<float>((vy - 1) / 2);
+  // nearest 8 x 8 x 8 blocks first: every space reaches them
+  std::vector<std::pair<float, std::array<int, 3>>> blocks;
+  for (int z = 0; z < vz; z += 8)
+    for (int y = 0; y < vy; y += 8)
+      for (int x = 0; x < vx; x += 8) {
+        const float dx = x + 3.5f - cx, dy = y + 3.5f - cy, dz = z + 3.5f - cy;
+        const float R = std::sqrt(dx * dx + dy * dy + dz * dz);
+        if (R <= core) blocks.push_back({ R, { x, y, z } });
+      }
+  std::stable_sort(blocks.begin(), blocks.end(),
+                   [](const auto &a, const auto &b) { return a.first < b.first; });
+  for (const auto &b : blocks)
+    for (int i = 0; i < 64; ++i) {
+      const int x = b.second[0] + 2 * (i & 3), y = b.second[1] + 2 * ((i >> 2) & 3),
+                z = b.second[2] + 2 * (i >> 4);
+      if (x >= vx || y >= vy || z >= vz) continue;
+      out.push_back(x | y << 16);
+      out.push_back(z);
+    }
+  return out;
+}
+
+BrickSet make_brick_set(int vx, int vy, int vz, float depthScale, float core)
 {
   BrickSet set;
-  set.sorted = brick_candidates(vx, vy, vz, depthScale);
+  set.sorted = brick_candidates(vx, vy, vz, depthScale, core);
   std::stable_sort(set.sorted.begin(), set.sorted.end(),
                    [](const BrickCand &a, const BrickCand &b) { return a.est > b.est; });
   for (const BrickCand &b : set.sorted) set.estSum += b.est;
@@ -452,9 +497,9 @@ std::vector<BrickOrigin> make_schedule(const std::vector<JobWork> &jobs, bool sp
 }
 
 std::vector<BrickOrigin> make_brick_schedule(int vx, int vy, int vz, bool splitHeavy,
-                                             const SchedParams &sp)
+                                             const SchedParams &sp, float core)
 {
-  const BrickSet set = make_brick_set(vx, vy, vz, sp.depthScale);
+  const BrickSet set = make_brick_set(vx, vy, vz, sp.depthScale, core);
   return make_schedule({ JobWork{ &set, 0, 1.0 } }, splitHeavy, sp);
 }
 

@@ -61,7 +61,13 @@ struct BrickCand {
   int x, y, z, d;
   float est;
 };
-std::vector<BrickCand> brick_candidates(int vx, int vy, int vz, float depthScale = 1.f);
+// 8 x 8 x 8 blocks up to `core` from the centre are left out.
+std::vector<BrickCand> brick_candidates(int vx, int vy, int vz, float depthScale = 1.f,
+                                        float core = 0.f);
+// The core radius of a volume for plain exact launches, and its cells of 2 x 2 x 2 voxels, two ints
+// each: x | y << 16 and z.
+float core_radius(int vx, int vy, int vz);
+std::vector<int> core_cells(int vx, int vy, int vz, float core);
 
 // A volume's bricks sorted by estimated cost (heaviest first, ties in brick order) and the
 // costs' sum: what make_schedule needs of a volume, built once per volume shape.
@@ -69,7 +75,7 @@ struct BrickSet {
   std::vector<BrickCand> sorted;
   double estSum = 0;
 };
-BrickSet make_brick_set(int vx, int vy, int vz, float depthScale = 1.f);
+BrickSet make_brick_set(int vx, int vy, int vz, float depthScale = 1.f, float core = 0.f);
 
 // The bricks of one job in a launch, `scale` = slices the launch inserts for it.
 struct JobWork {
@@ -89,7 +95,8 @@ void make_schedule(const std::vector<JobWork> &jobs, bool splitHeavy, const Sche
 
 // make_schedule for a single job
 std::vector<BrickOrigin> make_brick_schedule(int vx, int vy, int vz, bool splitHeavy,
-                                             const SchedParams &sp = SchedParams());
+                                             const SchedParams &sp = SchedParams(),
+                                             float core = 0.f);
 
 // The 4 x 4 x 4 blocks covering a volume, nearest to the centre first, two ints each: x | y << 16
 // and z (the small-problem kernel's work items).

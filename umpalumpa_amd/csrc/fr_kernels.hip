@@ -26,7 +26,7 @@
 // fr_insert_kernel covers every mode, precision and strategy; fr_insert_staged_kernel, for the
 // exact FP32 lookup strategy, gathers the predicate's hits of several spaces together (see
 // there).
-#include "fr_gather.hpp"
+#include "fr_cell.hpp"
 
 namespace umpa {
 
@@ -44,7 +44,7 @@ constexpr int kVox = kEdge * kEdge * kEdge;
 
 // Per-wave LDS state: running sums of the wave's 8 x 8 x 8 brick and the queue of voxels that
 // pass the slab test for the current space.
-struct WaveScratch {
+struct alignas(16) WaveScratch {
   float accR[kVox];
   float accI[kVox];
   float accW[kVox];
@@ -69,6 +69,45 @@ __device__ __forceinline__ T uniform_load(const T *p, int index)
   T out;
   __builtin_memcpy(&out, w, sizeof(T));
   return out;
+}
+
+// The wavefront's number in the launch, workgroups first: consecutive numbers are different CUs.
+__device__ __forceinline__ int wave_number()
+{
+  return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * (int)gridDim.x + (int)blockIdx.x;
+}
+
+// Items are taken in order, heaviest first: a wavefront's first is its number, the others come
+// from the counter, which counts on from the launch's `claimed` wavefronts.  (Every claim on the
+// one counter holds up the others by about 8 ns: with the first ones counted too, a launch of 3,072
+// wavefronts spent 25 us before its first brick; box 192, 333 spaces, exact 404 -> 373 us.)
+// Each item taken makes one claim, so the last of the launch finds nItems - 1: it clears the
+// counter for the next launch.
+__device__ __forceinline__ int claim_item(const FrLaunch &l, int lane, int claimed)
+{
+  int next = 0;
+  if (lane == 0) {
+    next = atomicAdd(l.counter, 1);
+    if (next == l.nItems - 1) atomicExch(l.counter, 0);
+  }
+  return __builtin_amdgcn_readfirstlane(next) + claimed;
+}
+
+// Bounded launches (l.waveItems items per wavefront, the grid covering the items) need no counter:
+// workgroups go by groups of one per CU, a group takes the next items in order and deals them out
+// across its workgroups, so that a workgroup's wavefronts have items of about the same cost and
+// the heaviest lie on different CUs.  (With the counter, a four-job serving tick of 63,000 items
+// made 95,000 claims: 1737 -> 1635 us.)
+struct DealtItems {
+  int first, step;
+};
+__device__ __forceinline__ DealtItems deal_items(const FrLaunch &l, int waves)
+{
+  const int group = (int)blockIdx.x / l.numCUs, in = (int)blockIdx.x - group * l.numCUs;
+  const int start = group * l.numCUs;
+  const int size = min(l.numCUs, (int)gridDim.x - start);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  return { start * waves * l.waveItems + wave * size + in, waves * size };
 }
 
 // ---- the brick's steps shared by the insertion kernels ----------------------------------------
@@ -269,20 +308,30 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
   WaveScratch &ws = s_wave[threadIdx.x >> 6];
   constexpr int kPix = kHalf ? 4 : 8;
 
-  // bounded launches (batches): lane 0 claims at most l.waveItems items, then an index past
-  // the items.  Only the batched instantiations carry the bound: in the others any bound on
-  // this loop costs the compiler's schedule (per-pair FP16 kernel 84 -> 71 VGPRs, 1.22 ->
-  // 1.75 ms per 1,000-slice chunk at box 256).
-  int budget = l.waveItems > 0 ? l.waveItems : -1;
-  for (;;) {
-    int b = 0;
-    if constexpr (kBatched) {
-      if (lane == 0) b = budget-- == 0 ? 0x7fffffff : atomicAdd(l.counter, 1);
-    } else {
-      if (lane == 0) b = atomicAdd(l.counter, 1);
+  const int number = wave_number(), claimed = kWaves * (int)gridDim.x;
+  if constexpr (!kFastMath && !kBatched) {
+    if (job0.spaceBegin >= job0.spaceEnd) return;
+    // the volume's core, cell by cell, as in fr_insert_staged_kernel
+    for (int b = number; b < l.nCore; b += claimed) {
+      const int2 bo = make_uniform(reinterpret_cast<const int2 *>(l.core)[b]);
+      const __amdgpu_buffer_rsrc_t all = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)job0.fft, 0, (int)((uint32_t)job0.nProj * (uint32_t)(job0.sliceElems * kPix)),
+        kBufferConfig);
+      unsigned long long n = 0;
+      cell_item<kMode, kOrder, kNB, kMode == kModeLookup && kTableLds, kShift, kCount>(
+        job0, bo.x & 0xffff, bo.x >> 16, bo.y, job0.spaceBegin, job0.spaceEnd,
+        reinterpret_cast<uint32_t *>(ws.queue), ws.accR, nTable, all, tbl, lane, n);
+      if constexpr (kCount) {
+        if (lane == 0 && n) atomicAdd(l.updates, n);
+      }
     }
-    b = __builtin_amdgcn_readfirstlane(__shfl(b, 0));
-    if (b >= l.nItems) break;
+  }
+  const bool bounded = kBatched && l.waveItems > 0;
+  DealtItems dealt{ !kFastMath && !kBatched ? claimed - 1 - number : number, 0 };
+  if (bounded) dealt = deal_items(l, kWaves);
+  int left = l.waveItems;
+  for (int b = dealt.first; b < l.nItems;
+       b = bounded ? (--left > 0 ? b + dealt.step : l.nItems) : claim_item(l, lane, claimed)) {
     const int4 bo = make_uniform(reinterpret_cast<const int4 *>(l.items)[b]);
     // work item: brick 8 x 8 x depth at (bo.x, bo.y, bo.z & 0xffff) of job bo.z >> 16; heavy
     // bricks run at raised wave priority; a brick split into `parts` slice ranges accumulates
@@ -494,17 +543,13 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fr_insert_carry_kernel(FrJob j
   CarryScratch &ws = s_wave[wv];
   CarrySlot *slots = s_slot[wv];
 
-  // bounded launches (batches only, as in fr_insert_kernel)
-  int budget = l.waveItems > 0 ? l.waveItems : -1;
-  for (;;) {
-    int b = 0;
-    if constexpr (kBatched) {
-      if (lane == 0) b = budget-- == 0 ? 0x7fffffff : atomicAdd(l.counter, 1);
-    } else {
-      if (lane == 0) b = atomicAdd(l.counter, 1);
-    }
-    b = __builtin_amdgcn_readfirstlane(__shfl(b, 0));
-    if (b >= l.nItems) break;
+  const int number = wave_number(), claimed = kWaves * (int)gridDim.x;
+  const bool bounded = kBatched && l.waveItems > 0;
+  DealtItems dealt{ number, 0 };
+  if (bounded) dealt = deal_items(l, kWaves);
+  int left = l.waveItems;
+  for (int b = dealt.first; b < l.nItems;
+       b = bounded ? (--left > 0 ? b + dealt.step : l.nItems) : claim_item(l, lane, claimed)) {
     const int4 bo = make_uniform(reinterpret_cast<const int4 *>(l.items)[b]);
     const FrJob a = kBatched ? make_uniform(l.jobs[bo.z >> 16]) : job0;
     const int s0 = a.spaceBegin, s1 = a.spaceEnd;
@@ -682,15 +727,23 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
   const int cxi = c.cMaxVolumeIndexX / 2, cyi = c.cMaxVolumeIndexYZ / 2;
   const float slabR = c.cBlobRadius * kSlabMargin;
 
-  for (;;) {
-    int b = 0;
-    if (lane == 0) b = atomicAdd(l.counter, 1);
-    b = __builtin_amdgcn_readfirstlane(__shfl(b, 0));
-    if (b >= l.nItems) break;
+  const int sBegin = a.spaceBegin, sEnd = a.spaceEnd;
+  if (sBegin >= sEnd) return;
+  const int number = wave_number(), claimed = kWaves * (int)gridDim.x;
+  // the volume's core, cell by cell (a loop of its own: as a branch of the brick loop it cost that
+  // loop's schedule 4 %)
+  for (int b = number; b < l.nCore; b += claimed) {
+    const int2 bo = uniform_load(reinterpret_cast<const int2 *>(l.core), b);
+    unsigned long long none = 0;
+    cell_item<kModeLookup, 0, kNB, true, kShift, false>(
+      a, bo.x & 0xffff, bo.x >> 16, bo.y, sBegin, sEnd,
+      reinterpret_cast<uint32_t *>(ws.queue), ws.accR, nTable, rsrc, tbl, lane, none);
+  }
+
+  // wavefronts with a cell of the core start on the lighter of the first bricks
+  for (int b = claimed - 1 - number; b < l.nItems;) {
     const int4 bo = uniform_load(reinterpret_cast<const int4 *>(l.items), b);
     // work item: brick 8 x 8 x depth at (bo.x, bo.y, bo.z); the exact schedules never split
-    const int sBegin = a.spaceBegin, sEnd = a.spaceEnd;
-    if (sBegin >= sEnd) continue;
     const bool heavy = (bo.w >> 4) & 1;
     if (heavy) __builtin_amdgcn_s_setprio(2);
     const BrickCtx bk = make_brick(a, bo, lane);
@@ -764,10 +817,9 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
     }
     if (loaded) store_brick(ws, a, bk, lane, false);
     if (heavy) __builtin_amdgcn_s_setprio(0);
+    b = claim_item(l, lane, claimed);
   }
 }
-
-__global__ void fr_reset_counter(int *counter) { *counter = 0; }
 
 // ---- host-side dispatch ------------------------------------------------------------------
 // The kernel is instantiated per (mode, order, footprint width, FP16, fast math, counting, LDS
@@ -917,27 +969,35 @@ hipError_t prepare_fr_insert(const FrVariant &v, int nTable)
   return e;
 }
 
-// Does this launch run the small-problem kernel?  The brick kernels take as long as the central
-// brick's chain of spaces (about 1 us each; 2.7 with the blob evaluated) however small the
-// volume, the cell kernel about 0.03 us per space and 1,000 voxels of a plane plus 0.05 us per
-// 1,000 voxels.  Measured (us, bricks / cells, r 1.9): exact, 400 slices: box 40 448 / 85, 64
-// 388 / 106, 100 463 / 187, 128 404 / 283, 144 415 / 357, 160 429 / 442; 100 slices: 100
-// 151 / 96, 112 137 / 122, 128 154 / 161, 144 171 / 210; fast math, whose schedules split the
-// central bricks, 1,500 slices: 80 787 / 402, 100 771 / 554, 112 728 / 655, 128 709 / 828; FP16
-// 112 816 / 614, 128 793 / 775; blob evaluated, 400 slices: 100 1205 / 330, 160 1074 / 759, 200
-// 1223 / 1224, 50 slices: 100 190 / 129, 128 196 / 209; nearest, 400 slices: 128 386 / 263, 160
-// 437 / 427.  So: up to 117^3 voxels always; without fast math, from 256 spaces, up to 145^3
-// (161^3 with the blob evaluated).
+// Does this launch run the small-problem kernel?  The brick kernels take a space per 0.3 to 1.2 us
+// (their heaviest brick's chain) whatever the volume, the cell kernel a fixed 4 us per round of
+// blocks and less per space.  Measured (us, bricks / cells at r 1.9, slices): exact, box 48 20
+// 28 / 29, 400 206 / 90; 64 20 32 / 43, 100 66 / 53, 400 188 / 107; 80 100 64 / 68, 400 184 / 136;
+// 90 400 193 / 163; 100 400 186 / 188; r 1.5 100 1,004 336 / 299, 112 1,000 326 / 362; r 2.5 100
+// 100 179 / 149, 112 600 603 / 562, 128 600 647 / 709.  Fast math: 64 20 37 / 43, 100 111 / 50,
+// 80 100 65 / 66, 100 100 87 / 93, 400 213 / 175; 112 400 219 / 208; 128 1,500 691 / 826; FP16
+// 112 400 232 / 196, 128 1,500 765 / 766.  Blob evaluated: 80 50 104 / 78, 100 50 116 / 128, 400
+// 518 / 328; 128 300 386 / 404, 400 542 / 494.  Nearest: 64 400 131 / 122, 80 400 140 / 126, 100
+// 400 147 / 184.  So, with V the volume's mean extent: from (V - from) * slope spaces, up to a V.
 bool use_cells(const FrJob &job, const FrLaunch &l, const FrVariant &v)
 {
   if (l.nCells <= 0 || v.batched || v.count || v.kernel != kKernelAuto || v.tableGlobal) return false;
   if (v.mode == kModeLookup && l.nTable > kMaxLdsTable) return false;  // the table stays global
   if (!carry_fits(job, v.half)) return false;  // the chunk's slices need one buffer resource each
+  struct Rule {
+    int upTo;
+    float from, slope;
+  };
+  const Rule rule = v.mode == kModeNearest  ? Rule{ 85, 45.f, 4.f }
+                    : v.mode != kModeLookup ? Rule{ 129, 75.f, 6.f }
+                    : v.fastMath            ? Rule{ 121, 55.f, 5.f }
+                    : v.nb == 3             ? Rule{ 105, 45.f, 4.f }
+                    : v.nb == 4             ? Rule{ 97, 45.f, 4.f }
+                                            : Rule{ 121, 45.f, 1.5f };
   const int64_t voxels = (int64_t)job.vx * job.vy * job.vz;
-  auto cube = [](int64_t n) { return n * n * n; };
-  if (voxels <= cube(117)) return true;
-  const bool blob = v.mode == kModeFastKaiser || v.mode == kModePreciseKaiser;
-  return !v.fastMath && job.spaceEnd - job.spaceBegin >= 256 && voxels <= cube(blob ? 161 : 145);
+  if (voxels > (int64_t)rule.upTo * rule.upTo * rule.upTo) return false;
+  const float spaces = (float)(job.spaceEnd - job.spaceBegin);
+  return spaces >= (cbrtf((float)voxels) - rule.from) * rule.slope;
 }
 
 hipError_t launch_fr_insert(const FrJob &job, const FrLaunch &l, const FrVariant &v0, int numCUs,
@@ -983,9 +1043,9 @@ hipError_t launch_fr_insert(const FrJob &job, const FrLaunch &l, const FrVariant
     if (l.maxBlocks > 0 && blocks > l.maxBlocks) blocks = l.maxBlocks;
   }
   if (blocks < 1) blocks = 1;
-  hipLaunchKernelGGL(fr_reset_counter, dim3(1), dim3(1), 0, st, l.counter);
   FrJob j = job;
   FrLaunch ll = l;
+  ll.numCUs = numCUs;
   void *args[] = { &j, &ll };
   return hipLaunchKernel(k, dim3(blocks), dim3(64 * waves), args, shmem, st);
 }

@@ -19,6 +19,9 @@ namespace umpa {
 constexpr size_t kScratchHeader = 256;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
+// A launch leaves the counter at zero; calls that raced may not have.
+__global__ void fr_clear_counter(int *counter) { *counter = 0; }
+
 namespace {
 
 struct DeviceScratch {
@@ -77,6 +80,10 @@ hipError_t launch_fr_insert_noalloc(int device, const FrJob &job, const FrVarian
   l.table = table;
   l.nTable = nTable;
   e = prepare_fr_insert(v, nTable);
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(fr_clear_counter, dim3(1), dim3(1), 0, st, l.counter);
+    e = hipGetLastError();
+  }
   if (e == hipSuccess) e = launch_fr_insert(job, l, v, numCUs, st);
   return e;
 }

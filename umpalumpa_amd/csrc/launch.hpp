@@ -35,14 +35,17 @@ static_assert(sizeof(FrJob) == 128, "job records are 128 B on host and device");
 // blob table shared by all its jobs.
 struct FrLaunch {
   const FrJob *jobs;    // device array of jobs (batched launches only)
-  const int *items;     // int4 {x, y, z | job << 16, key} per work item
+  const int *items;     // int4 {x, y, z | job << 16, flags} per work item
   int nItems;
-  int *counter;         // work counter, zeroed before the launch
+  const int *core;      // int2 {x | y << 16, z} per cell of 2 x 2 x 2 voxels (plain exact launches):
+  int nCore;            // the volume's core, which `items` then leaves out
+  int *counter;         // work counter: zero between launches
   unsigned long long *updates;  // voxel-update counter (counting variant only)
   const float *table;   // blob table (kLookup)
   int nTable;
   int waveItems;        // items per wave before it leaves (0: until the items run out)
   int maxBlocks;        // persistent launches: at most this many workgroups (0: one per CU)
+  int numCUs;           // set by the launch
   const int *cells;     // int2 {x | y << 16, z | edge << 16} per block of the volume, heaviest first
   int nCells;           // (plain launches whose host keeps the list; 0: none)
   int *cellCounter;     // blocks claimed so far: zero between launches
@@ -76,14 +79,14 @@ enum : int { kKernelAuto = 0, kKernelPair = 1, kKernelCarry = 2, kKernelStaged =
 // Dynamic LDS and workgroup count of an insertion launch; `prepare` sets the kernel's LDS
 // attribute once (outside any stream capture).
 hipError_t prepare_fr_insert(const FrVariant &v, int nTable);
-// Enqueues the counter reset and the insertion kernel on `st`.
+// Enqueues the insertion kernel on `st`.
 hipError_t launch_fr_insert(const FrJob &job, const FrLaunch &l, const FrVariant &v, int numCUs,
                             hipStream_t st);
 
 // May a volume of these extents run the small-problem kernel (its host then keeps the block list)?
 inline bool cells_possible(int vx, int vy, int vz)
 {
-  return (int64_t)vx * vy * vz <= (int64_t)161 * 161 * 161 && vx < 65536 && vy < 65536 && vz < 32768;
+  return (int64_t)vx * vy * vz <= (int64_t)129 * 129 * 129 && vx < 65536 && vy < 65536 && vz < 32768;
 }
 // Does the launch run the small-problem kernel (which needs no `prepare`)?
 bool use_cells(const FrJob &job, const FrLaunch &l, const FrVariant &v);

@@ -93,6 +93,14 @@ __device__ __forceinline__ int claim_item(const FrLaunch &l, int lane, int claim
   return __builtin_amdgcn_readfirstlane(next) + claimed;
 }
 
+// A wavefront's first brick where the first nCore of them begin with a cell of the core: the others
+// start on the heaviest bricks, these on the lightest of the first ones.
+__device__ __forceinline__ int first_after_core(const FrLaunch &l, int number, int claimed)
+{
+  const int core = l.nCore % claimed;
+  return number >= core ? number - core : number + claimed - core;
+}
+
 // Bounded launches (l.waveItems items per wavefront, the grid covering the items) need no counter:
 // workgroups go by groups of one per CU, a group takes the next items in order and deals them out
 // across its workgroups, so that a workgroup's wavefronts have items of about the same cost and
@@ -327,7 +335,7 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
     }
   }
   const bool bounded = kBatched && l.waveItems > 0;
-  DealtItems dealt{ !kFastMath && !kBatched ? claimed - 1 - number : number, 0 };
+  DealtItems dealt{ !kFastMath && !kBatched ? first_after_core(l, number, claimed) : number, 0 };
   if (bounded) dealt = deal_items(l, kWaves);
   int left = l.waveItems;
   for (int b = dealt.first; b < l.nItems;
@@ -741,7 +749,7 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
   }
 
   // wavefronts with a cell of the core start on the lighter of the first bricks
-  for (int b = claimed - 1 - number; b < l.nItems;) {
+  for (int b = first_after_core(l, number, claimed); b < l.nItems;) {
     const int4 bo = uniform_load(reinterpret_cast<const int4 *>(l.items), b);
     // work item: brick 8 x 8 x depth at (bo.x, bo.y, bo.z); the exact schedules never split
     const bool heavy = (bo.w >> 4) & 1;

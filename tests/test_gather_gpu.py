@@ -49,3 +49,25 @@ def test_tight_boxes_at_pixel_ties(box, radius):
     ov, ow, _ = run_oracle(s, deq, spaces, table, box)
     v, w, _ = run_hip(s, fft, spaces, desc, table, box, half=(h, scales))
     assert rel_l2(v, ov) <= 1e-5 and rel_l2(w, ow) <= 1e-5
+
+
+@pytest.mark.parametrize("alpha,order", [(15.0, 0), (16.0, 2)])
+@pytest.mark.parametrize("radius", [0.3, 1.9, 2.0, 2.6])
+@pytest.mark.parametrize("box,n", [(6, 9), (30, 13), (130, 3)])
+def test_evaluated_blobs(box, n, radius, alpha, order):
+    """Blob values computed for a wavefront's candidates together: no candidate or few inside
+    (r = 0.3), boxes with a fifth column (r = 2.0 at ties, 2.6 always: the general loop beside
+    the box in one wavefront), slices narrower than a box, weights other than 1.  Small boxes
+    take cells, the counting pass and box 130 bricks (its core: cells)."""
+    s = settings(F.FR_DYNAMIC, F.FR_PRECISE, alpha, radius, order)
+    rots = np.concatenate([_half_step_rotations()[:2], pyoracle.uniform_rotations(n, 3)])
+    fft = synthetic_slices(box, len(rots), 5)
+    spaces = F.traverse_spaces(rots, box, s, weight=0.75)
+    spaces["weight"][::2] = 1.0
+    desc = F.fr_desc(box // 2 + 1, box, len(rots), box + 1, len(spaces), 0)
+    ov, ow, updates = run_oracle(s, fft, spaces, None, box)
+    v, w, _ = run_hip(s, fft, spaces, desc, None, box)
+    assert np.array_equal(v, ov, equal_nan=True) and np.array_equal(w, ow, equal_nan=True)
+    v, w, got = run_hip(s, fft, spaces, desc, None, box, count=True)
+    assert np.array_equal(v, ov, equal_nan=True) and np.array_equal(w, ow, equal_nan=True)
+    assert got == updates

@@ -117,10 +117,12 @@ __device__ __forceinline__ Cell make_cell(const FrJob &a, int x0, int y0, int z0
 // gather per lane, the contributions through LDS (`part`, 192 floats) to the lanes that own the
 // sums, which add the eight spaces' in order, so a voxel receives its spaces in index order.  A
 // pair that misses adds -0, which changes no float.  Entry i of the queue names space base + i.
+// `blob`: kBlobList floats of the wavefront's LDS for the evaluated blob modes.
 template <int kMode, int kOrder, int kNB, bool kHalf, bool kFastMath, bool kTableLds, bool kShift,
           int kRows, bool kCount, typename Entry>
 __device__ __forceinline__ void cell_take(Cell &k, const FrJob &a, int base, const Entry *queue,
-                                          float *part, int &head, int &pend, int least, int nTable,
+                                          float *part, float *blob, int &head, int &pend, int least,
+                                          int nTable,
                                           __amdgpu_buffer_rsrc_t rsrc, const float *tbl,
                                           uint32_t sliceBytes, int lane, unsigned long long &nupd)
 {
@@ -161,7 +163,11 @@ __device__ __forceinline__ void cell_take(Cell &k, const FrJob &a, int base, con
       k.loaded = true;
     }
     Contribution o{ -0.f, -0.f, -0.f };
-    if (hit) {
+    if constexpr (evaluates_blob(kMode)) {
+      const Contribution got = gather_evaluated<kMode, kOrder>(a, rsrc, blob, lane, hit, qx, qy, zs,
+                                                               sp.weight, sp.off);
+      if (hit) o = got;
+    } else if (hit) {
       if constexpr (kMode == kModeNearest) {
         o = gather_nearest<kHalf>(a, rsrc, qx, qy, sp.weight, sp.scale, sp.off);
       } else {
@@ -191,10 +197,12 @@ __device__ __forceinline__ void cell_take(Cell &k, const FrJob &a, int base, con
 }
 
 // A work item of the brick kernels that is one cell: culls the spaces 64 at a time and takes the
-// survivors.  `queue` and `part` are kCellRing and 192 dwords of the wavefront's LDS.
+// survivors.  `queue`, `part` and `blob` are kCellRing, 192 and (evaluated blobs) kBlobList dwords
+// of the wavefront's LDS.
 template <int kMode, int kOrder, int kNB, bool kTableLds, bool kShift, bool kCount>
 __device__ __forceinline__ void cell_item(const FrJob &a, int x0, int y0, int z0, int sBegin,
-                                          int sEnd, uint32_t *queue, float *part, int nTable,
+                                          int sEnd, uint32_t *queue, float *part, float *blob,
+                                          int nTable,
                                           __amdgpu_buffer_rsrc_t rsrc, const float *tbl, int lane,
                                           unsigned long long &nupd)
 {
@@ -213,7 +221,7 @@ __device__ __forceinline__ void cell_item(const FrJob &a, int x0, int y0, int z0
     pend += __popcll(m);
     wave_sync();
     cell_take<kMode, kOrder, kNB, false, false, kTableLds, kShift, 2, kCount>(
-      cell, a, 0, queue, part, head, pend, base + 64 < sEnd ? 8 : 1, nTable, rsrc, tbl, sliceBytes,
+      cell, a, 0, queue, part, blob, head, pend, base + 64 < sEnd ? 8 : 1, nTable, rsrc, tbl, sliceBytes,
       lane, nupd);
   }
   if (cell.loaded && cell.owner) *cell.sum = cell.acc;

@@ -43,6 +43,7 @@ __global__ __launch_bounds__(kCellThreads, 4) void fr_insert_cell_kernel(FrJob a
   constexpr int kRows = kHalf ? (kNB <= 4 ? kNB : 3) : kNB <= 3 ? 3 : 2;
   extern __shared__ float s_table[];
   __shared__ __align__(16) float s_part[kCellWaves][3 * 64];
+  __shared__ float s_blob[evaluates_blob(kMode) ? kCellWaves : 1][evaluates_blob(kMode) ? kBlobList : 1];
   __shared__ uint16_t s_list[kCellTile];
   __shared__ uint16_t s_queue[kCellWaves][kCellRing];
   __shared__ int s_count[kCellWaves];
@@ -53,7 +54,7 @@ __global__ __launch_bounds__(kCellThreads, 4) void fr_insert_cell_kernel(FrJob a
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  float *part = s_part[wave];
+  float *part = s_part[wave], *blob = evaluates_blob(kMode) ? s_blob[wave] : nullptr;
   uint16_t *queue = s_queue[wave];
   const umpa_fr_constants &c = a.c;
   const int cxi = c.cMaxVolumeIndexX / 2, cyi = c.cMaxVolumeIndexYZ / 2;
@@ -125,7 +126,7 @@ __global__ __launch_bounds__(kCellThreads, 4) void fr_insert_cell_kernel(FrJob a
           wave_sync();
           // the last entries also make a partial step
           cell_take<kMode, kOrder, kNB, kHalf, kFastMath, kTableLds, kShift, kRows, false>(
-            cell, a, base, queue, part, head, pend, t0 + 64 < n ? 8 : 1, nTable, rsrc, tbl,
+            cell, a, base, queue, part, blob, head, pend, t0 + 64 < n ? 8 : 1, nTable, rsrc, tbl,
             sliceBytes, lane, nupd);
         }
         if (cell.loaded && cell.owner) *cell.sum = cell.acc;

@@ -307,6 +307,7 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
   extern __shared__ float s_table[];
   __shared__ WaveScratch s_wave[kWaves];
   __shared__ umpa_traverse_space s_space[kWaves];  // the space the wave works on
+  __shared__ float s_blob[evaluates_blob(kMode) ? kWaves : 1][evaluates_blob(kMode) ? kBlobList : 1];
   const int nTable = l.nTable;
   if constexpr (kMode == kModeLookup && kTableLds) {
     stage_table<kThreads>(s_table, l.table, nTable);
@@ -315,6 +316,7 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
   const int lane = threadIdx.x & 63;
   WaveScratch &ws = s_wave[threadIdx.x >> 6];
   constexpr int kPix = kHalf ? 4 : 8;
+  static_assert(kBlobList <= kVox, "a cell's evaluations fit one of the wave's arrays of sums");
 
   const int number = wave_number(), claimed = kWaves * (int)gridDim.x;
   if constexpr (!kFastMath && !kBatched) {
@@ -328,7 +330,7 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
       unsigned long long n = 0;
       cell_item<kMode, kOrder, kNB, kMode == kModeLookup && kTableLds, kShift, kCount>(
         job0, bo.x & 0xffff, bo.x >> 16, bo.y, job0.spaceBegin, job0.spaceEnd,
-        reinterpret_cast<uint32_t *>(ws.queue), ws.accR, nTable, all, tbl, lane, n);
+        reinterpret_cast<uint32_t *>(ws.queue), ws.accR, ws.accI, nTable, all, tbl, lane, n);
       if constexpr (kCount) {
         if (lane == 0 && n) atomicAdd(l.updates, n);
       }
@@ -427,9 +429,14 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
           } else {
             hit = act && blob_predicate<false>(sp, sp.transformInv, c, xv, yv, zv, pxv, pyv, pzv, inside, qx, qy, zs);
           }
+          Contribution o;
+          if constexpr (evaluates_blob(kMode))
+            o = gather_evaluated<kMode, kOrder>(a, rsrc, s_blob[threadIdx.x >> 6], lane, hit, qx, qy,
+                                                zs, sp.weight);
           if (hit) {
-            Contribution o;
-            if constexpr (kMode == kModeNearest) {
+            if constexpr (evaluates_blob(kMode)) {
+              // gathered above, by the whole wavefront
+            } else if constexpr (kMode == kModeNearest) {
               o = gather_nearest<kHalf>(a, rsrc, qx, qy, sp.weight, scale);
             } else {
               o = gather_update<kMode, kOrder, kNB, kHalf, kFastMath, kTableLds, kShift>(
@@ -745,7 +752,7 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
     unsigned long long none = 0;
     cell_item<kModeLookup, 0, kNB, true, kShift, false>(
       a, bo.x & 0xffff, bo.x >> 16, bo.y, sBegin, sEnd,
-      reinterpret_cast<uint32_t *>(ws.queue), ws.accR, nTable, rsrc, tbl, lane, none);
+      reinterpret_cast<uint32_t *>(ws.queue), ws.accR, ws.accI, nTable, rsrc, tbl, lane, none);
   }
 
   // wavefronts with a cell of the core start on the lighter of the first bricks

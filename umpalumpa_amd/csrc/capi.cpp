@@ -45,11 +45,12 @@ struct umpa_fr_op {
   int strategy = UMPA_FR_EXACT;
   bool countUpdates = false;
   unsigned long long lastUpdates = 0;
-  int *dBricks = nullptr;      // exact schedule: every brick owned by one wavefront
+  int *dState = nullptr;       // owns the following (one allocation, one upload at Init):
+  int *dBricks = nullptr;      //   exact schedule: every brick owned by one wavefront
   int nBricks = 0;
-  int *dBricksSplit = nullptr; // fast-math schedule: central bricks split over wavefronts
+  int *dBricksSplit = nullptr; //   fast-math schedule: central bricks split over wavefronts
   int nBricksSplit = 0;
-  int *dState = nullptr;       // owns the following:
+  int *dTuned[2] = { nullptr, nullptr };  // schedules (exact, fast math) that replaced Init's
   int *dCounter = nullptr;     //   work counter of the brick kernels; the cell kernel's 128 bytes on
   unsigned long long *dUpdates = nullptr;
   int *dCells = nullptr;       //   small volumes: the blocks of the small-problem kernel
@@ -61,8 +62,10 @@ struct umpa_fr_op {
 
   void release()
   {
-    if (dBricks) (void)hipFree(dBricks);
-    if (dBricksSplit) (void)hipFree(dBricksSplit);
+    for (int *&t : dTuned) {
+      if (t) (void)hipFree(t);
+      t = nullptr;
+    }
     if (dState) (void)hipFree(dState);
     dState = nullptr;
     dBricks = nullptr;
@@ -79,16 +82,24 @@ struct umpa_fr_op {
   }
 };
 
-// Work items as the kernel reads them (int4 per item) in a new device buffer.
+// Work items as the kernel reads them (int4 per item), appended to `flat`.
+static void append_bricks(const std::vector<umpa::host::BrickOrigin> &bricks, std::vector<int> &flat)
+{
+  size_t at = flat.size();
+  flat.resize(at + bricks.size() * 4);
+  for (const auto &b : bricks) {
+    flat[at++] = b.x;
+    flat[at++] = b.y;
+    flat[at++] = b.z;
+    flat[at++] = b.w;
+  }
+}
+
+// ... in a new device buffer.
 static hipError_t upload_bricks(const std::vector<umpa::host::BrickOrigin> &bricks, int **dst)
 {
-  std::vector<int> flat(bricks.size() * 4);
-  for (size_t i = 0; i < bricks.size(); ++i) {
-    flat[4 * i + 0] = bricks[i].x;
-    flat[4 * i + 1] = bricks[i].y;
-    flat[4 * i + 2] = bricks[i].z;
-    flat[4 * i + 3] = bricks[i].w;
-  }
+  std::vector<int> flat;
+  append_bricks(bricks, flat);
   hipError_t e = hipMalloc(dst, std::max<size_t>(flat.size(), 4) * sizeof(int));
   if (e == hipSuccess && !flat.empty())
     e = hipMemcpy(*dst, flat.data(), flat.size() * sizeof(int), hipMemcpyHostToDevice);
@@ -200,9 +211,15 @@ int umpa_fr_init(umpa_fr_op *op, const umpa_fr_desc *desc, const umpa_fr_setting
     const int vx = (int)desc->volume.x, vy = (int)desc->volume.y, vz = (int)desc->volume.z;
     const auto bricks = op_schedule(op, false, op->params[0]);
     const auto split = op_schedule(op, true, op->params[1]);
-    // the counters (work items, blocks, updates; zero) and the blocks of a small volume, each
-    // counter in 128-byte lines of its own: the blocks beside it made box 32 take 19 us, not 15
-    std::vector<int> state(96, 0);
+    // the counters (work items, blocks, updates; zero), each in 128-byte lines of its own (the
+    // blocks beside one made box 32 take 19 us, not 15), then the schedules and the blocks of a
+    // small volume: one allocation and one upload, which Init of a small volume waits for longest
+    std::vector<int> state;
+    state.reserve(96 + 4 * (bricks.size() + split.size()));
+    state.resize(96, 0);
+    append_bricks(bricks, state);
+    append_bricks(split, state);
+    const size_t atCells = state.size();
     if (umpa::cells_possible(vx, vy, vz)) {
       const auto cells = umpa::host::make_cell_blocks(vx, vy, vz);
       op->nCells = (int)(cells.size() / 2);
@@ -213,9 +230,7 @@ int umpa_fr_init(umpa_fr_op *op, const umpa_fr_desc *desc, const umpa_fr_setting
       op->nCore = (int)(cells.size() / 2);
       state.insert(state.end(), cells.begin(), cells.end());
     }
-    hipError_t e = upload_bricks(bricks, &op->dBricks);
-    if (e == hipSuccess) e = upload_bricks(split, &op->dBricksSplit);
-    if (e == hipSuccess) e = hipMalloc(&op->dState, state.size() * sizeof(int));
+    hipError_t e = hipMalloc(&op->dState, state.size() * sizeof(int));
     if (e == hipSuccess)
       e = hipMemcpy(op->dState, state.data(), state.size() * sizeof(int), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
@@ -224,8 +239,10 @@ int umpa_fr_init(umpa_fr_op *op, const umpa_fr_desc *desc, const umpa_fr_setting
     }
     op->dCounter = op->dState;
     op->dUpdates = reinterpret_cast<unsigned long long *>(op->dState + 64);
-    op->dCells = op->nCells > 0 ? op->dState + 96 : nullptr;
-    op->dCore = op->nCore > 0 ? op->dState + 96 + 2 * op->nCells : nullptr;
+    op->dBricks = op->dState + 96;
+    op->dBricksSplit = op->dBricks + 4 * bricks.size();
+    op->dCells = op->nCells > 0 ? op->dState + atCells : nullptr;
+    op->dCore = op->nCore > 0 ? op->dState + atCells + 2 * op->nCells : nullptr;
     op->nBricksSplit = (int)split.size();
     op->nBricks = (int)bricks.size();
     op->nb = fr_footprint(*s);
@@ -575,15 +592,15 @@ static int fr_autotune_impl(umpa_fr_op *op, const void *fft, const float *scales
     int *items = nullptr;
     e = upload_bricks(bricks, &items);
     if (e != hipSuccess) return from_hip(e);
-    int *&dst = v.fastMath ? op->dBricksSplit : op->dBricks;
     // executes already enqueued on the stream may still read the old schedule
     e = hipStreamSynchronize(op->stream);
     if (e != hipSuccess) {
       (void)hipFree(items);
       return from_hip(e);
     }
-    (void)hipFree(dst);
-    dst = items;
+    (void)hipFree(op->dTuned[v.fastMath ? 1 : 0]);
+    op->dTuned[v.fastMath ? 1 : 0] = items;
+    (v.fastMath ? op->dBricksSplit : op->dBricks) = items;
     (v.fastMath ? op->nBricksSplit : op->nBricks) = (int)bricks.size();
   } catch (const std::bad_alloc &) {
     return UMPA_ERR_OUT_OF_MEMORY;
@@ -640,9 +657,9 @@ int umpa_fr_set_sched_params(umpa_fr_op *op, int strategy, const umpa_fr_sched_p
       (void)hipFree(items);
       return from_hip(e);
     }
-    int *&dst = slot == 1 ? op->dBricksSplit : op->dBricks;
-    (void)hipFree(dst);
-    dst = items;
+    (void)hipFree(op->dTuned[slot]);
+    op->dTuned[slot] = items;
+    (slot == 1 ? op->dBricksSplit : op->dBricks) = items;
     (slot == 1 ? op->nBricksSplit : op->nBricks) = (int)bricks.size();
     op->params[slot] = sp;
     return UMPA_OK;

@@ -222,10 +222,11 @@ int umpa_fr_batch_num_steps(umpa_fr_batch *b, uint32_t *steps);
 /* counting variant for the next execute / step (bypasses the graph); result after it */
 int umpa_fr_batch_set_count_updates(umpa_fr_batch *b, int enable);
 int umpa_fr_batch_last_updates(umpa_fr_batch *b, uint64_t *updates);
-/* Bounded launches: with itemsPerWave > 0 every wavefront of the batch's later launches (and
- * plans) leaves after that many work items, and the grid covers all items, so CUs come free
- * while a launch runs and another stream's launches (a second batch) start at once instead of
- * after it; 0 (the default) keeps one persistent workgroup per CU.  Results do not change. */
+/* Bounded launches: with itemsPerWave > 0 every workgroup of the batch's later launches (and
+ * plans) leaves after that many work items for each of its wavefronts, and the grid covers all
+ * items, so CUs come free while a launch runs and another stream's launches (a second batch)
+ * start at once instead of after it; 0 (the default) keeps one persistent workgroup per CU.
+ * Results do not change. */
 int umpa_fr_batch_set_wave_items(umpa_fr_batch *b, uint32_t itemsPerWave);
 /* Persistent launches (itemsPerWave 0) of the batch's later steps (and plans) use at most this
  * many workgroups, one per CU, leaving the other CUs to another stream's launches; 0 (the

@@ -147,7 +147,7 @@ struct umpa_fr_batch {
   std::map<std::tuple<int, int, int, float>, umpa::host::BrickSet> cands;
   std::vector<umpa::host::BrickOrigin> schedBuf;  // make_schedule's output, reused
   umpa::host::SchedParams params[2];  // schedule knobs for exact / fast-math launches
-  int waveItems = 0;  // items per wave before it leaves (0: persistent workgroups)
+  int waveItems = 0;  // a workgroup leaves after this many items a wave (0: persistent)
   int maxWorkgroups = 0;  // persistent launches: at most this many workgroups (0: one per CU)
 
   // static plan

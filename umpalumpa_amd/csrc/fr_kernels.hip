@@ -28,6 +28,8 @@
 // there).
 #include "fr_cell.hpp"
 
+#include <algorithm>
+
 namespace umpa {
 
 constexpr int kMaxLdsTable = kFrMaxLdsTable;  // floats next to the per-wave state; larger tables stay global
@@ -101,21 +103,36 @@ __device__ __forceinline__ int first_after_core(const FrLaunch &l, int number, i
   return number >= core ? number - core : number + claimed - core;
 }
 
-// Bounded launches (l.waveItems items per wavefront, the grid covering the items) need no counter:
-// workgroups go by groups of one per CU, a group takes the next items in order and deals them out
-// across its workgroups, so that a workgroup's wavefronts have items of about the same cost and
-// the heaviest lie on different CUs.  (With the counter, a four-job serving tick of 63,000 items
-// made 95,000 claims: 1737 -> 1635 us.)
+// Bounded launches (l.waveItems items for each of a workgroup's wavefronts, the grid covering the
+// items) need no global counter: workgroups go by groups of one per CU, a group takes the next
+// items in order and deals them out across its workgroups, so that a workgroup's items cost about
+// the same and the heaviest lie on different CUs.  (With the counter, a four-job serving tick of
+// 63,000 items made 95,000 claims: 1737 -> 1635 us.)  A workgroup's wavefronts take its items in
+// order from a count in LDS: its LDS comes free only with its last wavefront, and items of one
+// estimated cost differ (the same tick, two items each: 1665 -> 1580 us).
 struct DealtItems {
-  int first, step;
+  int first, step, n;  // the workgroup's items: first + k step, k < n
 };
 __device__ __forceinline__ DealtItems deal_items(const FrLaunch &l, int waves)
 {
   const int group = (int)blockIdx.x / l.numCUs, in = (int)blockIdx.x - group * l.numCUs;
   const int start = group * l.numCUs;
   const int size = min(l.numCUs, (int)gridDim.x - start);
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  return { start * waves * l.waveItems + wave * size + in, waves * size };
+  const int n = waves * l.waveItems;
+  return { start * n + in, size, n };
+}
+
+// Item k of the workgroup's (nItems: none left).
+__device__ __forceinline__ int dealt_item(const FrLaunch &l, const DealtItems &d, int k)
+{
+  return k < d.n ? min(d.first + k * d.step, l.nItems) : l.nItems;
+}
+
+__device__ __forceinline__ int next_dealt(const FrLaunch &l, const DealtItems &d, int *taken, int lane)
+{
+  int k = 0;
+  if (lane == 0) k = atomicAdd(taken, 1);
+  return dealt_item(l, d, __builtin_amdgcn_readfirstlane(k));
 }
 
 // ---- the brick's steps shared by the insertion kernels ----------------------------------------
@@ -337,11 +354,17 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
     }
   }
   const bool bounded = kBatched && l.waveItems > 0;
-  DealtItems dealt{ !kFastMath && !kBatched ? first_after_core(l, number, claimed) : number, 0 };
-  if (bounded) dealt = deal_items(l, kWaves);
-  int left = l.waveItems;
-  for (int b = dealt.first; b < l.nItems;
-       b = bounded ? (--left > 0 ? b + dealt.step : l.nItems) : claim_item(l, lane, claimed)) {
+  DealtItems dealt{};
+  __shared__ int s_taken;  // bounded launches: items of the workgroup taken so far
+  int begin = !kFastMath && !kBatched ? first_after_core(l, number, claimed) : number;
+  if (bounded) {
+    dealt = deal_items(l, kWaves);
+    if (threadIdx.x == 0) s_taken = kWaves;
+    __syncthreads();
+    begin = dealt_item(l, dealt, __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)));
+  }
+  for (int b = begin; b < l.nItems;
+       b = bounded ? next_dealt(l, dealt, &s_taken, lane) : claim_item(l, lane, claimed)) {
     const int4 bo = make_uniform(reinterpret_cast<const int4 *>(l.items)[b]);
     // work item: brick 8 x 8 x depth at (bo.x, bo.y, bo.z & 0xffff) of job bo.z >> 16; heavy
     // bricks run at raised wave priority; a brick split into `parts` slice ranges accumulates
@@ -560,11 +583,17 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fr_insert_carry_kernel(FrJob j
 
   const int number = wave_number(), claimed = kWaves * (int)gridDim.x;
   const bool bounded = kBatched && l.waveItems > 0;
-  DealtItems dealt{ number, 0 };
-  if (bounded) dealt = deal_items(l, kWaves);
-  int left = l.waveItems;
-  for (int b = dealt.first; b < l.nItems;
-       b = bounded ? (--left > 0 ? b + dealt.step : l.nItems) : claim_item(l, lane, claimed)) {
+  DealtItems dealt{};
+  __shared__ int s_taken;  // bounded launches: items of the workgroup taken so far
+  int begin = number;
+  if (bounded) {
+    dealt = deal_items(l, kWaves);
+    if (threadIdx.x == 0) s_taken = kWaves;
+    __syncthreads();
+    begin = dealt_item(l, dealt, __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)));
+  }
+  for (int b = begin; b < l.nItems;
+       b = bounded ? next_dealt(l, dealt, &s_taken, lane) : claim_item(l, lane, claimed)) {
     const int4 bo = make_uniform(reinterpret_cast<const int4 *>(l.items)[b]);
     const FrJob a = kBatched ? make_uniform(l.jobs[bo.z >> 16]) : job0;
     const int s0 = a.spaceBegin, s1 = a.spaceEnd;
@@ -1061,6 +1090,8 @@ hipError_t launch_fr_insert(const FrJob &job, const FrLaunch &l, const FrVariant
   FrJob j = job;
   FrLaunch ll = l;
   ll.numCUs = numCUs;
+  if (l.waveItems > 0)  // (a workgroup's count of items stays an int)
+    ll.waveItems = (int)std::min<int64_t>(l.waveItems, ((int64_t)l.nItems + waves - 1) / waves);
   void *args[] = { &j, &ll };
   return hipLaunchKernel(k, dim3(blocks), dim3(64 * waves), args, shmem, st);
 }

@@ -43,7 +43,7 @@ struct FrLaunch {
   unsigned long long *updates;  // voxel-update counter (counting variant only)
   const float *table;   // blob table (kLookup)
   int nTable;
-  int waveItems;        // items per wave before it leaves (0: until the items run out)
+  int waveItems;        // a workgroup leaves after this many items a wave (0: when they run out)
   int maxBlocks;        // persistent launches: at most this many workgroups (0: one per CU)
   int numCUs;           // set by the launch
   const int *cells;     // int2 {x | y << 16, z | edge << 16} per block of the volume, heaviest first

@@ -387,9 +387,9 @@ class FRBatch:
               "set_sched_params")
 
     def set_wave_items(self, items_per_wave: int) -> None:
-        """Bounded launches (umpa_fr_batch_set_wave_items): every wavefront leaves after that
-        many work items (0: persistent workgroups), so another stream's launches get CUs while
-        this batch's launches run."""
+        """Bounded launches (umpa_fr_batch_set_wave_items): a workgroup leaves after that many
+        work items for each of its wavefronts (0: persistent workgroups), so another stream's
+        launches get CUs while this batch's launches run."""
         check(_lib.load().umpa_fr_batch_set_wave_items(self._h, items_per_wave),
               "set_wave_items")
 

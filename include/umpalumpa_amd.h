@@ -249,7 +249,8 @@ void umpa_fr_batch_destroy(umpa_fr_batch *b);
  * reused without timing.  Results are the same, bit for bit, under every schedule and kernel
  * knob for UMPA_FR_EXACT. */
 typedef struct umpa_fr_sched_params {
-  float depthScale;  /* bricks 8x8x{8,4,2,1} beyond radius {48,24,12} x depthScale */
+  float depthScale;  /* bricks 8x8x{8,4,2,1} beyond radius {48,24,12} x depthScale, times a
+                        scale of the launch's own (by volume, spaces and strategy) */
   int32_t priority;  /* heavy bricks at raised wave priority */
   int32_t maxParts;  /* split heavy bricks into at most this many slice ranges (fast math) */
   float splitAt;     /* ... above splitAt x one wavefront's fair share of the launch */
@@ -266,7 +267,7 @@ typedef struct umpa_fr_sched_params {
 
 enum {
   UMPA_FR_KERNEL_AUTO = 0,   /* staged for UMPA_FR_EXACT, carried for fast-math FP32, else pair;
-                                small volumes of a plain operation (up to 129^3 voxels, by mode
+                                small volumes of a plain operation (up to 121^3 voxels, by mode
                                 and number of spaces) run eight spaces at a time in cells of
                                 2 x 2 x 2 voxels, whatever the schedule knobs */
   UMPA_FR_KERNEL_PAIR = 1,   /* one queue of slab voxels per (brick, space), 16 or 12 waves */

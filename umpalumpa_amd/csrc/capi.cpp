@@ -190,8 +190,11 @@ static std::vector<umpa::host::BrickOrigin> op_schedule(const umpa_fr_op *op, bo
                                                         const umpa::host::SchedParams &sp)
 {
   const umpa_fr_desc &d = op->desc;
-  return umpa::host::make_brick_schedule((int)d.volume.x, (int)d.volume.y, (int)d.volume.z, split,
-                                         sp, split ? 0.f : op_core(d));
+  const int vx = (int)d.volume.x, vy = (int)d.volume.y, vz = (int)d.volume.z;
+  umpa::host::SchedParams scaled = sp;
+  scaled.depthScale *=
+    umpa::host::plain_depth_scale(vx, vy, vz, d.traverseSpaces, op->settings, split);
+  return umpa::host::make_brick_schedule(vx, vy, vz, split, scaled, split ? 0.f : op_core(d));
 }
 
 int umpa_fr_init(umpa_fr_op *op, const umpa_fr_desc *desc, const umpa_fr_settings *s)

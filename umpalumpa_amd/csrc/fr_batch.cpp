@@ -215,7 +215,10 @@ void build_step(umpa_fr_batch *b, const std::vector<JobInfo> &infos,
       rec.spaceEnd = s1;
       if (sp.boxFixed) rec.shiftBox = 0;
       recs.push_back(rec);
-      work.push_back({ &b->candidates(rec.vx, rec.vy, rec.vz, sp.depthScale), (int)k,
+      const float depth =
+        sp.depthScale *
+        umpa::host::batch_depth_scale(rec.vx, rec.vy, rec.vz, b->waveItems > 0);
+      work.push_back({ &b->candidates(rec.vx, rec.vy, rec.vz, depth), (int)k,
                        (double)(s1 - s0) });
     }
     umpa::host::make_schedule(work, first.v.fastMath, sp, b->schedBuf);

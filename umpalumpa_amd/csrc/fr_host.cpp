@@ -279,6 +279,42 @@ float core_radius(int vx, int vy, int vz)
   return voxels <= cube(161) ? 17.f : voxels <= cube(225) ? 11.f : 0.f;
 }
 
+namespace {
+
+bool at_most_cube(int vx, int vy, int vz, int64_t n) { return (int64_t)vx * vy * vz <= n * n * n; }
+
+}  // namespace
+
+// Thin bricks even out the work but fill fewer of a gather's lanes and cost a set-up each.  Volumes
+// up to 165^3 have few bricks for 4,096 wavefronts and want them thinner farther out, if there are
+// enough spaces to pay for the set-up (us at scale 1 / 1.4: box 128, 1,500 slices exact 661 / 579,
+// fast math 686 / 580, FP16 767 / 642; 400 211 / 187, 197 / 190, 214 / 200; 100 109 / 116, 110 /
+// 124; 144, 1,500 FP16 732 / 676; 160, 400 exact 295 / 269), or if the blob is evaluated, whose
+// chain is longer (128, 100 196 / 155; 160, 100 238 / 221); the nearest pixel's is shorter (128,
+// 400 177 / 193).  Larger ones have bricks enough and want them thicker (at 1 / 0.7 / 0.5: box 176,
+// 1,500 exact 903 / 820 / 946, fast math 791 / 775 / 930; 192 983 / 988 / 986, 944 / 923 / 932;
+// 256 1741 / 1725 / 1820, 1565 / 1543 / 1529; 320, 1,500 FP16 2474 / 2443 / 2428; 192, 400, nearest
+// pixel 300 / 272 / 298): under the exact strategy, which splits none, not below 0.7.
+float plain_depth_scale(int vx, int vy, int vz, uint64_t spaces, const umpa_fr_settings &s,
+                        bool split)
+{
+  const bool nearest = s.type == UMPA_FR_FAST;
+  const bool evaluated = !nearest && s.interpolation == UMPA_FR_DYNAMIC;
+  if (at_most_cube(vx, vy, vz, 165))
+    return !nearest && (evaluated || spaces >= 250) ? 1.4f : 1.f;
+  return split && !at_most_cube(vx, vy, vz, 209) ? 0.5f : 0.7f;
+}
+
+// A batch's volumes fill the GPU together, so small ones need no thinner bricks (seven FP16 jobs of
+// boxes 64 to 320 at 1 / 1.4 for boxes up to 165 and 0.5 for the others: 3881 / 3974 us; all at 1:
+// 3930; the small ones at 0.7, 4150, lose a launch's last chunks, where they are alone).  Bounded
+// launches, whose workgroups turn over, want fewer items (a tick of four jobs, boxes 96 to 256, at
+// 1 / 0.7 / 0.5: FP16 1578 / 1512 / 1463 us, exact 2221 / 2096 / 2103).
+float batch_depth_scale(int vx, int vy, int vz, bool bounded)
+{
+  return !bounded && at_most_cube(vx, vy, vz, 165) ? 1.f : 0.5f;
+}
+
 std::vector<BrickCand> brick_candidates(int vx, int vy, int vz, float depthScale, float core)
 {
   // Bricks are 8 x 8 x D columns, D in {8, 4, 2, 1}.  A voxel at distance R from the centre

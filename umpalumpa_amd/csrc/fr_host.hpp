@@ -43,6 +43,7 @@ struct BrickOrigin {
 // Tunable knobs of the work-item schedule and of the kernel (the autotuner's search space).
 struct SchedParams {
   float depthScale = 1.f;  // brick depth 8 / 4 / 2 / 1 beyond radius 48 / 24 / 12 times this
+                           // (times the launch's own scale: *_depth_scale)
   bool priority = true;    // run bricks above a quarter of a wave's fair share at priority 2
   int maxParts = 16;       // split heavy bricks into at most this many slice ranges (fast math)
   float splitAt = 0.5f;    // ... when their cost exceeds splitAt times a wave's fair share
@@ -68,6 +69,12 @@ std::vector<BrickCand> brick_candidates(int vx, int vy, int vz, float depthScale
 // each: x | y << 16 and z.
 float core_radius(int vx, int vy, int vz);
 std::vector<int> core_cells(int vx, int vy, int vz, float core);
+
+// Scale of the brick depths' radii: of a plain operation's launches of up to `spaces` spaces, by
+// the blob (of the settings) and whether heavy bricks are split; of a volume in a batch's launch.
+float plain_depth_scale(int vx, int vy, int vz, uint64_t spaces, const umpa_fr_settings &s,
+                        bool split);
+float batch_depth_scale(int vx, int vy, int vz, bool bounded);
 
 // A volume's bricks sorted by estimated cost (heaviest first, ties in brick order) and the
 // costs' sum: what make_schedule needs of a volume, built once per volume shape.

@@ -1015,14 +1015,15 @@ hipError_t prepare_fr_insert(const FrVariant &v, int nTable)
 
 // Does this launch run the small-problem kernel?  The brick kernels take a space per 0.3 to 1.2 us
 // (their heaviest brick's chain) whatever the volume, the cell kernel a fixed 4 us per round of
-// blocks and less per space.  Measured (us, bricks / cells at r 1.9, slices): exact, box 48 20
-// 28 / 29, 400 206 / 90; 64 20 32 / 43, 100 66 / 53, 400 188 / 107; 80 100 64 / 68, 400 184 / 136;
-// 90 400 193 / 163; 100 400 186 / 188; r 1.5 100 1,004 336 / 299, 112 1,000 326 / 362; r 2.5 100
-// 100 179 / 149, 112 600 603 / 562, 128 600 647 / 709.  Fast math: 64 20 37 / 43, 100 111 / 50,
-// 80 100 65 / 66, 100 100 87 / 93, 400 213 / 175; 112 400 219 / 208; 128 1,500 691 / 826; FP16
-// 112 400 232 / 196, 128 1,500 765 / 766.  Blob evaluated: 80 50 104 / 78, 100 50 116 / 128, 400
-// 518 / 328; 128 300 386 / 404, 400 542 / 494.  Nearest: 64 400 131 / 122, 80 400 140 / 126, 100
-// 400 147 / 184.  So, with V the volume's mean extent: from (V - from) * slope spaces, up to a V.
+// blocks and less per space.  Measured (us, bricks / cells at r 1.9, slices): exact, box 64 60
+// 50 / 48, 150 92 / 63; 80 60 55 / 67, 150 87 / 78, 400 167 / 144, 1,200 442 / 365; 90 150 90 / 96,
+// 400 149 / 171; 100 400 172 / 198; r 1.5 90 150 79 / 85, 1,200 368 / 330; 100 1,200 405 / 387, 112
+// 390 / 464; r 2.5 100 150 228 / 186, 112 150 202 / 233, 1,200 1165 / 1101, 128 1218 / 1398.  Fast
+// math: 64 60 73 / 47; 80 60 58 / 65, 150 89 / 75; 100 150 102 / 104, 400 188 / 179, 1,200 482 /
+// 462; 112 400 189 / 211; FP16 100 1,200 554 / 433, 112 400 206 / 201, 1,200 541 / 514; 128 400 198 /
+// 253.  Blob evaluated: 80 60 106 / 75, 100 60 114 / 117, 150 192 / 152; 112 60 127 / 146, 150 196 /
+// 188, 400 392 / 334; 128 150 198 / 247.  Nearest: 64 150 62 / 54, 80 150 60 / 65, 1,200 485 / 351;
+// 90 414 / 430.  So, with V the volume's mean extent: from (V - from) * slope spaces, up to a V.
 bool use_cells(const FrJob &job, const FrLaunch &l, const FrVariant &v)
 {
   if (l.nCells <= 0 || v.batched || v.count || v.kernel != kKernelAuto || v.tableGlobal) return false;
@@ -1033,11 +1034,12 @@ bool use_cells(const FrJob &job, const FrLaunch &l, const FrVariant &v)
     float from, slope;
   };
   const Rule rule = v.mode == kModeNearest  ? Rule{ 85, 45.f, 4.f }
-                    : v.mode != kModeLookup ? Rule{ 129, 75.f, 6.f }
-                    : v.fastMath            ? Rule{ 121, 55.f, 5.f }
+                    : v.mode != kModeLookup ? Rule{ 121, 85.f, 5.f }
+                    : v.half                ? Rule{ 115, 55.f, 5.f }
+                    : v.fastMath            ? Rule{ 105, 55.f, 5.f }
                     : v.nb == 3             ? Rule{ 105, 45.f, 4.f }
-                    : v.nb == 4             ? Rule{ 97, 45.f, 4.f }
-                                            : Rule{ 121, 45.f, 1.5f };
+                    : v.nb == 4             ? Rule{ 87, 45.f, 4.f }
+                                            : Rule{ 121, 45.f, 3.f };
   const int64_t voxels = (int64_t)job.vx * job.vy * job.vz;
   if (voxels > (int64_t)rule.upTo * rule.upTo * rule.upTo) return false;
   const float spaces = (float)(job.spaceEnd - job.spaceBegin);

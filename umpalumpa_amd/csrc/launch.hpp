@@ -86,7 +86,7 @@ hipError_t launch_fr_insert(const FrJob &job, const FrLaunch &l, const FrVariant
 // May a volume of these extents run the small-problem kernel (its host then keeps the block list)?
 inline bool cells_possible(int vx, int vy, int vz)
 {
-  return (int64_t)vx * vy * vz <= (int64_t)129 * 129 * 129 && vx < 65536 && vy < 65536 && vz < 32768;
+  return (int64_t)vx * vy * vz <= (int64_t)121 * 121 * 121 && vx < 65536 && vy < 65536 && vz < 32768;
 }
 // Does the launch run the small-problem kernel (which needs no `prepare`)?
 bool use_cells(const FrJob &job, const FrLaunch &l, const FrVariant &v);

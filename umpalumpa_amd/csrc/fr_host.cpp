@@ -10,6 +10,7 @@
 #include <cfloat>
 #include <cmath>
 #include <cstdlib>
+#include <utility>
 #include <cstring>
 #include <functional>
 #include <fstream>
@@ -380,10 +381,33 @@ std::vector<int> core_cells(int vx, int vy, int vz, float core)
 
 BrickSet make_brick_set(int vx, int vy, int vz, float depthScale, float core)
 {
+  // a stable sort by cost, most first: costs are positive, so their bits grow with them, and the
+  // bits' complement sorts by radix, 11 bits at a time (box 64, 1,832 bricks and 256, 36,325: 181 ->
+  // 64 us and 2.7 -> 1.4 ms with the candidates)
+  const std::vector<BrickCand> cand = brick_candidates(vx, vy, vz, depthScale, core);
+  const size_t n = cand.size();
+  std::vector<uint64_t> keys(n), other(n);  // cost bits, complemented, and the brick's index
+  constexpr int kBits = 11, kPasses = 3;
+  std::vector<uint32_t> start((size_t)kPasses << kBits, 0);
+  auto digit = [](uint64_t key, int pass) {
+    return (size_t)pass << kBits | (size_t)(key >> (32 + kBits * pass) & ((1u << kBits) - 1));
+  };
+  for (size_t i = 0; i < n; ++i) {
+    uint32_t bits;
+    std::memcpy(&bits, &cand[i].est, 4);
+    keys[i] = (uint64_t)~bits << 32 | i;
+    for (int p = 0; p < kPasses; ++p) ++start[digit(keys[i], p)];
+  }
+  for (int p = 0; p < kPasses; ++p) {
+    uint32_t at = 0;
+    for (size_t d = (size_t)p << kBits; d < (size_t)(p + 1) << kBits; ++d)
+      at += std::exchange(start[d], at);
+    for (uint64_t key : keys) other[start[digit(key, p)]++] = key;
+    keys.swap(other);
+  }
   BrickSet set;
-  set.sorted = brick_candidates(vx, vy, vz, depthScale, core);
-  std::stable_sort(set.sorted.begin(), set.sorted.end(),
-                   [](const BrickCand &a, const BrickCand &b) { return a.est > b.est; });
+  set.sorted.reserve(n);
+  for (uint64_t key : keys) set.sorted.push_back(cand[(size_t)(uint32_t)key]);
   for (const BrickCand &b : set.sorted) set.estSum += b.est;
   return set;
 }

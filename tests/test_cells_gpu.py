@@ -158,3 +158,22 @@ def test_dealt_items_cover_every_brick(items, strategy):
                 assert v.tobytes() == ref[k][0].tobytes() and w.tobytes() == ref[k][1].tobytes()
             else:
                 assert rel_l2(v, ref[k][0]) <= 1e-5 and rel_l2(w, ref[k][1]) <= 1e-5
+
+
+@pytest.mark.parametrize("interp,typ", [(F.FR_LOOKUP, F.FR_PRECISE), (F.FR_DYNAMIC, F.FR_PRECISE),
+                                        (F.FR_DYNAMIC, F.FR_FAST)])
+@pytest.mark.parametrize("box,n", [(2, 60), (4, 61), (10, 95), (56, 97), (58, 64), (16, 1057)])
+def test_shared_cells(box, n, interp, typ):
+    """Cells that four wavefronts share (from 60 spaces on, volumes up to 57^3, or 85^3 without a
+    table): cells outside the volume, rounds of 32 spaces with a remainder, several tiles; the same
+    operation with fewer spaces than a round, and onto values it holds."""
+    s = settings(interp, typ, 15.0, 1.9)
+    fft, spaces, desc, table = problem(box, n, s, seed=box + n)
+    spaces["weight"][::3] = 0.5
+    ov, ow, _ = run_oracle(s, fft, spaces, table, box)
+    for chunks in (1, 5):
+        v, w, _ = run_hip(s, fft, spaces, desc, table, box, chunks=chunks)
+        assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()
+    if interp == F.FR_LOOKUP:
+        v, w, _ = run_hip(s, fft, spaces, desc, table, box, strategy=F.FR_FAST_MATH)
+        assert rel_l2(v, ov) <= 1e-5 and rel_l2(w, ow) <= 1e-5

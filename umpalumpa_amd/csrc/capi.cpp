@@ -55,6 +55,7 @@ struct umpa_fr_op {
   unsigned long long *dUpdates = nullptr;
   int *dCells = nullptr;       //   small volumes: the blocks of the small-problem kernel
   int nCells = 0;
+  bool cellsShared = false;
   int *dCore = nullptr;        //   the core's cells (exact launches)
   int nCore = 0;
   int nb = 0;
@@ -224,7 +225,8 @@ int umpa_fr_init(umpa_fr_op *op, const umpa_fr_desc *desc, const umpa_fr_setting
     append_bricks(split, state);
     const size_t atCells = state.size();
     if (umpa::cells_possible(vx, vy, vz)) {
-      const auto cells = umpa::host::make_cell_blocks(vx, vy, vz);
+      op->cellsShared = umpa::host::share_cells(vx, vy, vz, desc->traverseSpaces, *s);
+      const auto cells = umpa::host::make_cell_blocks(vx, vy, vz, op->cellsShared);
       op->nCells = (int)(cells.size() / 2);
       state.insert(state.end(), cells.begin(), cells.end());
     }
@@ -396,6 +398,7 @@ static int fr_execute_impl(umpa_fr_op *op, const void *fft, const float *scales,
   }
   l.cells = op->dCells;
   l.nCells = op->nCells;
+  l.cellsShared = op->cellsShared;
   l.cellCounter = op->dCounter + 32;
   l.counter = op->dCounter;
   l.updates = op->dUpdates;
@@ -544,6 +547,7 @@ static int fr_autotune_impl(umpa_fr_op *op, const void *fft, const float *scales
       }
       l.cells = op->dCells;
       l.nCells = op->nCells;
+      l.cellsShared = op->cellsShared;
       l.cellCounter = op->dCounter + 32;
       l.counter = op->dCounter;
       l.updates = op->dUpdates;

@@ -40,26 +40,26 @@ __device__ __forceinline__ CellSpace load_space(const FrJob &a, int index, bool 
   return s;
 }
 
-// Does space `si` reach the block of edge `e` at (x0, y0, z0)?  As cull_space of the brick kernels;
-// `inside` as brick_inside.
-__device__ __forceinline__ bool cull_block(const FrJob &a, int si, int x0, int y0, int z0, int e,
-                                           int cxi, int cyi, bool &inside)
+// Does space `si` reach the block of `wide` columns and edge `e` otherwise at (x0, y0, z0)?  As
+// cull_space of the brick kernels; `inside` as brick_inside.
+__device__ __forceinline__ bool cull_block(const FrJob &a, int si, int x0, int y0, int z0, int wide,
+                                           int e, int cxi, int cyi, bool &inside)
 {
   const umpa_traverse_space &sp = a.spaces[si];
   const float(*t)[3] = sp.transformInv;
-  const float half = 0.5f * (float)(e - 1);
-  const float cx = (float)(x0 - cxi) + half, cy = (float)(y0 - cyi) + half,
+  const float half = 0.5f * (float)(e - 1), halfX = 0.5f * (float)(wide - 1);
+  const float cx = (float)(x0 - cxi) + halfX, cy = (float)(y0 - cyi) + half,
               cz = (float)(z0 - cyi) + half;
   const float norm = sqrtf(cx * cx + cy * cy + cz * cz);
-  const float dmin = fmaxf(norm - 1.7321f * half, 0.f);
+  const float dmin = fmaxf(norm - 1.7321f * halfX, 0.f);  // (wide >= e)
   const float eps = 0.02f + 1e-5f * norm;
   const float qz = t[2][0] * cx + t[2][1] * cy + t[2][2] * cz;
-  const float ez = half * (fabsf(t[2][0]) + fabsf(t[2][1]) + fabsf(t[2][2]));
+  const float ez = halfX * fabsf(t[2][0]) + half * (fabsf(t[2][1]) + fabsf(t[2][2]));
   const float qx = t[0][0] * cx + t[0][1] * cy + t[0][2] * cz;
-  const float ex = half * (fabsf(t[0][0]) + fabsf(t[0][1]) + fabsf(t[0][2]));
+  const float ex = halfX * fabsf(t[0][0]) + half * (fabsf(t[0][1]) + fabsf(t[0][2]));
   const float mds = sp.maxDistanceSqr;
   const int proj = sp.projectionIndex, dir = sp.dir;
-  const int x1 = x0 + e - 1, y1 = y0 + e - 1, z1 = z0 + e - 1;
+  const int x1 = x0 + wide - 1, y1 = y0 + e - 1, z1 = z0 + e - 1;
   const int mx = max(abs(x0 - cxi), abs(x1 - cxi));
   const int my = max(abs(y0 - cyi), abs(y1 - cyi));
   const int mz = max(abs(z0 - cyi), abs(z1 - cyi));
@@ -113,6 +113,68 @@ __device__ __forceinline__ Cell make_cell(const FrJob &a, int x0, int y0, int z0
   return k;
 }
 
+// The lane's pair: does space `sp` reach the cell's voxel, and where does it lie in the slice's frame?
+template <int kMode>
+__device__ __forceinline__ bool cell_pair(const Cell &k, const FrJob &a, const CellSpace &sp, bool act,
+                                          float &qx, float &qy, float &zs)
+{
+  const umpa_traverse_space &rec = a.spaces[sp.index];
+  bool hit;
+  if constexpr (kMode == kModeNearest) {
+    const float dsq = k.px * k.px + k.py * k.py + k.pz * k.pz;
+    qx = sp.t[0][0] * k.px + sp.t[0][1] * k.py + sp.t[0][2] * k.pz;
+    qy = sp.t[1][0] * k.px + sp.t[1][1] * k.py + sp.t[1][2] * k.pz;
+    zs = 0.f;
+    hit = act && !(dsq > rec.maxDistanceSqr) && !(qx < 0.f) && visited_nearest(rec, k.x, k.y, k.z);
+  } else {
+    hit = act && blob_predicate<false>(rec, sp.t, a.c, k.x, k.y, k.z, k.px, k.py, k.pz, sp.inside,
+                                       qx, qy, zs);
+  }
+  return hit;
+}
+
+// Its contribution (-0, which changes no float, for a pair that misses); called by the whole
+// wavefront.  `blob`: kBlobList floats of the wavefront's LDS for the evaluated blob modes.
+template <int kMode, int kOrder, int kNB, bool kHalf, bool kFastMath, bool kTableLds, bool kShift,
+          int kRows>
+__device__ __forceinline__ Contribution cell_gather(const FrJob &a, const CellSpace &sp, bool hit,
+                                                    float qx, float qy, float zs, float *blob,
+                                                    int nTable, __amdgpu_buffer_rsrc_t rsrc,
+                                                    const float *tbl, int lane)
+{
+  Contribution o{ -0.f, -0.f, -0.f };
+  if constexpr (evaluates_blob(kMode)) {
+    const Contribution got = gather_evaluated<kMode, kOrder>(a, rsrc, blob, lane, hit, qx, qy, zs,
+                                                             sp.weight, sp.off);
+    if (hit) o = got;
+  } else if (hit) {
+    if constexpr (kMode == kModeNearest) {
+      o = gather_nearest<kHalf>(a, rsrc, qx, qy, sp.weight, sp.scale, sp.off);
+    } else {
+      // (a weight of 1 changes no product, so one copy of the gather serves all)
+      o = gather_update<kMode, kOrder, kNB, kHalf, kFastMath, kTableLds, kShift, kRows>(
+        a, nTable, rsrc, tbl, qx, qy, zs, sp.weight, false, sp.scale, sp.off);
+    }
+  }
+  return o;
+}
+
+// Adds eight spaces' contributions (`part`, 192 floats: component, voxel, space) in order; lanes
+// 0..23, each its sum.
+__device__ __forceinline__ void cell_add(Cell &k, const float *part, int lane)
+{
+  const float4 p = reinterpret_cast<const float4 *>(part)[2 * lane],
+               q = reinterpret_cast<const float4 *>(part)[2 * lane + 1];
+  k.acc = k.acc + p.x;
+  k.acc = k.acc + p.y;
+  k.acc = k.acc + p.z;
+  k.acc = k.acc + p.w;
+  k.acc = k.acc + q.x;
+  k.acc = k.acc + q.y;
+  k.acc = k.acc + q.z;
+  k.acc = k.acc + q.w;
+}
+
 // Takes the queue's spaces eight at a time while at least `least` are pending: predicate and
 // gather per lane, the contributions through LDS (`part`, 192 floats) to the lanes that own the
 // sums, which add the eight spaces' in order, so a voxel receives its spaces in index order.  A
@@ -142,56 +204,21 @@ __device__ __forceinline__ void cell_take(Cell &k, const FrJob &a, int base, con
     head = (head + n) & (kCellRing - 1);
     pend -= n;
 
-    const bool act = k.valid && s < n;
-    const umpa_traverse_space &rec = a.spaces[sp.index];
     float qx, qy, zs;
-    bool hit;
-    if constexpr (kMode == kModeNearest) {
-      const float dsq = k.px * k.px + k.py * k.py + k.pz * k.pz;
-      qx = sp.t[0][0] * k.px + sp.t[0][1] * k.py + sp.t[0][2] * k.pz;
-      qy = sp.t[1][0] * k.px + sp.t[1][1] * k.py + sp.t[1][2] * k.pz;
-      zs = 0.f;
-      hit = act && !(dsq > rec.maxDistanceSqr) && !(qx < 0.f) && visited_nearest(rec, k.x, k.y, k.z);
-    } else {
-      hit = act && blob_predicate<false>(rec, sp.t, a.c, k.x, k.y, k.z, k.px, k.py, k.pz, sp.inside,
-                                         qx, qy, zs);
-    }
+    const bool hit = cell_pair<kMode>(k, a, sp, k.valid && s < n, qx, qy, zs);
     if (!__any(hit)) continue;
     if constexpr (kCount) nupd += (unsigned long long)__popcll(__ballot(hit));
     if (!k.loaded) {
       if (k.owner) k.acc = *k.sum;
       k.loaded = true;
     }
-    Contribution o{ -0.f, -0.f, -0.f };
-    if constexpr (evaluates_blob(kMode)) {
-      const Contribution got = gather_evaluated<kMode, kOrder>(a, rsrc, blob, lane, hit, qx, qy, zs,
-                                                               sp.weight, sp.off);
-      if (hit) o = got;
-    } else if (hit) {
-      if constexpr (kMode == kModeNearest) {
-        o = gather_nearest<kHalf>(a, rsrc, qx, qy, sp.weight, sp.scale, sp.off);
-      } else {
-        // (a weight of 1 changes no product, so one copy of the gather serves all)
-        o = gather_update<kMode, kOrder, kNB, kHalf, kFastMath, kTableLds, kShift, kRows>(
-          a, nTable, rsrc, tbl, qx, qy, zs, sp.weight, false, sp.scale, sp.off);
-      }
-    }
+    const Contribution o = cell_gather<kMode, kOrder, kNB, kHalf, kFastMath, kTableLds, kShift, kRows>(
+      a, sp, hit, qx, qy, zs, blob, nTable, rsrc, tbl, lane);
     part[lane] = o.re;
     part[64 + lane] = o.im;
     part[128 + lane] = o.w;
     wave_sync();
-    if (lane < 24) {
-      const float4 p = reinterpret_cast<const float4 *>(part)[2 * lane],
-                   q = reinterpret_cast<const float4 *>(part)[2 * lane + 1];
-      k.acc = k.acc + p.x;
-      k.acc = k.acc + p.y;
-      k.acc = k.acc + p.z;
-      k.acc = k.acc + p.w;
-      k.acc = k.acc + q.x;
-      k.acc = k.acc + q.y;
-      k.acc = k.acc + q.z;
-      k.acc = k.acc + q.w;
-    }
+    if (lane < 24) cell_add(k, part, lane);
     wave_sync();
   } while (pend >= least);
 }
@@ -214,7 +241,7 @@ __device__ __forceinline__ void cell_item(const FrJob &a, int x0, int y0, int z0
   for (int base = sBegin; base < sEnd; base += 64) {
     const int si = base + lane;
     bool in = false;
-    const unsigned long long m = __ballot(si < sEnd && cull_block(a, si, x0, y0, z0, 2, cxi, cyi, in));
+    const unsigned long long m = __ballot(si < sEnd && cull_block(a, si, x0, y0, z0, 2, 2, cxi, cyi, in));
     if ((m >> lane) & 1ull)
       queue[lanes_below(m, (unsigned)(head + pend)) & (kCellRing - 1)] =
         (uint32_t)si | (in ? kInsideBit<uint32_t> : 0u);

@@ -9,7 +9,8 @@
 // chain is an eighth as long and a volume has 64 times the wavefronts' work items.
 //
 // A workgroup of eight wavefronts owns a block of 4 x 4 x 4 voxels (a cell per wavefront), or
-// away from the centre, where few spaces reach a cell, of 8 x 8 x 8 (eight cells per wavefront).
+// away from the centre, where few spaces reach a cell, of 8 x 8 x 8 (eight cells per wavefront),
+// or at the centre of the smallest volumes of 4 x 2 x 2 (four wavefronts per cell, shared_cell).
 // It culls a tile of spaces against the block, two per thread, into a list in index order; each
 // wavefront culls the list further against its cell, 64 entries at a time, into a queue, and
 // takes the queue eight spaces at a time: predicate and gather per lane (fr_gather.hpp), the
@@ -34,7 +35,61 @@ constexpr int kCellWaves = 8;
 constexpr int kCellThreads = 64 * kCellWaves;
 constexpr int kCellTile = 2 * kCellThreads;  // spaces culled together
 
-template <int kMode, int kOrder, int kNB, bool kHalf, bool kFastMath, bool kShift>
+// A cell that four wavefronts share: each takes every fourth eight of the list's spaces, and the first
+// of them adds the 32 spaces' contributions in order while the others gather the next.  `part` and
+// `hit` are written in turn, so one barrier a round separates their uses.  Every wavefront of the
+// workgroup makes the same rounds (the cell may lie outside the volume).
+// The chain of the central cells' spaces is what a very small volume's launch waits for (about 1.5
+// us per eight spaces; box 32, 500 slices, exact 97 -> 57 us, r 2.5 170 -> 110; rule: share_cells).
+template <int kMode, int kOrder, int kNB, bool kHalf, bool kFastMath, bool kTableLds, bool kShift,
+          int kRows>
+__device__ __forceinline__ void shared_cell(const FrJob &a, int x0, int y0, int z0, int base,
+                                            const uint16_t *list, int n,
+                                            float (*part)[kCellWaves][3 * 64],
+                                            int (*hits)[kCellWaves], float *blob, int nTable,
+                                            __amdgpu_buffer_rsrc_t rsrc, const float *tbl,
+                                            uint32_t sliceBytes, int wave, int lane)
+{
+  if (n == 0) return;
+  Cell cell = make_cell(a, x0, y0, z0, lane);
+  auto space_at = [&](int i) {
+    const uint32_t e = list[i < n ? i : 0];
+    return load_space<kHalf>(a, base + (int)(e & 0x7fffu), (e & 0x8000u) != 0, sliceBytes);
+  };
+  int turn = 0;
+  int i = 8 * (wave & 3) + (lane & 7);
+  CellSpace next = space_at(i);
+  for (int r = 0; r < n; r += 32, i += 32, turn ^= 1) {
+    const CellSpace sp = next;
+    if (r + 32 < n) next = space_at(i + 32);
+    float qx, qy, zs;
+    const bool hit = cell_pair<kMode>(cell, a, sp, cell.valid && i < n, qx, qy, zs);
+    const bool any = __any(hit);
+    if (any) {
+      const Contribution o =
+        cell_gather<kMode, kOrder, kNB, kHalf, kFastMath, kTableLds, kShift, kRows>(
+          a, sp, hit, qx, qy, zs, blob, nTable, rsrc, tbl, lane);
+      float *mine = part[turn][wave];
+      mine[lane] = o.re;
+      mine[64 + lane] = o.im;
+      mine[128 + lane] = o.w;
+    }
+    if (lane == 0) hits[turn][wave] = any;
+    __syncthreads();
+    if ((wave & 3) != 0) continue;
+    for (int w = wave; w < wave + 4; ++w) {
+      if (!__builtin_amdgcn_readfirstlane(hits[turn][w])) continue;
+      if (!cell.loaded) {
+        if (cell.owner) cell.acc = *cell.sum;
+        cell.loaded = true;
+      }
+      if (lane < 24) cell_add(cell, part[turn][w], lane);
+    }
+  }
+  if (cell.loaded && cell.owner) *cell.sum = cell.acc;
+}
+
+template <int kMode, int kOrder, int kNB, bool kHalf, bool kFastMath, bool kShift, bool kShared>
 __global__ __launch_bounds__(kCellThreads, 4) void fr_insert_cell_kernel(FrJob a, FrLaunch l)
 {
   constexpr bool kTableLds = kMode == kModeLookup;
@@ -42,7 +97,8 @@ __global__ __launch_bounds__(kCellThreads, 4) void fr_insert_cell_kernel(FrJob a
   // rows of the gather in flight: what 128 registers hold beside two spaces' records
   constexpr int kRows = kHalf ? (kNB <= 4 ? kNB : 3) : kNB <= 3 ? 3 : 2;
   extern __shared__ float s_table[];
-  __shared__ __align__(16) float s_part[kCellWaves][3 * 64];
+  __shared__ __align__(16) float s_part[kShared ? 2 : 1][kCellWaves][3 * 64];
+  __shared__ int s_hit[kShared ? 2 : 1][kCellWaves];
   __shared__ float s_blob[evaluates_blob(kMode) ? kCellWaves : 1][evaluates_blob(kMode) ? kBlobList : 1];
   __shared__ uint16_t s_list[kCellTile];
   __shared__ uint16_t s_queue[kCellWaves][kCellRing];
@@ -54,7 +110,7 @@ __global__ __launch_bounds__(kCellThreads, 4) void fr_insert_cell_kernel(FrJob a
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  float *part = s_part[wave], *blob = evaluates_blob(kMode) ? s_blob[wave] : nullptr;
+  float *part = s_part[0][wave], *blob = evaluates_blob(kMode) ? s_blob[wave] : nullptr;
   uint16_t *queue = s_queue[wave];
   const umpa_fr_constants &c = a.c;
   const int cxi = c.cMaxVolumeIndexX / 2, cyi = c.cMaxVolumeIndexYZ / 2;
@@ -76,17 +132,19 @@ __global__ __launch_bounds__(kCellThreads, 4) void fr_insert_cell_kernel(FrJob a
     }
     const int2 item = reinterpret_cast<const int2 *>(l.cells)[b];
     const int x0 = item.x & 0xffff, y0 = (item.x >> 16) & 0xffff, z0 = item.y & 0xffff;
-    const int edge = item.y >> 16;       // 4: a cell per wavefront; 8: eight cells
-    const int nMine = edge == 4 ? 1 : 8;  // the wavefront's cells: one, or its octant's
+    // 2: two cells side by side, four wavefronts each; 4: a cell per wavefront; 8: eight cells
+    const int edge = item.y >> 16;
+    const int wide = kShared && edge == 2 ? 4 : edge;
+    const int nMine = edge == 8 ? 8 : kShared && edge == 2 ? 0 : 1;  // the wavefront's own
 
     for (int base = a.spaceBegin; base < a.spaceEnd; base += kCellTile) {
       // cull the tile: wavefront w takes spaces base + 128 w ..., in index order
       const int s0 = base + wave * 128 + lane, s1 = s0 + 64;
       bool in0 = false, in1 = false;
       const unsigned long long m0 =
-        __ballot(s0 < a.spaceEnd && cull_block(a, s0, x0, y0, z0, edge, cxi, cyi, in0));
+        __ballot(s0 < a.spaceEnd && cull_block(a, s0, x0, y0, z0, wide, edge, cxi, cyi, in0));
       const unsigned long long m1 =
-        __ballot(s1 < a.spaceEnd && cull_block(a, s1, x0, y0, z0, edge, cxi, cyi, in1));
+        __ballot(s1 < a.spaceEnd && cull_block(a, s1, x0, y0, z0, wide, edge, cxi, cyi, in1));
       const int mine = __popcll(m0) + __popcll(m1);
       if (lane == 0) s_count[wave] = mine;
       __syncthreads();  // (also: every wavefront is done with the previous list)
@@ -103,6 +161,12 @@ __global__ __launch_bounds__(kCellThreads, 4) void fr_insert_cell_kernel(FrJob a
         s_list[lanes_below(m1, (unsigned)at)] = (uint16_t)((s1 - base) | (in1 ? 0x8000 : 0));
       __syncthreads();
 
+      if constexpr (kShared) {
+        if (edge == 2)
+          shared_cell<kMode, kOrder, kNB, kHalf, kFastMath, kTableLds, kShift, kRows>(
+            a, x0 + 2 * (wave >> 2), y0, z0, base, s_list, n, s_part, s_hit, blob, nTable, rsrc, tbl,
+            sliceBytes, wave, lane);
+      }
       for (int ci = 0; ci < nMine; ++ci) {
         // octant of the block = wave; in an octant of edge 4, cell ci
         const int step0 = edge >> 1;
@@ -137,40 +201,41 @@ __global__ __launch_bounds__(kCellThreads, 4) void fr_insert_cell_kernel(FrJob a
 }
 
 // ---- host-side dispatch ------------------------------------------------------------------
-template <int kNB>
+template <int kNB, bool kShared>
 static const void *pick_lookup(const FrVariant &v)
 {
   if (v.half)
-    return v.shift ? (const void *)fr_insert_cell_kernel<kModeLookup, 0, kNB, true, true, true>
-                   : (const void *)fr_insert_cell_kernel<kModeLookup, 0, kNB, true, true, false>;
+    return v.shift ? (const void *)fr_insert_cell_kernel<kModeLookup, 0, kNB, true, true, true, kShared>
+                   : (const void *)fr_insert_cell_kernel<kModeLookup, 0, kNB, true, true, false, kShared>;
   if (v.fastMath)
-    return v.shift ? (const void *)fr_insert_cell_kernel<kModeLookup, 0, kNB, false, true, true>
-                   : (const void *)fr_insert_cell_kernel<kModeLookup, 0, kNB, false, true, false>;
-  return v.shift ? (const void *)fr_insert_cell_kernel<kModeLookup, 0, kNB, false, false, true>
-                 : (const void *)fr_insert_cell_kernel<kModeLookup, 0, kNB, false, false, false>;
+    return v.shift ? (const void *)fr_insert_cell_kernel<kModeLookup, 0, kNB, false, true, true, kShared>
+                   : (const void *)fr_insert_cell_kernel<kModeLookup, 0, kNB, false, true, false, kShared>;
+  return v.shift ? (const void *)fr_insert_cell_kernel<kModeLookup, 0, kNB, false, false, true, kShared>
+                 : (const void *)fr_insert_cell_kernel<kModeLookup, 0, kNB, false, false, false, kShared>;
 }
 
+template <bool kShared>
 static const void *pick_cells(const FrVariant &v)
 {
   switch (v.mode) {
   case kModeLookup:
     switch (v.nb) {
-    case 3: return pick_lookup<3>(v);
-    case 4: return pick_lookup<4>(v);
-    case 5: return pick_lookup<5>(v);
-    default: return pick_lookup<6>(v);
+    case 3: return pick_lookup<3, kShared>(v);
+    case 4: return pick_lookup<4, kShared>(v);
+    case 5: return pick_lookup<5, kShared>(v);
+    default: return pick_lookup<6, kShared>(v);
     }
   case kModeFastKaiser:
-    return (const void *)fr_insert_cell_kernel<kModeFastKaiser, 0, 4, false, false, false>;
+    return (const void *)fr_insert_cell_kernel<kModeFastKaiser, 0, 4, false, false, false, kShared>;
   case kModeNearest:
-    return (const void *)fr_insert_cell_kernel<kModeNearest, 0, 4, false, false, false>;
+    return (const void *)fr_insert_cell_kernel<kModeNearest, 0, 4, false, false, false, kShared>;
   case kModePreciseKaiser:
     switch (v.order) {
-    case 0: return (const void *)fr_insert_cell_kernel<kModePreciseKaiser, 0, 4, false, false, false>;
-    case 1: return (const void *)fr_insert_cell_kernel<kModePreciseKaiser, 1, 4, false, false, false>;
-    case 2: return (const void *)fr_insert_cell_kernel<kModePreciseKaiser, 2, 4, false, false, false>;
-    case 3: return (const void *)fr_insert_cell_kernel<kModePreciseKaiser, 3, 4, false, false, false>;
-    case 4: return (const void *)fr_insert_cell_kernel<kModePreciseKaiser, 4, 4, false, false, false>;
+    case 0: return (const void *)fr_insert_cell_kernel<kModePreciseKaiser, 0, 4, false, false, false, kShared>;
+    case 1: return (const void *)fr_insert_cell_kernel<kModePreciseKaiser, 1, 4, false, false, false, kShared>;
+    case 2: return (const void *)fr_insert_cell_kernel<kModePreciseKaiser, 2, 4, false, false, false, kShared>;
+    case 3: return (const void *)fr_insert_cell_kernel<kModePreciseKaiser, 3, 4, false, false, false, kShared>;
+    case 4: return (const void *)fr_insert_cell_kernel<kModePreciseKaiser, 4, 4, false, false, false, kShared>;
     }
   }
   return nullptr;
@@ -179,7 +244,8 @@ static const void *pick_cells(const FrVariant &v)
 hipError_t launch_fr_cells(const FrJob &job, const FrLaunch &l, const FrVariant &v, int numCUs,
                            hipStream_t st)
 {
-  const void *k = pick_cells(v);
+  // (an instantiation of its own: as a branch, shared cells cost the others 1 to 2 %)
+  const void *k = l.cellsShared ? pick_cells<true>(v) : pick_cells<false>(v);
   if (!k || l.nCells <= 0) return hipErrorInvalidValue;
   // two workgroups per CU: registers for 16 wavefronts, LDS for both tables (at most 47 KB each)
   const int blocks = l.nCells < 2 * numCUs ? l.nCells : 2 * numCUs;

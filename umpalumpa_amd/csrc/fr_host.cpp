@@ -563,8 +563,20 @@ std::vector<BrickOrigin> make_brick_schedule(int vx, int vy, int vz, bool splitH
   return make_schedule({ JobWork{ &set, 0, 1.0 } }, splitHeavy, sp);
 }
 
-std::vector<int> make_cell_blocks(int vx, int vy, int vz)
+// Sharing the cells near the centre shortens the longest chains and adds blocks, so it pays where the
+// chains are what a launch waits for (us, own / shared up to 8 voxels from the centre, r 1.9 exact:
+// box 32, 30 spaces 19.8 / 19.2, 100 31 / 25, 500 97 / 57, 1,500 284 / 155; 48 30 30.6 / 32.7, 100
+// 37 / 36, 500 114 / 78; 64 500 133 / 136; blob evaluated 64 500 224 / 202, 80 251 / 238, 100 336 /
+// 333; nearest pixel 64 156 / 101, 80 155 / 132, 100 216 / 218).
+bool share_cells(int vx, int vy, int vz, uint64_t spaces, const umpa_fr_settings &s)
 {
+  const bool table = s.type != UMPA_FR_FAST && s.interpolation == UMPA_FR_LOOKUP;
+  return spaces >= 60 && at_most_cube(vx, vy, vz, table ? 57 : 85);
+}
+
+std::vector<int> make_cell_blocks(int vx, int vy, int vz, bool share)
+{
+  const float shareFrom = share ? 3.f / 8.f : 2.f;  // a 4 x 4 x 4 block's cost
   const int cx = (vx - 1) / 2, cy = (vy - 1) / 2;
   // a wavefront's steps per space and block: a random plane passes within w of a point at
   // distance R with probability ~w/R, times the wavefront's cells
@@ -572,7 +584,7 @@ std::vector<int> make_cell_blocks(int vx, int vy, int vz)
     const float h = 0.5f * (float)(e - 1);
     const float dx = x + h - cx, dy = y + h - cy, dz = z + h - cy;
     const float R = std::sqrt(dx * dx + dy * dy + dz * dz), w = 3.f;
-    return (e == 4 ? 1.f : 8.f) * w / std::max(R, w);
+    return (e == 2 ? 0.25f : e == 4 ? 1.f : 8.f) * w / std::max(R, w);
   };
   struct Block {
     int x, y, z, e, bin;
@@ -593,7 +605,14 @@ std::vector<int> make_cell_blocks(int vx, int vy, int vz)
           add(x, y, z, 8);
           continue;
         }
-        for (int i = 0; i < 8; ++i) add(x + 4 * (i & 1), y + 4 * ((i >> 1) & 1), z + 4 * (i >> 2), 4);
+        for (int i = 0; i < 8; ++i) {
+          const int bx = x + 4 * (i & 1), by = y + 4 * ((i >> 1) & 1), bz = z + 4 * (i >> 2);
+          if (cost(bx, by, bz, 4) < shareFrom) {
+            add(bx, by, bz, 4);
+          } else {
+            for (int k = 0; k < 4; ++k) add(bx, by + 2 * (k & 1), bz + 2 * (k >> 1), 2);
+          }
+        }
       }
   for (int i = 0; i < kBins; ++i) start[(size_t)i + 1] += start[(size_t)i];
   std::vector<int> out(2 * blocks.size());

@@ -105,9 +105,11 @@ std::vector<BrickOrigin> make_brick_schedule(int vx, int vy, int vz, bool splitH
                                              const SchedParams &sp = SchedParams(),
                                              float core = 0.f);
 
-// The 4 x 4 x 4 blocks covering a volume, nearest to the centre first, two ints each: x | y << 16
-// and z (the small-problem kernel's work items).
-std::vector<int> make_cell_blocks(int vx, int vy, int vz);
+// The blocks covering a volume, the costliest first, two ints each: x | y << 16 and z | edge << 16
+// (the small-problem kernel's work items).  With `share` (share_cells: by volume, spaces and blob)
+// those at the centre are of 4 x 2 x 2 voxels, edge 2, whose cells four wavefronts share.
+bool share_cells(int vx, int vy, int vz, uint64_t spaces, const umpa_fr_settings &s);
+std::vector<int> make_cell_blocks(int vx, int vy, int vz, bool share);
 
 // Persisted tuning results: one "key depthScale priority maxParts splitAt kernel tableGlobal
 // boxFixed ms" line per key in $UMPA_TUNING_DIR/fr_tuning.txt (default

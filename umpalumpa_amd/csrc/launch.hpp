@@ -48,6 +48,7 @@ struct FrLaunch {
   int numCUs;           // set by the launch
   const int *cells;     // int2 {x | y << 16, z | edge << 16} per block of the volume, heaviest first
   int nCells;           // (plain launches whose host keeps the list; 0: none)
+  bool cellsShared;     // the list holds blocks of edge 2
   int *cellCounter;     // blocks claimed so far: zero between launches
 };
 

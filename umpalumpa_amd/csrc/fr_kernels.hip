@@ -369,7 +369,7 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
     // work item: brick 8 x 8 x depth at (bo.x, bo.y, bo.z & 0xffff) of job bo.z >> 16; heavy
     // bricks run at raised wave priority; a brick split into `parts` slice ranges accumulates
     // its range from zero and merges the partial sums with atomics (fast-math schedules only)
-    const FrJob a = kBatched ? make_uniform(l.jobs[bo.z >> 16]) : job0;
+    const FrJob a = kBatched ? global_pointers(make_uniform(l.jobs[bo.z >> 16])) : job0;
     const int s0 = a.spaceBegin, s1 = a.spaceEnd;
     if (s0 >= s1) continue;
     const bool heavy = (bo.w >> 4) & 1;
@@ -595,7 +595,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fr_insert_carry_kernel(FrJob j
   for (int b = begin; b < l.nItems;
        b = bounded ? next_dealt(l, dealt, &s_taken, lane) : claim_item(l, lane, claimed)) {
     const int4 bo = make_uniform(reinterpret_cast<const int4 *>(l.items)[b]);
-    const FrJob a = kBatched ? make_uniform(l.jobs[bo.z >> 16]) : job0;
+    const FrJob a = kBatched ? global_pointers(make_uniform(l.jobs[bo.z >> 16])) : job0;
     const int s0 = a.spaceBegin, s1 = a.spaceEnd;
     if (s0 >= s1) continue;
     const bool heavy = (bo.w >> 4) & 1;

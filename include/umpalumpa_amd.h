@@ -255,8 +255,9 @@ typedef struct umpa_fr_sched_params {
   int32_t maxParts;  /* split heavy bricks into at most this many slice ranges (fast math) */
   float splitAt;     /* ... above splitAt x one wavefront's fair share of the launch */
   /* Kernel knobs; 0 selects the default in each.  Batches keep the table in LDS and run the
-   * per-pair kernel, or the carried queues when `kernel` names them (fast math) and every
-   * job's slices fit one 2 GiB buffer resource. */
+   * per-pair kernel, or the carried queues when `kernel` names them (fast math; by default for
+   * FP32 slices in launches that are not bounded) and every job's slices fit one 2 GiB buffer
+   * resource. */
   int32_t kernel;      /* UMPA_FR_KERNEL_*: insertion kernel; one that does not cover the
                           variant (mode, strategy, footprint) runs as UMPA_FR_KERNEL_PAIR */
   int32_t tableGlobal; /* 1: blob table read from global memory instead of LDS */

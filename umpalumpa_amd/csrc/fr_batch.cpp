@@ -225,14 +225,18 @@ void build_step(umpa_fr_batch *b, const std::vector<JobInfo> &infos,
     const auto &items = b->schedBuf;
     LaunchImage li{};
     li.v = first.v;
-    // the carried-queue kernel reads a job's slices through one buffer resource: it runs only
-    // when the knob names it and every job's slices fit one
+    // the carried-queue kernel reads a job's slices through one buffer resource: it runs only if
+    // every job's slices fit one, when the knob names it, or by default for the launches it is the
+    // faster kernel of (us, per pair / carried, boxes 64 to 320: FP32 3868 / 3751, FP16 3666 / 3781;
+    // bounded FP32, boxes 96 to 256, 1382 / 1390, FP16 1285 / 1390)
     bool carryFits = true;
     for (const umpa::FrJob &rec : recs)
       carryFits = carryFits && (uint64_t)rec.nProj * (uint64_t)rec.sliceElems *
                                    (li.v.half ? 4u : 8u) <= 0x7fff0000ull;
-    li.v.kernel = sp.kernel == UMPA_FR_KERNEL_CARRY && carryFits ? UMPA_FR_KERNEL_CARRY
-                                                                 : UMPA_FR_KERNEL_PAIR;
+    const bool wanted = sp.kernel == UMPA_FR_KERNEL_AUTO
+                          ? li.v.fastMath && !li.v.half && b->waveItems == 0
+                          : sp.kernel == UMPA_FR_KERNEL_CARRY;
+    li.v.kernel = wanted && carryFits ? UMPA_FR_KERNEL_CARRY : UMPA_FR_KERNEL_PAIR;
     // the sliding-box instantiation only when every job of the launch slides
     li.v.shift = std::all_of(recs.begin(), recs.end(),
                              [](const umpa::FrJob &r) { return r.shiftBox != 0; });

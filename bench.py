@@ -145,7 +145,8 @@ def uniform_rotations(n, seed):
         2 * (x * z - y * w), 2 * (y * z + x * w), 1 - 2 * (x * x + y * y)], axis=1).reshape(n, 3, 3)
 
 
-KERNEL_SOURCE = os.path.join(ROOT, "umpalumpa_amd", "csrc", "fr_kernels.hip")
+KERNEL_SOURCES = [os.path.join(ROOT, "umpalumpa_amd", "csrc", name)
+                  for name in ("fr_kernels.hip", "fr_gather.hpp", "fr_cell.hpp")]
 
 
 # The kernel a plain Execute of the box-256, 1,000-slice chunk launches under each strategy
@@ -158,11 +159,14 @@ PLAIN_KERNEL = {"exact": "fr_insert_staged_kernel", "fast": "fr_insert_carry_ker
 
 def kernel_source_sha256():
     import hashlib
+    digest = hashlib.sha256()
     try:
-        with open(KERNEL_SOURCE, "rb") as f:
-            return hashlib.sha256(f.read()).hexdigest()
+        for path in KERNEL_SOURCES:
+            with open(path, "rb") as f:
+                digest.update(f.read())
     except OSError:
         return None
+    return digest.hexdigest()
 
 
 def profile_figure(key, strategy):

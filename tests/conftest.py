@@ -20,7 +20,7 @@ def _ensure_built():
     lib = os.path.join(ROOT, "umpalumpa_amd", "libumpalumpa_amd.so")
     orc = os.path.join(ROOT, "oracle", "liboracle.so")
     cpp = [os.path.join(ROOT, "tests", "cpp", "_build", name)
-           for name in ("fr_fp_tests", "fr_harness")]
+           for name in ("fr_fp_tests", "fr_harness", "launch_rules")]
     if not (os.path.exists(lib) and os.path.exists(orc) and all(map(os.path.exists, cpp))):
         import __graft_entry__
         __graft_entry__.build()

@@ -1,0 +1,95 @@
+// Prints what the library's launch rules choose, host arithmetic only: one line per line of input.
+//   insert key=value ...   choose_fr_insert of a launch: "<which> <blocks> <threads> <lds> <kernel>"
+#include <dlfcn.h>
+
+#include <cstdio>
+#include <iostream>
+#include <map>
+#include <sstream>
+#include <string>
+
+#include "../../umpalumpa_amd/csrc/fr_host.hpp"
+#include "../../umpalumpa_amd/csrc/launch.hpp"
+
+namespace {
+
+std::map<std::string, double> g_args;
+double arg(const char *key, double otherwise = 0)
+{
+  const auto it = g_args.find(key);
+  return it == g_args.end() ? otherwise : it->second;
+}
+
+const char *name_of(const void *kernel)
+{
+  Dl_info info{};
+  return kernel && dladdr(kernel, &info) && info.dli_sname ? info.dli_sname : "-";
+}
+
+umpa_fr_settings settings()
+{
+  umpa_fr_settings s{};
+  s.interpolation = arg("evaluated") || arg("nearest") ? UMPA_FR_DYNAMIC : UMPA_FR_LOOKUP;
+  s.type = arg("nearest") ? UMPA_FR_FAST : UMPA_FR_PRECISE;
+  s.alpha = 15.f;
+  s.blobRadius = (float)arg("radius", 1.9);
+  return s;
+}
+
+void insert()
+{
+  const int box = (int)arg("box"), side = box + 1, spaces = (int)arg("spaces", 1);
+  const umpa_fr_settings s = settings();
+  umpa::FrVariant v{};
+  v.mode = arg("nearest") ? umpa::kModeNearest
+           : arg("evaluated") ? umpa::kModeFastKaiser : umpa::kModeLookup;
+  v.nb = umpa::host::footprint(s);
+  v.half = arg("half") != 0;
+  v.fastMath = v.half || arg("fast") != 0;
+  v.count = arg("count") != 0;
+  v.batched = arg("batched") != 0;
+  v.kernel = (int)arg("kernel");
+  v.tableGlobal = arg("tableGlobal") != 0;
+  umpa::FrJob job{};
+  job.xSize = box / 2 + 1;
+  job.ySize = box;
+  job.sliceElems = (int64_t)job.xSize * job.ySize;
+  job.nProj = (int)arg("slices", spaces);
+  job.vx = job.vy = job.vz = side;
+  job.spaceEnd = spaces;
+  job.shiftBox = umpa::host::box_can_shift(s, (uint64_t)job.xSize, (uint64_t)job.ySize);
+  job.c.cBlobRadius = s.blobRadius;
+  v.shift = job.shiftBox != 0;
+  umpa::FrLaunch l{};
+  l.nTable = (int)arg("table", 10000);
+  l.waveItems = (int)arg("waveItems");
+  if (!v.batched && umpa::cells_possible(side, side, side)) {
+    l.cellsShared = umpa::host::share_cells(side, side, side, (uint64_t)spaces, s);
+    l.nCells = (int)umpa::host::make_cell_blocks(side, side, side, l.cellsShared).size() / 2;
+  }
+  const float core = v.batched || v.fastMath ? 0.f : umpa::host::core_radius(side, side, side);
+  l.nItems = (int)umpa::host::make_brick_schedule(side, side, side, v.fastMath, {}, core).size();
+  if (core > 0.f) l.nCore = (int)umpa::host::core_cells(side, side, side, core).size() / 2;
+  const umpa::FrChoice c = umpa::choose_fr_insert(job, l, v, (int)arg("cus", 256));
+  std::printf("%d %d %d %zu %s\n", c.which, c.blocks, c.threads, c.lds, name_of(c.kernel));
+}
+
+}  // namespace
+
+int main()
+{
+  std::string line;
+  while (std::getline(std::cin, line)) {
+    std::istringstream is(line);
+    std::string command, word;
+    is >> command;
+    g_args.clear();
+    while (is >> word) {
+      const size_t eq = word.find('=');
+      g_args[word.substr(0, eq)] = eq == std::string::npos ? 1 : std::stod(word.substr(eq + 1));
+    }
+    if (command == "insert") insert();
+    else return 2;
+  }
+  return 0;
+}

@@ -1,0 +1,37 @@
+"""The launch rules on the host: what a launch chooses fits the GPU it is for.  No GPU needed."""
+import pytest
+
+import launchtools as L
+
+LDS = 160 * 1024  # bytes a workgroup may use on gfx950
+
+
+@pytest.fixture(scope="module")
+def metadata():
+    pytest.importorskip("msgpack")
+    return L.kernel_metadata()
+
+
+@pytest.mark.parametrize("batched", [0, 1])
+@pytest.mark.parametrize("strategy", ["exact", "fast", "half"])
+@pytest.mark.parametrize("radius", [1.2, 1.9])
+def test_table_and_state_fit_lds(metadata, batched, strategy, radius):
+    """Tables around every kernel's limit: the chosen kernel's own LDS and the table's together
+    stay within the 160 KiB of a workgroup."""
+    tables = [100, 10238, 10239, 10240, *range(10740, 10756), 11774, 11775, 11776, 11777]
+    kernels = [0, L.PAIR, L.CARRY, L.STAGED]
+    cases = [{"box": 128, "spaces": 50, "radius": radius, strategy: 1, "batched": batched,
+              "table": n, "kernel": k} for n in tables for k in kernels
+             if not (batched and n > 11776)]
+    for case, (which, _, _, lds, symbol) in zip(cases, L.choices(cases)):
+        assert symbol in metadata, case
+        assert metadata[symbol][".group_segment_fixed_size"] + lds <= LDS, (case, which, symbol)
+
+
+def test_largest_table_of_the_carried_queues():
+    """The carried queues take tables up to what 160 KiB leave beside their state; a batch's launch
+    keeps a count there too, so its limit is a few samples lower."""
+    cases = [{"box": 128, "spaces": 50, "fast": 1, "batched": b, "table": n, "kernel": L.CARRY}
+             for b in (0, 1) for n in (10747, 10748, 10751, 10752)]
+    got = [c[0] for c in L.choices(cases)]
+    assert got == [L.CARRY, L.CARRY, L.CARRY, L.PAIR, L.CARRY, L.PAIR, L.PAIR, L.PAIR]

@@ -241,19 +241,18 @@ static const void *pick_cells(const FrVariant &v)
   return nullptr;
 }
 
-hipError_t launch_fr_cells(const FrJob &job, const FrLaunch &l, const FrVariant &v, int numCUs,
-                           hipStream_t st)
+FrChoice choose_fr_cells(const FrLaunch &l, const FrVariant &v, int numCUs)
 {
+  FrChoice c{};
+  c.which = kKernelCells;
+  if (l.nCells <= 0) return c;
   // (an instantiation of its own: as a branch, shared cells cost the others 1 to 2 %)
-  const void *k = l.cellsShared ? pick_cells<true>(v) : pick_cells<false>(v);
-  if (!k || l.nCells <= 0) return hipErrorInvalidValue;
+  c.kernel = l.cellsShared ? pick_cells<true>(v) : pick_cells<false>(v);
   // two workgroups per CU: registers for 16 wavefronts, LDS for both tables (at most 47 KB each)
-  const int blocks = l.nCells < 2 * numCUs ? l.nCells : 2 * numCUs;
-  const size_t lds = v.mode == kModeLookup ? (size_t)(l.nTable + 1) * sizeof(float) : 0;
-  FrJob j = job;
-  FrLaunch ll = l;
-  void *args[] = { &j, &ll };
-  return hipLaunchKernel(k, dim3(blocks), dim3(kCellThreads), args, lds, st);
+  c.blocks = l.nCells < 2 * numCUs ? l.nCells : 2 * numCUs;
+  c.threads = kCellThreads;
+  c.lds = v.mode == kModeLookup ? (size_t)(l.nTable + 1) * sizeof(float) : 0;
+  return c;
 }
 
 }  // namespace umpa

@@ -52,6 +52,9 @@ struct alignas(16) WaveScratch {
   float accW[kVox];
   uint16_t queue[kVox];
 };
+// fr_insert_kernel's LDS with its largest table (and the words beside the per-wave state)
+static_assert(kMaxWaves * (sizeof(WaveScratch) + sizeof(umpa_traverse_space)) + 16 +
+                (kMaxLdsTable + 1) * sizeof(float) <= 160 * 1024, "one workgroup per CU");
 
 // Element `index` (wave-uniform) of a buffer the kernels only read, through the constant
 // address space: the compiler then reads it with scalar loads into SGPRs instead of 16-byte
@@ -523,9 +526,13 @@ struct CarryScratch {
   uint16_t queue[kCarryQueue];  // voxel index (bits 0-8) | slot (bit 9)
 };
 
-// Largest blob table the carry kernel keeps in LDS beside its per-wave state.
-constexpr int kCarryMaxTable =
-  (160 * 1024 - kMaxWaves * (int)(sizeof(CarryScratch) + 2 * sizeof(CarrySlot))) / 4 - 1;
+// Largest blob table the carry kernel keeps in LDS beside its per-wave state (batched: and beside
+// the count of taken items).
+constexpr int carry_max_table(bool batched)
+{
+  return (160 * 1024 - kMaxWaves * (int)(sizeof(CarryScratch) + 2 * sizeof(CarrySlot)) -
+          (batched ? 16 : 0)) / 4 - 1;
+}
 
 // One batch of `n` (1..64) queue entries from `start`: the rest of the predicate, the gather and
 // the accumulation, space by space.
@@ -984,7 +991,7 @@ static bool staged_fits(const FrJob &job)
 static const void *pick_carry(const FrVariant &v, int nTable)
 {
   if (v.mode != kModeLookup || !v.fastMath) return nullptr;
-  if (!table_in_lds(v, nTable) || nTable > kCarryMaxTable) return nullptr;
+  if (!table_in_lds(v, nTable) || nTable > carry_max_table(v.batched)) return nullptr;
   if (v.nb != 3 && v.nb != 4) return nullptr;
 #define UMPA_CARRY(NB, H, B)                                                                 \
   (v.shift ? (v.count ? (const void *)fr_insert_carry_kernel<NB, H, true, B, true>           \
@@ -1056,17 +1063,18 @@ bool use_cells(const FrJob &job, const FrLaunch &l, const FrVariant &v)
   return spaces >= (cbrtf((float)voxels) - rule.from) * rule.slope;
 }
 
-hipError_t launch_fr_insert(const FrJob &job, const FrLaunch &l, const FrVariant &v0, int numCUs,
-                            hipStream_t st)
+FrChoice choose_fr_insert(const FrJob &job, const FrLaunch &l, const FrVariant &v0, int numCUs)
 {
   // a plain launch slides its boxes when its job does; a batch's host sets v.shift when every
   // job of the launch does
   FrVariant v = v0;
   if (!v.batched) v.shift = job.shiftBox != 0;
-  if (use_cells(job, l, v)) return launch_fr_cells(job, l, v, numCUs, st);
-  const void *k = pick_kernel(v, l.nTable);
-  if (!k) return hipErrorInvalidValue;
-  const size_t shmem = table_in_lds(v, l.nTable) ? (size_t)(l.nTable + 1) * sizeof(float) : 0;
+  if (use_cells(job, l, v)) return choose_fr_cells(l, v, numCUs);
+  FrChoice ch{};
+  ch.which = kKernelPair;
+  ch.kernel = pick_kernel(v, l.nTable);
+  if (!ch.kernel) return ch;
+  ch.lds = table_in_lds(v, l.nTable) ? (size_t)(l.nTable + 1) * sizeof(float) : 0;
   // persistent workgroups: the per-wave LDS state allows one per CU
   int waves = fr_waves(v.mode, v.half, v.fastMath);
   // kKernelAuto: the staged kernel for the exact strategy, the carried queues for fast-math
@@ -1081,31 +1089,42 @@ hipError_t launch_fr_insert(const FrJob &job, const FrLaunch &l, const FrVariant
   const void *staged = want == kKernelStaged ? pick_staged(v, l.nTable, v.shift) : nullptr;
   const void *carry = want == kKernelCarry ? pick_carry(v, l.nTable) : nullptr;
   if (staged && staged_fits(job)) {
-    k = staged;
+    ch.kernel = staged;
+    ch.which = kKernelStaged;
     waves = kStagedWaves;
   } else if (carry && carry_fits(job, v.half)) {
-    k = carry;
+    ch.kernel = carry;
+    ch.which = kKernelCarry;
   }
-  // persistent workgroups, one per CU, until the items run out; with l.waveItems, every wave
-  // leaves after that many items and the grid covers the items (CUs come free for other
-  // streams' launches as workgroups end)
-  int blocks;
+  ch.threads = 64 * waves;
+  // persistent workgroups, one per CU, until the items run out; with l.waveItems, every workgroup
+  // leaves after that many items for each of its waves and the grid covers the items (CUs come
+  // free for other streams' launches as workgroups end)
   if (l.waveItems > 0) {
     const int64_t per = (int64_t)waves * l.waveItems;
-    blocks = (int)((l.nItems + per - 1) / per);
+    ch.blocks = (int)((l.nItems + per - 1) / per);
   } else {
-    blocks = (l.nItems + waves - 1) / waves;
-    if (blocks > numCUs) blocks = numCUs;
-    if (l.maxBlocks > 0 && blocks > l.maxBlocks) blocks = l.maxBlocks;
+    ch.blocks = (l.nItems + waves - 1) / waves;
+    if (ch.blocks > numCUs) ch.blocks = numCUs;
+    if (l.maxBlocks > 0 && ch.blocks > l.maxBlocks) ch.blocks = l.maxBlocks;
   }
-  if (blocks < 1) blocks = 1;
+  if (ch.blocks < 1) ch.blocks = 1;
+  return ch;
+}
+
+hipError_t launch_fr_insert(const FrJob &job, const FrLaunch &l, const FrVariant &v, int numCUs,
+                            hipStream_t st)
+{
+  const FrChoice ch = choose_fr_insert(job, l, v, numCUs);
+  if (!ch.kernel) return hipErrorInvalidValue;
   FrJob j = job;
   FrLaunch ll = l;
   ll.numCUs = numCUs;
+  const int waves = ch.threads / 64;
   if (l.waveItems > 0)  // (a workgroup's count of items stays an int)
     ll.waveItems = (int)std::min<int64_t>(l.waveItems, ((int64_t)l.nItems + waves - 1) / waves);
   void *args[] = { &j, &ll };
-  return hipLaunchKernel(k, dim3(blocks), dim3(64 * waves), args, shmem, st);
+  return hipLaunchKernel(ch.kernel, dim3(ch.blocks), dim3(ch.threads), args, ch.lds, st);
 }
 
 }  // namespace umpa

@@ -76,9 +76,20 @@ struct FrVariant {
 // A kernel that does not cover a variant (mode, strategy, footprint, batching) or a chunk
 // (slices beyond one 2 GiB buffer resource) is replaced by the per-pair kernel.
 enum : int { kKernelAuto = 0, kKernelPair = 1, kKernelCarry = 2, kKernelStaged = 3 };
+constexpr int kKernelCells = 4;  // the small-problem kernel: chosen by size, no knob names it
 
-// Dynamic LDS and workgroup count of an insertion launch; `prepare` sets the kernel's LDS
-// attribute once (outside any stream capture).
+// What a launch runs: the kernel, workgroups of `threads`, and their dynamic LDS in bytes.
+struct FrChoice {
+  const void *kernel;  // nullptr: no kernel covers the variant
+  int which;           // kKernel*
+  int blocks, threads;
+  size_t lds;
+};
+// Host arithmetic only (no HIP call).
+FrChoice choose_fr_insert(const FrJob &job, const FrLaunch &l, const FrVariant &v, int numCUs);
+
+// Sets the LDS attribute of every kernel a launch of this variant may choose, once (outside any
+// stream capture).
 hipError_t prepare_fr_insert(const FrVariant &v, int nTable);
 // Enqueues the insertion kernel on `st`.
 hipError_t launch_fr_insert(const FrJob &job, const FrLaunch &l, const FrVariant &v, int numCUs,
@@ -92,8 +103,7 @@ inline bool cells_possible(int vx, int vy, int vz)
 // Does the launch run the small-problem kernel (which needs no `prepare`)?
 bool use_cells(const FrJob &job, const FrLaunch &l, const FrVariant &v);
 // The small-problem kernel (fr_cells.hip) over l.cells.
-hipError_t launch_fr_cells(const FrJob &job, const FrLaunch &l, const FrVariant &v, int numCUs,
-                           hipStream_t st);
+FrChoice choose_fr_cells(const FrLaunch &l, const FrVariant &v, int numCUs);
 
 // Allocation-free insertion: the work counter and the work items live in a static device
 // array of kNoAllocScratchBytes per GPU (a 256-byte header, then int4 items).  `items` is the

@@ -37,3 +37,63 @@ def test_batch_tables_around_the_carried_queues_limit(n_table, strategy):
             assert v.tobytes() == rv.tobytes() and w.tobytes() == rw.tobytes()
         else:
             assert rel_l2(v, rv) <= 1e-5 and rel_l2(w, rw) <= 1e-5
+
+
+def _beside_nan(box, n, s, **kw):
+    """A problem whose odd slices, which no space names, hold NaN."""
+    fft, spaces, desc, table = problem(box, 2 * n, s, **kw)
+    keep = np.ascontiguousarray(spaces[spaces["projectionIndex"] % 2 == 0])
+    fft[1::2] = np.complex64(complex(np.nan, np.nan))
+    return fft, keep, desc, table
+
+
+SLICES_BESIDE_NAN = [
+    # table radius that does not slide, evaluated blobs, the widest boxes, slices below a box
+    (30, F.FR_LOOKUP, 0.4), (30, F.FR_DYNAMIC, 1.9), (30, F.FR_LOOKUP, 3.2), (4, F.FR_LOOKUP, 1.9),
+    (30, F.FR_DYNAMIC, 2.6), (130, F.FR_DYNAMIC, 1.9), (130, F.FR_LOOKUP, 0.4)]
+
+
+@pytest.mark.parametrize("box,interp,radius", SLICES_BESIDE_NAN)
+@pytest.mark.parametrize("kernel", [F.FR_KERNEL_AUTO, F.FR_KERNEL_PAIR])
+def test_a_slice_beside_others_that_are_not_finite(box, interp, radius, kernel):
+    """Candidate boxes that reach past a slice's last row take nothing of the next slice, which is
+    NaN here and named by no space: the oracle's bits (exact), 1e-5 of them (fast math, FP16)."""
+    from frtools import quantize_f16, run_hip
+    s = settings(interp, radius=radius)
+    fft, spaces, desc, table = _beside_nan(box, 9, s, seed=box)
+    ov, ow, _ = run_oracle(s, fft, spaces, table, box)
+    assert np.isfinite(ov.view(np.float32)).all() and ow.max() > 0
+    sched = F.SchedParams(1.0, 1, 1, 0.5, kernel, 0, 0)
+    v, w, _ = run_hip(s, fft, spaces, desc, table, box, sched=sched)
+    assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()
+    if interp != F.FR_LOOKUP:
+        return
+    v, w, _ = run_hip(s, fft, spaces, desc, table, box, strategy=F.FR_FAST_MATH, sched=sched)
+    assert rel_l2(v, ov) <= 1e-5 and rel_l2(w, ow) <= 1e-5
+    h, scales, deq = quantize_f16(np.where(np.isfinite(fft), fft, np.complex64(1)))
+    h[1::2] = np.nan
+    ov, ow, _ = run_oracle(s, deq, spaces, table, box)
+    v, w, _ = run_hip(s, fft, spaces, desc, table, box, half=(h, scales), sched=sched)
+    assert rel_l2(v, ov) <= 1e-5 and rel_l2(w, ow) <= 1e-5
+
+
+@pytest.mark.parametrize("radius", [0.4, 1.9])
+def test_a_batch_beside_slices_that_are_not_finite(radius):
+    """The same through a batch of FP32 jobs (carried queues), slices of 3 x 4 pixels among them."""
+    dev = torch.device("cuda:0")
+    s = settings(radius=radius)
+    jobs, ref = [], []
+    for box in (4, 30):
+        fft, spaces, _, table = _beside_nan(box, 9, s, seed=box)
+        jobs.append(F.BatchJob(torch.from_numpy(fft).to(dev),
+                               torch.zeros((box + 1,) * 3, dtype=torch.complex64, device=dev),
+                               torch.zeros((box + 1,) * 3, dtype=torch.float32, device=dev),
+                               torch.from_numpy(spaces.view(np.uint8)).to(dev), s,
+                               torch.from_numpy(table).to(dev)))
+        ref.append(run_oracle(s, fft, spaces, table, box)[:2])
+    b = F.FRBatch(0)
+    b.step(jobs, [0, 0], [j.n_spaces for j in jobs], F.FR_FAST_MATH)
+    b.synchronize()
+    for job, (rv, rw) in zip(jobs, ref):
+        assert rel_l2(job.volume.cpu().numpy(), rv) <= 1e-5
+        assert rel_l2(job.weights.cpu().numpy(), rw) <= 1e-5

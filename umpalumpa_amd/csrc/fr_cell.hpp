@@ -152,7 +152,7 @@ __device__ __forceinline__ Contribution cell_gather(const FrJob &a, const CellSp
       o = gather_nearest<kHalf>(a, rsrc, qx, qy, sp.weight, sp.scale, sp.off);
     } else {
       // (a weight of 1 changes no product, so one copy of the gather serves all)
-      o = gather_update<kMode, kOrder, kNB, kHalf, kFastMath, kTableLds, kShift, kRows>(
+      o = gather_update<kMode, kOrder, kNB, kHalf, kFastMath, kTableLds, kShift, true, kRows>(
         a, nTable, rsrc, tbl, qx, qy, zs, sp.weight, false, sp.scale, sp.off);
     }
   }

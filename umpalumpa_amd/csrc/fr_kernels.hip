@@ -475,7 +475,7 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
             } else if constexpr (kMode == kModeNearest) {
               o = gather_nearest<kHalf>(a, rsrc, qx, qy, sp.weight, scale);
             } else {
-              o = gather_update<kMode, kOrder, kNB, kHalf, kFastMath, kTableLds, kShift>(
+              o = gather_update<kMode, kOrder, kNB, kHalf, kFastMath, kTableLds, kShift, false>(
                 a, nTable, rsrc, tbl, qx, qy, zs, sp.weight, unit, scale);
             }
             // volume += contribution, in space order (one item per voxel per space)
@@ -560,7 +560,7 @@ __device__ __forceinline__ void carry_batch(CarryScratch &ws, const CarrySlot *s
     act && blob_predicate<false>(sp, sp.transformInv, c, xv, yv, zv, pxv, pyv, pzv, slt.inside != 0, qx, qy, zs);
   Contribution o{ 0.f, 0.f, 0.f };
   if (hit) {
-    o = gather_update<kModeLookup, 0, kNB, kHalf, true, true, kShift>(
+    o = gather_update<kModeLookup, 0, kNB, kHalf, true, true, kShift, true>(
       a, nTable, rsrc, tbl, qx, qy, zs, sp.weight, false, slt.scale, slt.sliceOff);
   }
   // lane 0 holds the batch's oldest entry: its space is added first
@@ -740,7 +740,7 @@ __device__ __forceinline__ void staged_gather(const FrJob &a, int nTable,
   const uint32_t off = act ? st.off[e] : 0u, key = act ? st.key[e] : 0u;
   Contribution o{ 0.f, 0.f, 0.f };
   if (act) {
-    o = gather_update<kModeLookup, 0, kNB, false, false, true, kShift>(
+    o = gather_update<kModeLookup, 0, kNB, false, false, true, kShift, true>(
       a, nTable, rsrc, tbl, qx, qy, zs, dw, __all(dw == 1.f), 1.f, off);
   }
   // add space by space (the lowest remaining lane holds the earliest space): within a space
@@ -779,8 +779,7 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
   const int lane = threadIdx.x & 63;
   WaveScratch &ws = s_wave[threadIdx.x >> 6];
   WaveStage &st = s_stage[threadIdx.x >> 6];
-  // one resource over the chunk's slices (the host keeps it under 2 GiB); a candidate row
-  // read past its slice's end reads the next slice or zeros, always at weight 0
+  // one resource over the chunk's slices (the host keeps it under 2 GiB)
   const uint32_t sliceBytes = (uint32_t)(a.sliceElems * kPix);
   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
     (void *)a.fft, 0, (int)((uint32_t)a.nProj * sliceBytes), kBufferConfig);

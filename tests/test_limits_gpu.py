@@ -97,3 +97,22 @@ def test_a_batch_beside_slices_that_are_not_finite(radius):
     for job, (rv, rw) in zip(jobs, ref):
         assert rel_l2(job.volume.cpu().numpy(), rv) <= 1e-5
         assert rel_l2(job.weights.cpu().numpy(), rw) <= 1e-5
+
+
+@pytest.mark.parametrize("strategy", [F.FR_EXACT, F.FR_FAST_MATH])
+def test_transforms_that_are_no_rotation(strategy):
+    """A record's transform may be any matrix.  With its third row 1,500 times a rotation's, q.z
+    rounds by hundredths at the slab's faces, and every voxel that passes the reference's rounded
+    test has to be found: the oracle's number of updates, and under the exact strategy its bits."""
+    from frtools import run_hip
+    s = settings()
+    box = 256
+    fft, spaces, desc, table = problem(box, 200, s, seed=11)
+    spaces["transformInv"][:, 2, :] *= np.float32(1500)
+    ov, ow, updates = run_oracle(s, fft, spaces, table, box)
+    v, w, n = run_hip(s, fft, spaces, desc, table, box, strategy=strategy, count=True)
+    assert n == updates > 0
+    if strategy == F.FR_EXACT:
+        assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()
+        v, w, _ = run_hip(s, fft, spaces, desc, table, box)
+        assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()

@@ -143,13 +143,15 @@ constexpr float kHalfEdge = 0.5f * (kEdge - 1);
 // |qz| <= r (1 + 1e-6) holds wherever the float qz * qz is at most the float r * r
 constexpr float kSlabMargin = 1.f + 1e-6f;
 
-// The slab test's bound for half width `r`.  With u = 2^-24 and v the volume's depth, t22 pz rounds
-// by at most u v / 2 in either sum; the sums near the slab are below 16 and round by 16 u at most,
-// eight times where qz steps: together less than u (v + 160) = 6e-8 (v + 160).
-__device__ __forceinline__ float slab_reach(float r, int v)
+// The slab test's bound for half width `r` and transforms of |t22| up to `t` (see slab_queue).  With
+// u = 2^-24 and v the volume's depth: in either sum t22 pz rounds by at most u t v / 2, and a sum by
+// u times its size, which is r where the voxel passes and at most r + 7 t at the up to eight levels
+// that qz steps through: together less than u ((v + 56) t + 9 r), u = 6e-8.
+__device__ __forceinline__ float slab_reach(float r, int v, float t)
 {
-  return r * kSlabMargin + 1e-7f * (float)(v + 160);
+  return r * kSlabMargin + 1e-7f * ((float)(v + 64) * t + 10.f * r);
 }
+constexpr float kSlabT22 = 2.f;  // rotations, and more; larger ones: slab_limit
 
 // Brick of the work item and the lane's column of it.
 struct BrickCtx {
@@ -275,12 +277,16 @@ __device__ __forceinline__ void store_brick(const Scratch &ws, const FrJob &a,
 // the record (box 1024, D7: 141.5 -> 131.2 ms per 512-slice step), while closer bricks load every
 // field at once (box 256: the early rejection would cost 1 to 3 %).
 constexpr float kEarlyCullRadius = 128.f;
+// `t22` is the record's |t22| (0 past the last space).
 template <bool kEarly>
-__device__ __forceinline__ bool cull_space(const FrJob &a, const BrickCtx &b, int si, int sEnd)
+__device__ __forceinline__ bool cull_space(const FrJob &a, const BrickCtx &b, int si, int sEnd,
+                                           float &t22)
 {
+  t22 = 0.f;
   if (si >= sEnd) return false;
   const umpa_traverse_space &sp = a.spaces[si];
   const float(*t)[3] = sp.transformInv;
+  t22 = fabsf(t[2][2]);
   const float qz = t[2][0] * b.bcx + t[2][1] * b.bcy + t[2][2] * b.bcz;
   const float ez = kHalfEdge * (fabsf(t[2][0]) + fabsf(t[2][1])) + b.hz * fabsf(t[2][2]);
   const bool slab = fabsf(qz) <= a.cullHalfWidth + ez + b.eps;
@@ -296,25 +302,35 @@ __device__ __forceinline__ bool cull_space(const FrJob &a, const BrickCtx &b, in
          (dir >= 0) & (dir <= 2);
 }
 
+// The column's limit of the slab test for 64 spaces, `t22` from the lane's: its limit for transforms
+// up to kSlabT22, or where one of them is larger, for the largest.  (Decided per 64 spaces: a bound
+// per space took the exact strategy's box 256 from 1231 to 1241 us.)
+__device__ __forceinline__ float slab_limit(float usual, const FrJob &a, const BrickCtx &b, float r,
+                                            float t22)
+{
+  if (!__any(!(t22 <= kSlabT22))) return usual;
+  for (int d = 32; d > 0; d >>= 1) t22 = fmaxf(t22, __shfl_xor(t22, d));
+  return b.colIn ? slab_reach(r, a.vz, fmaxf(t22, kSlabT22)) : -1.f;
+}
+
 // Phase 1: the slab test of the column's nz voxels; the voxels that pass go to the wave's queue
 // behind `pending` entries (index k * 64 + lane, plus `tag`), their number is returned.
 // qz steps by t22 from level to level, one addition each where the reference's left-to-right sum
-// (t20 px + t21 py) + t22 pz takes a conversion, a product and an addition; `slabR` is above the
-// slab's half width by what the two can differ (slab_reach), so that |qz| <= slabR holds for every
+// (t20 px + t21 py) + t22 pz takes a conversion, a product and an addition; `lim` is above the
+// slab's half width by what the two can differ (slab_reach), so that |qz| <= lim holds for every
 // voxel that passes the reference's rounded q.z^2 <= r^2, which phase 2 tests: one compare per
 // level, whose lane mask is the ballot.  (A column outside the volume compares against -1, which
 // nothing passes.)  Box 256, 1,000 slices: fast math 1100 -> 1094 us, exact 1236 -> 1231; box 1024,
 // D7, FP16 116.7 -> 114.9 ms; mixed batch 3710 -> 3671 us.
 template <typename Scratch>
 __device__ __forceinline__ int slab_queue(Scratch &ws, const FrJob &a, const BrickCtx &b,
-                                          const umpa_traverse_space &sp, float slabR, int lane,
+                                          const umpa_traverse_space &sp, float lim, int lane,
                                           int pending = 0, uint32_t tag = 0)
 {
   const int cyi = a.c.cMaxVolumeIndexYZ / 2;
   const float t20 = sp.transformInv[2][0], t21 = sp.transformInv[2][1],
               t22 = sp.transformInv[2][2];
   const float cz = t20 * b.px + t21 * b.py;
-  const float lim = b.colIn ? slabR : -1.f;
   uint32_t entry = (uint32_t)lane | tag;
   int end = pending;
   float qz = cz + t22 * (float)(b.z0 - cyi);
@@ -394,10 +410,12 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
     const int cxi = c.cMaxVolumeIndexX / 2, cyi = c.cMaxVolumeIndexYZ / 2;
     // phase-1 filter on the slab coordinate: the reference's own test for blobs; for the
     // nearest-neighbour traversal the visited voxel lies within 1.5 of the plane
-    const float slabR = slab_reach(kMode == kModeNearest ? 1.6f : c.cBlobRadius, a.vz);
+    const float slab = kMode == kModeNearest ? 1.6f : c.cBlobRadius;
+    const float reach = slab_reach(slab, a.vz, kSlabT22);
     if (heavy) __builtin_amdgcn_s_setprio(2);
     // the lane owns the z column (x, y, z0 .. z0 + depth - 1) of the brick
     const BrickCtx bk = make_brick(a, bo, lane);
+    const float usual = bk.colIn ? reach : -1.f;  // the slab test's limit (slab_limit)
     const int bz = bk.z0;
     const float ox = (float)(bo.x - cxi), oy = (float)(bo.y - cyi), oz = (float)(bz - cyi);
     bool loaded = false;  // the sums are read when the first space reaches the brick
@@ -405,9 +423,11 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
     const bool earlyCull = __builtin_amdgcn_readfirstlane((int)(bk.dmin > kEarlyCullRadius)) != 0;
     unsigned long long nupd = 0;
     for (int base = sBegin; base < sEnd; base += 64) {
+      float t22;
       unsigned long long mask = earlyCull
-                                  ? __ballot(cull_space<true>(a, bk, base + lane, sEnd))
-                                  : __ballot(cull_space<false>(a, bk, base + lane, sEnd));
+                                  ? __ballot(cull_space<true>(a, bk, base + lane, sEnd, t22))
+                                  : __ballot(cull_space<false>(a, bk, base + lane, sEnd, t22));
+      const float lim = slab_limit(usual, a, bk, slab, t22);
       if (mask && !loaded) {
         load_brick(ws, a, bk, lane, split);
         loaded = true;
@@ -438,7 +458,7 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
 
         // phase 1: slab test of the column's nz voxels (nz is wave-uniform: shallow bricks
         // run fewer levels)
-        const int cnt = slab_queue(ws, a, bk, sp, slabR, lane);
+        const int cnt = slab_queue(ws, a, bk, sp, lim, lane);
         if (cnt == 0) continue;
         wave_sync();
         const bool unit = sp.weight == 1.f;
@@ -620,10 +640,11 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fr_insert_carry_kernel(FrJob j
     const bool split = parts > 1;
     const int sBegin = split ? s0 + (int)((int64_t)(s1 - s0) * part / parts) : s0;
     const int sEnd = split ? s0 + (int)((int64_t)(s1 - s0) * (part + 1) / parts) : s1;
-    const float slabR = slab_reach(a.c.cBlobRadius, a.vz);
+    const float slab = a.c.cBlobRadius, reach = slab_reach(slab, a.vz, kSlabT22);
     const int cxi = a.c.cMaxVolumeIndexX / 2, cyi = a.c.cMaxVolumeIndexYZ / 2;
     if (heavy) __builtin_amdgcn_s_setprio(2);
     const BrickCtx bk = make_brick(a, bo, lane);
+    const float usual = bk.colIn ? reach : -1.f;  // the slab test's limit (slab_limit)
     const int bz = bk.z0;
     load_brick(ws, a, bk, lane, split);
     bool loaded = false;
@@ -636,9 +657,11 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fr_insert_carry_kernel(FrJob j
     int pendSpaces = 0;  // spaces they come from (at most 2)
     int slot = 0;        // record slot of the next space
     for (int base = sBegin; base < sEnd; base += 64) {
+      float t22;
       unsigned long long mask = earlyCull
-                                  ? __ballot(cull_space<true>(a, bk, base + lane, sEnd))
-                                  : __ballot(cull_space<false>(a, bk, base + lane, sEnd));
+                                  ? __ballot(cull_space<true>(a, bk, base + lane, sEnd, t22))
+                                  : __ballot(cull_space<false>(a, bk, base + lane, sEnd, t22));
+      const float lim = slab_limit(usual, a, bk, slab, t22);
       if (mask && !loaded) {
         loaded = true;
       }
@@ -670,7 +693,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fr_insert_carry_kernel(FrJob j
         const bool ins = brick_inside(bk, slots[slot].rec, cxi, cyi);
         if (lane == 0) slots[slot].inside = ins ? 1 : 0;
         const int cnt =
-          slab_queue(ws, a, bk, slots[slot].rec, slabR, lane, pending, (uint32_t)slot << 9);
+          slab_queue(ws, a, bk, slots[slot].rec, lim, lane, pending, (uint32_t)slot << 9);
         if (cnt == 0) continue;  // the slot stays free for the next space
         pending += cnt;
         ++pendSpaces;
@@ -785,7 +808,7 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
     (void *)a.fft, 0, (int)((uint32_t)a.nProj * sliceBytes), kBufferConfig);
   const umpa_fr_constants &c = a.c;
   const int cxi = c.cMaxVolumeIndexX / 2, cyi = c.cMaxVolumeIndexYZ / 2;
-  const float slabR = slab_reach(c.cBlobRadius, a.vz);
+  const float slab = c.cBlobRadius, reach = slab_reach(slab, a.vz, kSlabT22);
 
   const int sBegin = a.spaceBegin, sEnd = a.spaceEnd;
   if (sBegin >= sEnd) return;
@@ -807,6 +830,7 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
     const bool heavy = (bo.w >> 4) & 1;
     if (heavy) __builtin_amdgcn_s_setprio(2);
     const BrickCtx bk = make_brick(a, bo, lane);
+    const float usual = bk.colIn ? reach : -1.f;  // the slab test's limit (slab_limit)
     const int bz = bk.z0;
     const float ox = (float)(bo.x - cxi), oy = (float)(bo.y - cyi), oz = (float)(bz - cyi);
     bool loaded = false;  // the sums are read when the first space reaches the brick
@@ -815,9 +839,11 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
     int head = 0, waiting = 0;  // the ring's oldest entry and its number of entries
     uint32_t ordinal = 0;       // spaces taken so far by this work item (mod 2^16)
     for (int base = sBegin; base < sEnd; base += 64) {
+      float t22;
       unsigned long long mask = earlyCull
-                                  ? __ballot(cull_space<true>(a, bk, base + lane, sEnd))
-                                  : __ballot(cull_space<false>(a, bk, base + lane, sEnd));
+                                  ? __ballot(cull_space<true>(a, bk, base + lane, sEnd, t22))
+                                  : __ballot(cull_space<false>(a, bk, base + lane, sEnd, t22));
+      const float lim = slab_limit(usual, a, bk, slab, t22);
       if (mask && !loaded) {
         load_brick(ws, a, bk, lane, false);
         loaded = true;
@@ -830,7 +856,7 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
         const uint32_t sliceOff =
           (uint32_t)__builtin_amdgcn_readfirstlane(sp.projectionIndex) * sliceBytes;
         // phase 1: the slab test, as in fr_insert_kernel
-        const int cnt = slab_queue(ws, a, bk, sp, slabR, lane);
+        const int cnt = slab_queue(ws, a, bk, sp, lim, lane);
         if (cnt == 0) continue;
         wave_sync();
         const bool inside = brick_inside(bk, sp, cxi, cyi);

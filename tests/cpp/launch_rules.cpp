@@ -1,5 +1,7 @@
 // Prints what the library's launch rules choose, host arithmetic only: one line per line of input.
-//   insert key=value ...   choose_fr_insert of a launch: "<which> <blocks> <threads> <lds> <kernel>"
+//   insert key=value ...        choose_fr_insert of a launch: "<which> <blocks> <threads> <lds> <kernel>"
+//   batch_tuner key=value ...   what the batch tuner times: "<kernel>,<boxFixed>" of the first schedule
+//                               and of the candidates over it, then the number of schedules
 #include <dlfcn.h>
 
 #include <cstdio>
@@ -74,6 +76,17 @@ void insert()
   std::printf("%d %d %d %zu %s\n", c.which, c.blocks, c.threads, c.lds, name_of(c.kernel));
 }
 
+void batch_tuner()
+{
+  const bool half = arg("half") != 0, fast = half || arg("fast") != 0;
+  const auto schedules = umpa::host::batch_tuning_candidates(
+    fast, umpa::host::batch_auto_kernel(fast, half, arg("bounded") != 0));
+  std::printf("%d,%d", schedules[0].kernel, schedules[0].boxFixed ? 1 : 0);
+  for (const auto &c : umpa::host::batch_kernel_candidates(schedules[0], fast))
+    std::printf(" %d,%d", c.kernel, c.boxFixed ? 1 : 0);
+  std::printf(" %zu\n", schedules.size());
+}
+
 }  // namespace
 
 int main()
@@ -89,6 +102,7 @@ int main()
       g_args[word.substr(0, eq)] = eq == std::string::npos ? 1 : std::stod(word.substr(eq + 1));
     }
     if (command == "insert") insert();
+    else if (command == "batch_tuner") batch_tuner();
     else return 2;
   }
   return 0;

@@ -35,3 +35,18 @@ def test_largest_table_of_the_carried_queues():
              for b in (0, 1) for n in (10747, 10748, 10751, 10752)]
     got = [c[0] for c in L.choices(cases)]
     assert got == [L.CARRY, L.CARRY, L.CARRY, L.PAIR, L.CARRY, L.PAIR, L.PAIR, L.PAIR]
+
+
+@pytest.mark.parametrize("case,first", [({"fast": 1}, "2,0"), ({"fast": 1, "bounded": 1}, "1,0"),
+                                        ({"half": 1}, "1,0"), ({"half": 1, "bounded": 1}, "1,0")])
+def test_batch_tuner_times_each_kernel_and_box_once(case, first):
+    """Fast math: the schedules run by the kernel such launches run by default, by its name; over the
+    fastest, per-pair and carried kernel with sliding and fixed boxes, each combination once."""
+    *got, schedules = L.ask("batch_tuner", [case])[0]
+    assert got[0] == first and sorted(got) == ["1,0", "1,1", "2,0", "2,1"]
+    assert int(schedules) == 24
+
+
+def test_batch_tuner_exact():
+    got = L.ask("batch_tuner", [{}])[0]
+    assert got == ["0,0", "6"]  # the schedules; one kernel

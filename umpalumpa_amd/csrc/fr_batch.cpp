@@ -226,17 +226,17 @@ void build_step(umpa_fr_batch *b, const std::vector<JobInfo> &infos,
     LaunchImage li{};
     li.v = first.v;
     // the carried-queue kernel reads a job's slices through one buffer resource: it runs only if
-    // every job's slices fit one, when the knob names it, or by default for the launches it is the
-    // faster kernel of (us, per pair / carried, boxes 64 to 320: FP32 3868 / 3751, FP16 3666 / 3781;
-    // bounded FP32, boxes 96 to 256, 1382 / 1390, FP16 1285 / 1390)
+    // every job's slices fit one
     bool carryFits = true;
     for (const umpa::FrJob &rec : recs)
       carryFits = carryFits && (uint64_t)rec.nProj * (uint64_t)rec.sliceElems *
                                    (li.v.half ? 4u : 8u) <= 0x7fff0000ull;
-    const bool wanted = sp.kernel == UMPA_FR_KERNEL_AUTO
-                          ? li.v.fastMath && !li.v.half && b->waveItems == 0
-                          : sp.kernel == UMPA_FR_KERNEL_CARRY;
-    li.v.kernel = wanted && carryFits ? UMPA_FR_KERNEL_CARRY : UMPA_FR_KERNEL_PAIR;
+    const int wanted =
+      sp.kernel == UMPA_FR_KERNEL_AUTO
+        ? umpa::host::batch_auto_kernel(li.v.fastMath, li.v.half, b->waveItems > 0)
+        : sp.kernel;
+    li.v.kernel = wanted == UMPA_FR_KERNEL_CARRY && carryFits ? UMPA_FR_KERNEL_CARRY
+                                                              : UMPA_FR_KERNEL_PAIR;
     // the sliding-box instantiation only when every job of the launch slides
     li.v.shift = std::all_of(recs.begin(), recs.end(),
                              [](const umpa::FrJob &r) { return r.shiftBox != 0; });
@@ -581,30 +581,19 @@ static int batch_autotune_impl(umpa_fr_batch *b, const umpa_fr_job *jobs, uint32
   if (e == hipSuccess) e = hipEventCreate(&t0);
   if (e == hipSuccess) e = hipEventCreate(&t1);
   double bestMs = 1e300;
-  // batches keep the table in LDS and run the per-pair kernel or (fast math) the carried
-  // queues: those and boxFixed are tried over the fastest schedule
-  std::vector<umpa::host::SchedParams> cands;
-  for (auto c : umpa::host::tuning_candidates(fastMath)) {
-    c.kernel = UMPA_FR_KERNEL_AUTO;
-    c.tableGlobal = false;
-    const bool dup = std::any_of(cands.begin(), cands.end(), [&](const auto &o) {
-      return o.depthScale == c.depthScale && o.priority == c.priority &&
-             o.maxParts == c.maxParts && o.splitAt == c.splitAt;
-    });
-    if (!dup) cands.push_back(c);
-  }
-  const size_t nSched = cands.size(), nCand = nSched + (fastMath ? 3 : 0);
+  // batches keep the table in LDS: the schedules run by the launches' default kernel (by each
+  // launch's own where slices of both kinds are among the jobs), then the kernels and boxes over
+  // the fastest of them
+  const bool half = infos[0].v.half;
+  const bool mixed = std::any_of(infos.begin(), infos.end(),
+                                 [&](const JobInfo &j) { return j.v.half != half; });
+  std::vector<umpa::host::SchedParams> cands = umpa::host::batch_tuning_candidates(
+    fastMath, mixed ? UMPA_FR_KERNEL_AUTO
+                    : umpa::host::batch_auto_kernel(fastMath, half, b->waveItems > 0));
+  const size_t nSched = cands.size();
   try {
-    for (size_t ci = 0; ci < nCand; ++ci) {
+    for (size_t ci = 0; ci < cands.size(); ++ci) {
       if (e != hipSuccess) break;
-      if (ci == nSched) {  // the fastest schedule: fixed boxes, carried queues, both
-        for (int k = 1; k <= 3; ++k) {
-          umpa::host::SchedParams c = best;
-          c.boxFixed = (k & 1) != 0;
-          c.kernel = (k & 2) ? UMPA_FR_KERNEL_CARRY : UMPA_FR_KERNEL_AUTO;
-          cands.push_back(c);
-        }
-      }
       const umpa::host::SchedParams cand = cands[ci];
       std::vector<char> blob;
       std::vector<LaunchImage> launches;
@@ -632,6 +621,9 @@ static int batch_autotune_impl(umpa_fr_batch *b, const umpa_fr_job *jobs, uint32
         bestMs = ms;
         best = cand;
       }
+      if (ci + 1 == nSched)
+        for (const auto &c : umpa::host::batch_kernel_candidates(best, fastMath))
+          cands.push_back(c);
     }
   } catch (const std::bad_alloc &) {
     e = hipErrorOutOfMemory;

@@ -731,6 +731,43 @@ std::vector<SchedParams> kernel_candidates(const SchedParams &base, bool fastMat
   return out;
 }
 
+// The carried queues where they are the faster kernel (us, per pair / carried, boxes 64 to 320: FP32
+// 3868 / 3751, FP16 3666 / 3781; bounded FP32, boxes 96 to 256, 1382 / 1390, FP16 1285 / 1390).
+int batch_auto_kernel(bool fastMath, bool half, bool bounded)
+{
+  return fastMath && !half && !bounded ? UMPA_FR_KERNEL_CARRY : UMPA_FR_KERNEL_PAIR;
+}
+
+std::vector<SchedParams> batch_tuning_candidates(bool fastMath, int kernel)
+{
+  std::vector<SchedParams> out;
+  for (SchedParams c : tuning_candidates(fastMath)) {
+    c.kernel = fastMath ? kernel : UMPA_FR_KERNEL_AUTO;  // (exact batches have one kernel)
+    c.tableGlobal = false;
+    const bool dup = std::any_of(out.begin(), out.end(), [&](const SchedParams &o) {
+      return o.depthScale == c.depthScale && o.priority == c.priority &&
+             o.maxParts == c.maxParts && o.splitAt == c.splitAt;
+    });
+    if (!dup) out.push_back(c);
+  }
+  return out;
+}
+
+std::vector<SchedParams> batch_kernel_candidates(const SchedParams &best, bool fastMath)
+{
+  std::vector<SchedParams> out;
+  if (!fastMath) return out;
+  for (int kernel : { UMPA_FR_KERNEL_PAIR, UMPA_FR_KERNEL_CARRY })
+    for (bool fixed : { false, true }) {
+      if (kernel == best.kernel && fixed == best.boxFixed) continue;  // timed already
+      SchedParams c = best;
+      c.kernel = kernel;
+      c.boxFixed = fixed;
+      out.push_back(c);
+    }
+  return out;
+}
+
 namespace {
 std::mutex g_cacheMutex;
 

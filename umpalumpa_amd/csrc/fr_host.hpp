@@ -127,4 +127,13 @@ std::vector<SchedParams> tuning_candidates(bool fastMath);
 // Second stage (fast math only, else empty): the kernel knobs over the schedule `base`.
 std::vector<SchedParams> kernel_candidates(const SchedParams &base, bool fastMath);
 
+// The kernel that UMPA_FR_KERNEL_AUTO means in a batch's launch (per pair where the carried queues
+// do not cover the launch).
+int batch_auto_kernel(bool fastMath, bool half, bool bounded);
+// The batch tuner's first stage: the distinct schedules of tuning_candidates, all run by `kernel`,
+// which fast math names; then (fast math only, else empty) the other kernel and boxes over the
+// schedule `best`.
+std::vector<SchedParams> batch_tuning_candidates(bool fastMath, int kernel);
+std::vector<SchedParams> batch_kernel_candidates(const SchedParams &best, bool fastMath);
+
 }  // namespace umpa::host

@@ -2,6 +2,7 @@
 //   insert key=value ...        choose_fr_insert of a launch: "<which> <blocks> <threads> <lds> <kernel>"
 //   batch_tuner key=value ...   what the batch tuner times: "<kernel>,<boxFixed>" of the first schedule
 //                               and of the candidates over it, then the number of schedules
+//   op_tuner key=value ...      the kernels of an operation's schedule candidates
 #include <dlfcn.h>
 
 #include <cstdio>
@@ -87,6 +88,14 @@ void batch_tuner()
   std::printf(" %zu\n", schedules.size());
 }
 
+void op_tuner()
+{
+  const bool half = arg("half") != 0, fast = half || arg("fast") != 0;
+  for (const auto &c : umpa::host::op_tuning_candidates(fast, half, arg("cells") != 0))
+    std::printf("%d ", c.kernel);
+  std::printf("\n");
+}
+
 }  // namespace
 
 int main()
@@ -103,6 +112,7 @@ int main()
     }
     if (command == "insert") insert();
     else if (command == "batch_tuner") batch_tuner();
+    else if (command == "op_tuner") op_tuner();
     else return 2;
   }
   return 0;

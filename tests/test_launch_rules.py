@@ -50,3 +50,13 @@ def test_batch_tuner_times_each_kernel_and_box_once(case, first):
 def test_batch_tuner_exact():
     got = L.ask("batch_tuner", [{}])[0]
     assert got == ["0,0", "6"]  # the schedules; one kernel
+
+
+def test_op_tuner_times_schedules_where_the_default_is_cells():
+    """Where the default kernel may be the small-problem kernel, which runs no schedule, every
+    schedule names a brick kernel; elsewhere fast math leaves the kernel to the launch."""
+    fast, half, exact, plain = L.ask("op_tuner", [{"fast": 1, "cells": 1}, {"half": 1, "cells": 1},
+                                                  {"cells": 1}, {"fast": 1}])
+    assert set(fast) == {str(L.CARRY)} and set(half) == {str(L.PAIR)} and set(plain) == {"0"}
+    assert set(exact) == {str(L.STAGED), str(L.PAIR)}
+    assert len(fast) == len(half) == len(exact) == len(plain) == 24

@@ -569,18 +569,19 @@ static int fr_autotune_impl(umpa_fr_op *op, const void *fft, const float *scales
       }
     };
     try {
-      // the default choice where it may be the small-problem kernel, which no knob names
-      if (op->nCells > 0) {
-        umpa::host::SchedParams def;
-        if (!v.fastMath) def.maxParts = 1;
-        time_candidate(def);
-      }
       // schedules (exact: with every kernel knob), then the kernel knobs over the best one
-      for (const auto &cand : umpa::host::tuning_candidates(v.fastMath))
+      const bool cells = op->nCells > 0;
+      for (const auto &cand : umpa::host::op_tuning_candidates(v.fastMath, half, cells))
         if (e == hipSuccess) time_candidate(cand);
       const umpa::host::SchedParams sched = best;
       for (const auto &cand : umpa::host::kernel_candidates(sched, v.fastMath))
         if (e == hipSuccess) time_candidate(cand);
+      // the default choice where it may be the small-problem kernel, which no knob names
+      if (cells && e == hipSuccess) {
+        umpa::host::SchedParams def;
+        if (!v.fastMath) def.maxParts = 1;
+        time_candidate(def);
+      }
     } catch (const std::bad_alloc &) {
       e = hipErrorOutOfMemory;
     }

@@ -731,6 +731,16 @@ std::vector<SchedParams> kernel_candidates(const SchedParams &base, bool fastMat
   return out;
 }
 
+std::vector<SchedParams> op_tuning_candidates(bool fastMath, bool half, bool cells)
+{
+  std::vector<SchedParams> out = tuning_candidates(fastMath);
+  if (cells)
+    for (SchedParams &c : out)
+      if (c.kernel == UMPA_FR_KERNEL_AUTO)
+        c.kernel = half ? UMPA_FR_KERNEL_PAIR : UMPA_FR_KERNEL_CARRY;
+  return out;
+}
+
 // The carried queues where they are the faster kernel (us, per pair / carried, boxes 64 to 320: FP32
 // 3868 / 3751, FP16 3666 / 3781; bounded FP32, boxes 96 to 256, 1382 / 1390, FP16 1285 / 1390).
 int batch_auto_kernel(bool fastMath, bool half, bool bounded)

@@ -127,6 +127,11 @@ std::vector<SchedParams> tuning_candidates(bool fastMath);
 // Second stage (fast math only, else empty): the kernel knobs over the schedule `base`.
 std::vector<SchedParams> kernel_candidates(const SchedParams &base, bool fastMath);
 
+// The first stage for an operation.  Where `cells` (its launch may be the small-problem kernel,
+// which UMPA_FR_KERNEL_AUTO then means, whatever the schedule), the schedules name the brick kernel
+// that AUTO means otherwise, so that what is timed is theirs.
+std::vector<SchedParams> op_tuning_candidates(bool fastMath, bool half, bool cells);
+
 // The kernel that UMPA_FR_KERNEL_AUTO means in a batch's launch (per pair where the carried queues
 // do not cover the launch).
 int batch_auto_kernel(bool fastMath, bool half, bool bounded);

@@ -3,6 +3,8 @@
 //   batch_tuner key=value ...   what the batch tuner times: "<kernel>,<boxFixed>" of the first schedule
 //                               and of the candidates over it, then the number of schedules
 //   op_tuner key=value ...      the kernels of an operation's schedule candidates
+//   op_key key=value ...        the key of an operation's tuning result: Init told of `init` spaces
+//   batch_key key=value ...     ... of a batch of one job
 #include <dlfcn.h>
 
 #include <cstdio>
@@ -96,6 +98,27 @@ void op_tuner()
   std::printf("\n");
 }
 
+void op_key()
+{
+  const int side = (int)arg("box") + 1;
+  const bool half = arg("half") != 0, fast = half || arg("fast") != 0;
+  const umpa_fr_settings s = settings();
+  const uint64_t spaces = (uint64_t)arg("spaces"), init = (uint64_t)arg("init", arg("spaces"));
+  std::printf("%s\n", umpa::host::op_tuning_key(
+                        256, umpa::kModeLookup, fast, half, umpa::host::footprint(s), side, spaces,
+                        umpa::host::plain_depth_scale(side, side, side, init, s, fast),
+                        umpa::host::share_cells(side, side, side, init, s)).c_str());
+}
+
+void batch_key()
+{
+  const bool half = arg("half") != 0, fast = half || arg("fast") != 0;
+  std::printf("%s\n", umpa::host::batch_tuning_key(
+                        256, umpa::kModeLookup, fast, half, umpa::host::footprint(settings()),
+                        arg("bounded") != 0,
+                        { { (int)arg("box") + 1, (int)arg("spaces") } }).c_str());
+}
+
 }  // namespace
 
 int main()
@@ -113,6 +136,8 @@ int main()
     if (command == "insert") insert();
     else if (command == "batch_tuner") batch_tuner();
     else if (command == "op_tuner") op_tuner();
+    else if (command == "op_key") op_key();
+    else if (command == "batch_key") batch_key();
     else return 2;
   }
   return 0;

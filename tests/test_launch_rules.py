@@ -60,3 +60,19 @@ def test_op_tuner_times_schedules_where_the_default_is_cells():
     assert set(fast) == {str(L.CARRY)} and set(half) == {str(L.PAIR)} and set(plain) == {"0"}
     assert set(exact) == {str(L.STAGED), str(L.PAIR)}
     assert len(fast) == len(half) == len(exact) == len(plain) == 24
+
+
+def test_tuning_keys_name_all_that_a_launch_depends_on():
+    """Lines written when a knob meant another launch have other keys; so have launches whose depth
+    scale or cells differ by what Init was told, and bounded and unbounded batches."""
+    old_op, old_batch = "k2:op:cu256:m0:f1:h0:nb4:129x128", "k2:batch:cu256:m0:f1:h0:nb4:129x100,"
+    job = {"box": 128, "spaces": 100, "fast": 1}
+    small = {"box": 48, "spaces": 50, "fast": 1}
+    keys = [k for k, in L.ask("op_key", [job, {**job, "init": 1500}, {**job, "spaces": 1500},
+                                         small, {**small, "init": 200}])]
+    keys += [k for k, in L.ask("batch_key", [job, {**job, "bounded": 1}])]
+    assert len(set(keys)) == len(keys)
+    assert old_op not in keys and old_batch not in keys
+    # launches that do not differ share their line
+    a, b = L.ask("op_key", [{**job, "spaces": 70}, {**job, "spaces": 128}])
+    assert a == b

@@ -116,3 +116,20 @@ def test_transforms_that_are_no_rotation(strategy):
         assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()
         v, w, _ = run_hip(s, fft, spaces, desc, table, box)
         assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()
+
+
+def test_older_tuning_lines_are_not_used(tmp_path, monkeypatch):
+    """A line that a build wrote in which its knobs meant other launches is no result for this one:
+    the tuner times its candidates and writes a line of its own."""
+    monkeypatch.setenv("UMPA_TUNING_DIR", str(tmp_path))
+    dev = torch.device("cuda:0")
+    s = settings()
+    fft, spaces, desc, table = problem(48, 30, s)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    path = tmp_path / "fr_tuning.txt"
+    path.write_text(f"k2:op:cu{cus}:m0:f0:h0:nb4:49x32 0.5 0 1 0.5 1 1 0 0.1\n")
+    op = F.FourierReconstruction(0)
+    assert op.init(desc, s)
+    d = [torch.from_numpy(a).to(dev) for a in (fft, spaces.view(np.uint8), table)]
+    op.autotune(*d, use_cache=True)
+    assert len(path.read_text().splitlines()) == 2

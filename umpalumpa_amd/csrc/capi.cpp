@@ -501,14 +501,10 @@ static int fr_autotune_impl(umpa_fr_op *op, const void *fft, const float *scales
   v.count = false;
   const int slot = v.fastMath ? 1 : 0;
   const int vx = (int)op->desc.volume.x, vy = (int)op->desc.volume.y, vz = (int)op->desc.volume.z;
-  // spaces bucketed to a power of two
-  uint64_t bucket = 1;
-  while (bucket < nSpaces) bucket <<= 1;
-  // "k2": the format of lines with kernel knobs
-  const std::string key = "k2:op:cu" + std::to_string(op->numCUs) + ":m" +
-                          std::to_string(v.mode) + ":f" + std::to_string(slot) + ":h" +
-                          std::to_string(half ? 1 : 0) + ":nb" + std::to_string(v.nb) + ":" +
-                          std::to_string(vx) + "x" + std::to_string(bucket);
+  const std::string key = umpa::host::op_tuning_key(
+    op->numCUs, v.mode, v.fastMath, half, v.nb, vx, nSpaces,
+    umpa::host::plain_depth_scale(vx, vy, vz, op->desc.traverseSpaces, op->settings, v.fastMath),
+    op->cellsShared);
   umpa::host::SchedParams best = op->params[slot];
   bool found = useCache && umpa::host::tuning_cache_lookup(key, best);
   hipError_t e = hipSuccess;

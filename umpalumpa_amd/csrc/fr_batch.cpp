@@ -536,7 +536,6 @@ static int batch_autotune_impl(umpa_fr_batch *b, const umpa_fr_job *jobs, uint32
   const bool fastMath = infos[0].v.fastMath;
   for (const auto &j : infos)
     if (j.v.fastMath != fastMath) return UMPA_ERR_INVALID_ARG;
-  // key: device, strategy, precision, footprint, and the first step's (volume, spaces) list
   std::vector<std::pair<int, int>> shape;
   std::vector<std::tuple<int, int, int>> ranges;
   for (uint32_t i = 0; i < nJobs; ++i) {
@@ -545,11 +544,9 @@ static int batch_autotune_impl(umpa_fr_batch *b, const umpa_fr_job *jobs, uint32
     shape.emplace_back(infos[i].rec.vx, s1);
   }
   std::sort(shape.begin(), shape.end());
-  std::string key = "k2:batch:cu" + std::to_string(b->numCUs) + ":m" +
-                    std::to_string(infos[0].v.mode) + ":f" + std::to_string(fastMath ? 1 : 0) +
-                    ":h" + std::to_string(infos[0].v.half ? 1 : 0) + ":nb" +
-                    std::to_string(infos[0].v.nb) + ":";
-  for (auto &p : shape) key += std::to_string(p.first) + "x" + std::to_string(p.second) + ",";
+  const std::string key =
+    umpa::host::batch_tuning_key(b->numCUs, infos[0].v.mode, fastMath, infos[0].v.half,
+                                 infos[0].v.nb, b->waveItems > 0, shape);
   umpa::host::SchedParams best;
   auto report = [&](const umpa::host::SchedParams &p) {
     b->params[fastMath ? 1 : 0] = p;

@@ -731,6 +731,39 @@ std::vector<SchedParams> kernel_candidates(const SchedParams &base, bool fastMat
   return out;
 }
 
+namespace {
+
+// "k2": lines of seven knobs.  "v2": their meaning: depth scales times the launch's own, AUTO the
+// small-problem kernel, or the carried queues of a batch (lines without it are older).
+std::string key_head(const char *what, int numCUs, int mode, bool fastMath, bool half, int nb)
+{
+  return std::string("k2:") + what + ":v2:cu" + std::to_string(numCUs) + ":m" +
+         std::to_string(mode) + ":f" + std::to_string(fastMath ? 1 : 0) + ":h" +
+         std::to_string(half ? 1 : 0) + ":nb" + std::to_string(nb) + ":";
+}
+
+}  // namespace
+
+std::string op_tuning_key(int numCUs, int mode, bool fastMath, bool half, int nb, int vx,
+                          uint64_t spaces, float depthScale, bool sharedCells)
+{
+  uint64_t bucket = 1;
+  while (bucket < spaces) bucket <<= 1;
+  return key_head("op", numCUs, mode, fastMath, half, nb) + "d" +
+         std::to_string((int)std::lround(100.f * depthScale)) + ":s" +
+         std::to_string(sharedCells ? 1 : 0) + ":" + std::to_string(vx) + "x" +
+         std::to_string(bucket);
+}
+
+std::string batch_tuning_key(int numCUs, int mode, bool fastMath, bool half, int nb, bool bounded,
+                             const std::vector<std::pair<int, int>> &shape)
+{
+  std::string key = key_head("batch", numCUs, mode, fastMath, half, nb) + "b" +
+                    std::to_string(bounded ? 1 : 0) + ":";
+  for (const auto &p : shape) key += std::to_string(p.first) + "x" + std::to_string(p.second) + ",";
+  return key;
+}
+
 std::vector<SchedParams> op_tuning_candidates(bool fastMath, bool half, bool cells)
 {
   std::vector<SchedParams> out = tuning_candidates(fastMath);

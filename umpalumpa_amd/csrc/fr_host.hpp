@@ -3,6 +3,7 @@
 
 #include <cstdint>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "umpalumpa_amd.h"
@@ -113,7 +114,8 @@ std::vector<int> make_cell_blocks(int vx, int vy, int vz, bool share);
 
 // Persisted tuning results: one "key depthScale priority maxParts splitAt kernel tableGlobal
 // boxFixed ms" line per key in $UMPA_TUNING_DIR/fr_tuning.txt (default
-// $HOME/.cache/umpalumpa_amd); keys carry a format tag, so lines of another format are skipped.
+// $HOME/.cache/umpalumpa_amd); keys carry a tag, so lines of another format, or whose knobs meant
+// other launches, are skipped.
 bool tuning_cache_lookup(const std::string &key, SchedParams &out);
 void tuning_cache_store(const std::string &key, const SchedParams &p, double ms);
 
@@ -131,6 +133,15 @@ std::vector<SchedParams> kernel_candidates(const SchedParams &base, bool fastMat
 // which UMPA_FR_KERNEL_AUTO then means, whatever the schedule), the schedules name the brick kernel
 // that AUTO means otherwise, so that what is timed is theirs.
 std::vector<SchedParams> op_tuning_candidates(bool fastMath, bool half, bool cells);
+
+// Keys of the tuning results: all that a launch of given knobs depends on.  An operation's: mode,
+// precision and footprint, volume, launched spaces (to a power of two), and what Init decided by the
+// spaces it was told of: the launch's own depth scale and shared cells.  A batch's: also whether its
+// launches are bounded, and the first step's (volume, spaces), sorted.
+std::string op_tuning_key(int numCUs, int mode, bool fastMath, bool half, int nb, int vx,
+                          uint64_t spaces, float depthScale, bool sharedCells);
+std::string batch_tuning_key(int numCUs, int mode, bool fastMath, bool half, int nb, bool bounded,
+                             const std::vector<std::pair<int, int>> &shape);
 
 // The kernel that UMPA_FR_KERNEL_AUTO means in a batch's launch (per pair where the carried queues
 // do not cover the launch).

@@ -5,6 +5,7 @@
 //   op_tuner key=value ...      the kernels of an operation's schedule candidates
 //   op_key key=value ...        the key of an operation's tuning result: Init told of `init` spaces
 //   batch_key key=value ...     ... of a batch of one job
+//   core key=value ...          cells of a volume's core and bricks beside it (exact launches)
 #include <dlfcn.h>
 
 #include <cstdio>
@@ -119,6 +120,14 @@ void batch_key()
                         { { (int)arg("box") + 1, (int)arg("spaces") } }).c_str());
 }
 
+void core()
+{
+  const int side = (int)arg("box") + 1;
+  const float radius = umpa::host::core_radius(side, side, side);
+  std::printf("%zu %zu\n", umpa::host::core_cells(side, side, side, radius).size() / 2,
+              umpa::host::make_brick_schedule(side, side, side, false, {}, radius).size());
+}
+
 }  // namespace
 
 int main()
@@ -138,6 +147,7 @@ int main()
     else if (command == "op_tuner") op_tuner();
     else if (command == "op_key") op_key();
     else if (command == "batch_key") batch_key();
+    else if (command == "core") core();
     else return 2;
   }
   return 0;

@@ -76,3 +76,16 @@ def test_tuning_keys_name_all_that_a_launch_depends_on():
     # launches that do not differ share their line
     a, b = L.ask("op_key", [{**job, "spaces": 70}, {**job, "spaces": 128}])
     assert a == b
+
+
+@pytest.mark.parametrize("skip", [{"table": 15000}, {"kernel": L.PAIR}, {"kernel": L.STAGED},
+                                  {"count": 1}, {"tableGlobal": 1}])
+@pytest.mark.parametrize("box", [8, 16, 32, 48, 100, 160, 224])
+def test_exact_launches_spread_the_core(box, skip):
+    """Where the centre of a volume is taken as cells by the brick kernels, a launch has wavefronts
+    for them too, up to the GPU's: most of a small volume is cells (box 16: 728, and one brick)."""
+    which, blocks, threads, _, _ = L.choices([{"box": box, "spaces": 100, **skip}])[0]
+    assert which in (L.PAIR, L.STAGED)
+    cells, bricks = (int(n) for n in L.ask("core", [{"box": box}])[0])
+    waves = blocks * threads // 64
+    assert waves >= min(max(cells, bricks), 256 * threads // 64) and blocks <= 256

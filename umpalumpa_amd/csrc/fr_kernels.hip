@@ -1129,7 +1129,8 @@ FrChoice choose_fr_insert(const FrJob &job, const FrLaunch &l, const FrVariant &
     const int64_t per = (int64_t)waves * l.waveItems;
     ch.blocks = (int)((l.nItems + per - 1) / per);
   } else {
-    ch.blocks = (l.nItems + waves - 1) / waves;
+    // (as many as the core has cells or the rest has bricks, whichever is more)
+    ch.blocks = (std::max(l.nItems, l.nCore) + waves - 1) / waves;
     if (ch.blocks > numCUs) ch.blocks = numCUs;
     if (l.maxBlocks > 0 && ch.blocks > l.maxBlocks) ch.blocks = l.maxBlocks;
   }

@@ -247,7 +247,7 @@ __device__ __forceinline__ void cell_item(const FrJob &a, int x0, int y0, int z0
         (uint32_t)si | (in ? kInsideBit<uint32_t> : 0u);
     pend += __popcll(m);
     wave_sync();
-    cell_take<kMode, kOrder, kNB, false, false, kTableLds, kShift, 2, kCount>(
+    cell_take<kMode, kOrder, kNB, false, false, kTableLds, kShift, (kNB <= 5 ? 2 : 1), kCount>(
       cell, a, 0, queue, part, blob, head, pend, base + 64 < sEnd ? 8 : 1, nTable, rsrc, tbl, sliceBytes,
       lane, nupd);
   }

@@ -95,7 +95,7 @@ __global__ __launch_bounds__(kCellThreads, 4) void fr_insert_cell_kernel(FrJob a
   constexpr bool kTableLds = kMode == kModeLookup;
   constexpr int kPix = kHalf ? 4 : 8;
   // rows of the gather in flight: what 128 registers hold beside two spaces' records
-  constexpr int kRows = kHalf ? (kNB <= 4 ? kNB : 3) : kNB <= 3 ? 3 : 2;
+  constexpr int kRows = kHalf ? (kNB <= 4 ? kNB : 3) : kNB <= 3 ? 3 : kNB <= 5 ? 2 : 1;
   extern __shared__ float s_table[];
   __shared__ __align__(16) float s_part[kShared ? 2 : 1][kCellWaves][3 * 64];
   __shared__ int s_hit[kShared ? 2 : 1][kCellWaves];

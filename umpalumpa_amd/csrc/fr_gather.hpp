@@ -197,7 +197,10 @@ __device__ inline Contribution gather_generic(const FrJob &a, int nTable, __amdg
 // reference's table position (int)(d2 * cIDeltaSqrt + 0.5); skipped candidates read the LDS
 // copy's zero entry nTable.  Fast math with the table in LDS: a fused position, clamped into
 // the zero entry, so +inf and every d2 past the blob edge weigh 0 without a test.
-template <int kMode, int kOrder, bool kFastMath, bool kTableLds>
+// kAlwaysRead: the global table is read for skipped candidates too.  A branch each, which spares
+// their reads, is faster (box 64, 30 slices, r 1.9: 52 us, 84 without), but 36 of them, row by row,
+// spill in the six-wide fast-math FP32 kernels (r 2.8, box 112, 60 slices: 437 us, 289 without).
+template <int kMode, int kOrder, bool kFastMath, bool kTableLds, bool kAlwaysRead = false>
 __device__ __forceinline__ float candidate_weight(float d2, float r2, int nTable, const float *tbl,
                                                   const umpa_fr_constants &c)
 {
@@ -226,7 +229,12 @@ __device__ __forceinline__ float candidate_weight(float d2, float r2, int nTable
         return tbl[in ? aux : nTable];  // entry nTable of the LDS copy is 0
       } else {
         aux = aux > nTable - 1 ? nTable - 1 : aux;
-        return in ? tbl[aux] : 0.f;
+        if constexpr (kAlwaysRead) {
+          const float w = tbl[aux];
+          return in ? w : 0.f;
+        } else {
+          return in ? tbl[aux] : 0.f;
+        }
       }
     } else {
       return in ? blob_weight<kMode, kOrder>(d2, c) : 0.f;
@@ -342,7 +350,11 @@ __device__ __forceinline__ bool gather_box(const FrJob &a, int nTable,
   // make it wait for every row before loading the next (1.42 -> 1.84 ms per 1,000-slice chunk
   // at box 256 under the exact strategy).
   constexpr int kVecs = (kNB * kPix + 15) / 16;          // 16-byte loads per row
-  constexpr int kGroup = kRows ? kRows : kVecs == 1 ? kNB : kVecs == 2 ? (kNB <= 4 ? kNB : 3) : 2;
+  // Six FP32 columns go row by row: two rows' pixels and weights spilled up to 74 registers (r 2.8,
+  // 500 slices, box 256: exact 5226 -> 1999 us, fast math 1463 -> 1438; r 3.6 13510 -> 8533), while
+  // five columns want two (r 2.5, exact 1431 us, 1576 row by row).
+  constexpr int kGroup =
+    kRows ? kRows : kVecs == 1 ? kNB : kVecs == 2 ? (kNB <= 4 ? kNB : 3) : kNB == 5 ? 2 : 1;
   // wider boxes under the exact strategy mask skipped pixels, whatever their value
   constexpr bool kMask = kNB > 4 && !(kFastMath && kMode == kModeLookup && kTableLds);
   constexpr bool kSkipOutside = kChunk && !kShift;
@@ -365,8 +377,9 @@ __device__ __forceinline__ bool gather_box(const FrJob &a, int nTable,
       if (g + i >= kNB) continue;
 #pragma unroll
       for (int jj = 0; jj < kNB; ++jj)
-        wr[i][jj] = candidate_weight<kMode, kOrder, kFastMath, kTableLds>(xd2[jj] + yz[g + i], r2,
-                                                                        nTable, tbl, c);
+        wr[i][jj] = candidate_weight<kMode, kOrder, kFastMath, kTableLds,
+                                     kNB == 6 && kFastMath && !kHalf>(xd2[jj] + yz[g + i], r2,
+                                                                      nTable, tbl, c);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll

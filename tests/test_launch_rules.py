@@ -101,3 +101,25 @@ def test_six_wide_fp32_kernels_keep_their_registers(metadata):
     assert len(symbols) >= 10
     for symbol in symbols:
         assert metadata[symbol][".private_segment_fixed_size"] == 0, symbol
+
+
+# (options, largest box of the small-problem kernel, spaces from which it takes that box)
+CELL_RULES = [
+    ({"radius": 1.2}, 104, 240), ({"radius": 1.5}, 104, 240), ({}, 86, 168),
+    ({"radius": 2.5}, 120, 228), ({"radius": 3.6}, 120, 228), ({"fast": 1}, 104, 250),
+    ({"fast": 1, "radius": 2.8}, 104, 250), ({"half": 1}, 114, 300),
+    ({"half": 1, "radius": 2.8}, 96, 210), ({"evaluated": 1}, 120, 180), ({"nearest": 1}, 84, 160)]
+
+
+@pytest.mark.parametrize("options,box,spaces", CELL_RULES)
+def test_lines_of_the_small_problem_kernel(options, box, spaces):
+    """Which launches run the small-problem kernel: boxes up to the line of the mode, radius and
+    precision, from a number of spaces that grows with the box; no counting pass, named kernel or
+    table beyond LDS."""
+    case = {**options, "box": box, "spaces": spaces}
+    others = [{**case, "box": box + 2, "spaces": 5000}, {**case, "spaces": spaces - 1},
+              {**case, "count": 1}, {**case, "kernel": L.PAIR}, {**case, "batched": 1}]
+    if not (options.get("evaluated") or options.get("nearest")):
+        others += [{**case, "table": 11777}, {**case, "tableGlobal": 1}]
+    got = [c[0] for c in L.choices([case, *others])]
+    assert got[0] == L.CELLS and L.CELLS not in got[1:]

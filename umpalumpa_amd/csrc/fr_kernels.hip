@@ -1074,7 +1074,8 @@ hipError_t prepare_fr_insert(const FrVariant &v, int nTable)
 // 390 / 464; r 2.5 100 150 228 / 186, 112 150 202 / 233, 1,200 1165 / 1101, 128 1218 / 1398.  Fast
 // math: 64 60 73 / 47; 80 60 58 / 65, 150 89 / 75; 100 150 102 / 104, 400 188 / 179, 1,200 482 /
 // 462; 112 400 189 / 211; FP16 100 1,200 554 / 433, 112 400 206 / 201, 1,200 541 / 514; 128 400 198 /
-// 253.  Blob evaluated: 80 60 106 / 75, 100 60 114 / 117, 150 192 / 152; 112 60 127 / 146, 150 196 /
+// 253, six columns 96 1,000 r 3.6 3667 / 3208, r 3 811 / 1035, 112 3618 / 3991, 776 / 1100, r 5 6819 /
+// 9500.  Blob evaluated: 80 60 106 / 75, 100 60 114 / 117, 150 192 / 152; 112 60 127 / 146, 150 196 /
 // 188, 400 392 / 334; 128 150 198 / 247.  Nearest: 64 150 62 / 54, 80 150 60 / 65, 1,200 485 / 351;
 // 90 414 / 430.  So, with V the volume's mean extent: from (V - from) * slope spaces, up to a V.
 bool use_cells(const FrJob &job, const FrLaunch &l, const FrVariant &v)
@@ -1088,6 +1089,7 @@ bool use_cells(const FrJob &job, const FrLaunch &l, const FrVariant &v)
   };
   const Rule rule = v.mode == kModeNearest  ? Rule{ 85, 45.f, 4.f }
                     : v.mode != kModeLookup ? Rule{ 121, 85.f, 5.f }
+                    : v.half && v.nb == 6   ? Rule{ 97, 55.f, 5.f }
                     : v.half                ? Rule{ 115, 55.f, 5.f }
                     : v.fastMath            ? Rule{ 105, 55.f, 5.f }
                     : v.nb == 3             ? Rule{ 105, 45.f, 4.f }

@@ -2,7 +2,9 @@
 import numpy as np
 import pytest
 
+import launchtools
 from frtools import problem, rel_l2, run_oracle, settings
+from test_launch_rules import CELL_RULES
 from umpalumpa_amd import fr as F
 
 pytestmark = pytest.mark.gpu
@@ -133,3 +135,81 @@ def test_older_tuning_lines_are_not_used(tmp_path, monkeypatch):
     d = [torch.from_numpy(a).to(dev) for a in (fft, spaces.view(np.uint8), table)]
     op.autotune(*d, use_cache=True)
     assert len(path.read_text().splitlines()) == 2
+
+
+@pytest.mark.parametrize("options,box,spaces", CELL_RULES)
+def test_volumes_on_either_side_of_the_small_problem_kernels_line(options, box, spaces):
+    """The largest volume of the small-problem kernel in each mode, and the next box, which bricks
+    take, with the fewest spaces that reach the rule."""
+    from frtools import quantize_f16, run_hip
+    evaluated, nearest = options.get("evaluated"), options.get("nearest")
+    s = settings(F.FR_DYNAMIC if evaluated or nearest else F.FR_LOOKUP,
+                 F.FR_FAST if nearest else F.FR_PRECISE, 15.0, options.get("radius", 1.9))
+    for size, cells in ((box, True), (box + 2, False)):
+        which = launchtools.choices([{**options, "box": size, "spaces": spaces}])[0][0]
+        assert (which == launchtools.CELLS) == cells
+        fft, sp, desc, table = problem(size, spaces, s, seed=size)
+        if options.get("half"):
+            h, scales, deq = quantize_f16(fft)
+            ov, ow, _ = run_oracle(s, deq, sp, table, size)
+            v, w, _ = run_hip(s, fft, sp, desc, table, size, half=(h, scales))
+        else:
+            ov, ow, _ = run_oracle(s, fft, sp, table, size)
+            v, w, _ = run_hip(s, fft, sp, desc, table, size,
+                              strategy=F.FR_FAST_MATH if options.get("fast") else F.FR_EXACT)
+        if options.get("half") or options.get("fast"):
+            assert rel_l2(v, ov) <= 1e-5 and rel_l2(w, ow) <= 1e-5
+        else:
+            assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()
+
+
+@pytest.mark.parametrize("n_table", [10239, 10240, 10747, 10752, 11776])
+@pytest.mark.parametrize("strategy", [F.FR_EXACT, F.FR_FAST_MATH])
+def test_tables_across_the_brick_kernels_limits(n_table, strategy):
+    """Tables on both sides of the staged and carried queues' limits, and the largest in LDS, in a
+    volume that bricks take."""
+    from frtools import run_hip
+    s = settings()
+    box, n = 124, 12
+    which = launchtools.choices([{"box": box, "spaces": n, "table": n_table,
+                                  "fast": int(strategy == F.FR_FAST_MATH)}])[0][0]
+    limit, kernel = ((10751, launchtools.CARRY) if strategy == F.FR_FAST_MATH
+                     else (10239, launchtools.STAGED))
+    assert which == (kernel if n_table <= limit else launchtools.PAIR)
+    fft, sp, _, _ = problem(box, n, s, seed=6)
+    desc = F.fr_desc(box // 2 + 1, box, n, box + 1, len(sp), n_table)
+    table = F.fill_blob_table(n_table, desc, s)
+    ov, ow, _ = run_oracle(s, fft, sp, table, box)
+    v, w, _ = run_hip(s, fft, sp, desc, table, box, strategy=strategy)
+    if strategy == F.FR_EXACT:
+        assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()
+    else:
+        assert rel_l2(v, ov) <= 1e-5 and rel_l2(w, ow) <= 1e-5
+
+
+@pytest.mark.parametrize("half", [False, True])
+def test_every_fast_math_candidate_on_bricks(half):
+    """The fast-math tuner's knob sets in a volume whose default kernel runs schedules."""
+    from frtools import quantize_f16, run_hip
+    s = settings()
+    box, n = 124, 30
+    fft, sp, desc, table = problem(box, n, s, seed=43)
+    h = None
+    if half:
+        *h, fft = quantize_f16(fft)
+    ov, ow, _ = run_oracle(s, fft, sp, table, box)
+    for p in F.tuning_candidates(F.FR_FAST_MATH):
+        v, w, _ = run_hip(s, fft, sp, desc, table, box, strategy=F.FR_FAST_MATH, half=h, sched=p)
+        assert rel_l2(v, ov) <= 1e-5 and rel_l2(w, ow) <= 1e-5, p.as_tuple()
+
+
+@pytest.mark.parametrize("typ", [F.FR_PRECISE, F.FR_FAST])
+@pytest.mark.parametrize("box,n", [(84, 160), (84, 59), (86, 160)])
+def test_shared_cells_without_a_table(box, n, typ):
+    """Shared central cells up to 85^3 where no table is read, and beyond, from 60 spaces on."""
+    from frtools import run_hip
+    s = settings(F.FR_DYNAMIC, typ, 15.0, 1.9)
+    fft, sp, desc, table = problem(box, n, s, seed=n)
+    ov, ow, _ = run_oracle(s, fft, sp, table, box)
+    v, w, _ = run_hip(s, fft, sp, desc, table, box)
+    assert v.tobytes() == ov.tobytes() and w.tobytes() == ow.tobytes()

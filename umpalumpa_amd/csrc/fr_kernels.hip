@@ -143,14 +143,13 @@ constexpr float kHalfEdge = 0.5f * (kEdge - 1);
 // |qz| <= r (1 + 1e-6) holds wherever the float qz * qz is at most the float r * r
 constexpr float kSlabMargin = 1.f + 1e-6f;
 
-// The slab test's bound for half width `r` where q.z steps (see slab_queue), |t22| up to kSteppedT22.
-// With u = 2^-24, v the volume's depth and t that limit: in either sum t22 pz rounds by at most
-// u t v / 2, and a sum by u times its size, which is r where the voxel passes and at most r + 7 t at
-// the up to eight levels that qz steps through: together less than u ((v + 56) t + 9 r), u = 6e-8.
-constexpr float kSteppedT22 = 2.f;
-__device__ __forceinline__ float slab_reach(float r, int v)
+// The slab test's bound for half width `r` and transforms of |t22| up to `t` (see slab_queue).  With
+// u = 2^-24 and v the volume's depth: in either sum t22 pz rounds by at most u t v / 2, and a sum by
+// u times its size, which is r where the voxel passes and at most r + 7 t at the up to eight levels
+// that qz steps through: together less than u ((v + 56) t + 9 r), u = 6e-8.
+__device__ __forceinline__ float slab_reach(float r, int v, float t)
 {
-  return r * kSlabMargin + 1e-7f * ((float)(v + 64) * kSteppedT22 + 10.f * r);
+  return r * kSlabMargin + 1e-7f * ((float)(v + 64) * t + 10.f * r);
 }
 
 // Brick of the work item and the lane's column of it.
@@ -302,6 +301,28 @@ __device__ __forceinline__ bool cull_space(const FrJob &a, const BrickCtx &b, in
          (dir >= 0) & (dir <= 2);
 }
 
+// The column's limit in the slab tests of 64 spaces, `t22` from the lane's: `usual` where each is at
+// most kUsualT22, as a rotation's is, else what the largest needs.  The five- and six-wide kernels
+// (!kHold), which spill where one more register is held, compute it anew, for 4,096 or no limit at
+// all.  (us, the start / held / anew: box 256, 1,000 slices, exact 1220 / 1224 / 1226, FP16 1039 /
+// 1038 / 1044; four FP16 jobs, bounded 1306 / 1306 / 1338; box 256, 500, exact in a batch, r 2.5 1448
+// / 1583 / 1461.)
+constexpr float kUsualT22 = 2.f;
+template <bool kHold>
+__device__ __forceinline__ float slab_limit(float usual, const FrJob &a, const BrickCtx &b, float r,
+                                            float t22)
+{
+  const bool large = __any(!(t22 <= kUsualT22));
+  if constexpr (kHold) {
+    if (!large) return usual;
+    for (int d = 32; d > 0; d >>= 1) t22 = fmaxf(t22, __shfl_xor(t22, d));
+    return b.colIn ? slab_reach(r, a.vz, fmaxf(t22, kUsualT22)) : -1.f;
+  } else {
+    const float t = !large ? kUsualT22 : __any(!(t22 <= 4096.f)) ? __builtin_inff() : 4096.f;
+    return b.colIn ? slab_reach(r, a.vz, t) : -1.f;
+  }
+}
+
 // Phase 1: the slab test of the column's nz voxels; the voxels that pass go to the wave's queue
 // behind `pending` entries (index k * 64 + lane, plus `tag`), their number is returned.
 // qz steps by t22 from level to level, one addition each where the reference's left-to-right sum
@@ -311,12 +332,10 @@ __device__ __forceinline__ bool cull_space(const FrJob &a, const BrickCtx &b, in
 // level, whose lane mask is the ballot.  (A column outside the volume compares against -1, which
 // nothing passes.)  Box 256, 1,000 slices: fast math 1100 -> 1094 us, exact 1236 -> 1231; box 1024,
 // D7, FP16 116.7 -> 114.9 ms; mixed batch 3710 -> 3671 us.
-// `stepped` (wave-uniform): every |t22| of the space's 64 is at most kSteppedT22, as a rotation's
-// is; transforms with larger ones, for which that bound would not hold, take the reference's sum.
 template <typename Scratch>
 __device__ __forceinline__ int slab_queue(Scratch &ws, const FrJob &a, const BrickCtx &b,
-                                          const umpa_traverse_space &sp, float lim, bool stepped,
-                                          int lane, int pending = 0, uint32_t tag = 0)
+                                          const umpa_traverse_space &sp, float lim, int lane,
+                                          int pending = 0, uint32_t tag = 0)
 {
   const int cyi = a.c.cMaxVolumeIndexYZ / 2;
   const float t20 = sp.transformInv[2][0], t21 = sp.transformInv[2][1],
@@ -324,18 +343,13 @@ __device__ __forceinline__ int slab_queue(Scratch &ws, const FrJob &a, const Bri
   const float cz = t20 * b.px + t21 * b.py;
   uint32_t entry = (uint32_t)lane | tag;
   int end = pending;
-  auto level = [&](float qz) {
+  float qz = cz + t22 * (float)(b.z0 - cyi);
+  for (int k = 0; k < b.nz; ++k, qz += t22) {
     const bool ok = !(fabsf(qz) > lim);
     const unsigned long long m = __ballot(ok);
     if (ok) ws.queue[lanes_below(m, (unsigned)end)] = (uint16_t)entry;
     end += __popcll(m);
     entry += 64;
-  };
-  if (stepped) {
-    float qz = cz + t22 * (float)(b.z0 - cyi);
-    for (int k = 0; k < b.nz; ++k, qz += t22) level(qz);
-  } else {
-    for (int k = 0; k < b.nz; ++k) level(cz + t22 * (float)(b.z0 + k - cyi));
   }
   return end - pending;
 }
@@ -413,12 +427,11 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
     const int cxi = c.cMaxVolumeIndexX / 2, cyi = c.cMaxVolumeIndexYZ / 2;
     // phase-1 filter on the slab coordinate: the reference's own test for blobs; for the
     // nearest-neighbour traversal the visited voxel lies within 1.5 of the plane
-    const float reach =
-      slab_reach(kMode == kModeNearest ? 1.6f : c.cBlobRadius, a.vz);
+    const float slab = kMode == kModeNearest ? 1.6f : c.cBlobRadius;
     if (heavy) __builtin_amdgcn_s_setprio(2);
     // the lane owns the z column (x, y, z0 .. z0 + depth - 1) of the brick
     const BrickCtx bk = make_brick(a, bo, lane);
-    const float lim = bk.colIn ? reach : -1.f;  // of the slab test
+    const float usual = bk.colIn ? slab_reach(slab, a.vz, kUsualT22) : -1.f;
     const int bz = bk.z0;
     const float ox = (float)(bo.x - cxi), oy = (float)(bo.y - cyi), oz = (float)(bz - cyi);
     bool loaded = false;  // the sums are read when the first space reaches the brick
@@ -430,7 +443,7 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
       unsigned long long mask = earlyCull
                                   ? __ballot(cull_space<true>(a, bk, base + lane, sEnd, t22))
                                   : __ballot(cull_space<false>(a, bk, base + lane, sEnd, t22));
-      const bool stepped = !__any(!(t22 <= kSteppedT22));
+      const float lim = slab_limit<kNB <= 4>(usual, a, bk, slab, t22);
       if (mask && !loaded) {
         load_brick(ws, a, bk, lane, split);
         loaded = true;
@@ -461,7 +474,7 @@ __global__ __launch_bounds__(64 * fr_waves(kMode, kHalf, kFastMath)) void fr_ins
 
         // phase 1: slab test of the column's nz voxels (nz is wave-uniform: shallow bricks
         // run fewer levels)
-        const int cnt = slab_queue(ws, a, bk, sp, lim, stepped, lane);
+        const int cnt = slab_queue(ws, a, bk, sp, lim, lane);
         if (cnt == 0) continue;
         wave_sync();
         const bool unit = sp.weight == 1.f;
@@ -647,11 +660,10 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fr_insert_carry_kernel(FrJob j
     const bool split = parts > 1;
     const int sBegin = split ? s0 + (int)((int64_t)(s1 - s0) * part / parts) : s0;
     const int sEnd = split ? s0 + (int)((int64_t)(s1 - s0) * (part + 1) / parts) : s1;
-    const float reach = slab_reach(a.c.cBlobRadius, a.vz);
     const int cxi = a.c.cMaxVolumeIndexX / 2, cyi = a.c.cMaxVolumeIndexYZ / 2;
     if (heavy) __builtin_amdgcn_s_setprio(2);
     const BrickCtx bk = make_brick(a, bo, lane);
-    const float lim = bk.colIn ? reach : -1.f;  // of the slab test
+    const float usual = bk.colIn ? slab_reach(a.c.cBlobRadius, a.vz, kUsualT22) : -1.f;
     const int bz = bk.z0;
     load_brick(ws, a, bk, lane, split);
     bool loaded = false;
@@ -668,7 +680,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fr_insert_carry_kernel(FrJob j
       unsigned long long mask = earlyCull
                                   ? __ballot(cull_space<true>(a, bk, base + lane, sEnd, t22))
                                   : __ballot(cull_space<false>(a, bk, base + lane, sEnd, t22));
-      const bool stepped = !__any(!(t22 <= kSteppedT22));
+      const float lim = slab_limit<true>(usual, a, bk, a.c.cBlobRadius, t22);
       if (mask && !loaded) {
         loaded = true;
       }
@@ -700,7 +712,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fr_insert_carry_kernel(FrJob j
         const bool ins = brick_inside(bk, slots[slot].rec, cxi, cyi);
         if (lane == 0) slots[slot].inside = ins ? 1 : 0;
         const int cnt =
-          slab_queue(ws, a, bk, slots[slot].rec, lim, stepped, lane, pending, (uint32_t)slot << 9);
+          slab_queue(ws, a, bk, slots[slot].rec, lim, lane, pending, (uint32_t)slot << 9);
         if (cnt == 0) continue;  // the slot stays free for the next space
         pending += cnt;
         ++pendSpaces;
@@ -815,7 +827,6 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
     (void *)a.fft, 0, (int)((uint32_t)a.nProj * sliceBytes), kBufferConfig);
   const umpa_fr_constants &c = a.c;
   const int cxi = c.cMaxVolumeIndexX / 2, cyi = c.cMaxVolumeIndexYZ / 2;
-  const float reach = slab_reach(c.cBlobRadius, a.vz);
 
   const int sBegin = a.spaceBegin, sEnd = a.spaceEnd;
   if (sBegin >= sEnd) return;
@@ -837,7 +848,7 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
     const bool heavy = (bo.w >> 4) & 1;
     if (heavy) __builtin_amdgcn_s_setprio(2);
     const BrickCtx bk = make_brick(a, bo, lane);
-    const float lim = bk.colIn ? reach : -1.f;  // of the slab test
+    const float usual = bk.colIn ? slab_reach(c.cBlobRadius, a.vz, kUsualT22) : -1.f;
     const int bz = bk.z0;
     const float ox = (float)(bo.x - cxi), oy = (float)(bo.y - cyi), oz = (float)(bz - cyi);
     bool loaded = false;  // the sums are read when the first space reaches the brick
@@ -850,7 +861,7 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
       unsigned long long mask = earlyCull
                                   ? __ballot(cull_space<true>(a, bk, base + lane, sEnd, t22))
                                   : __ballot(cull_space<false>(a, bk, base + lane, sEnd, t22));
-      const bool stepped = !__any(!(t22 <= kSteppedT22));
+      const float lim = slab_limit<true>(usual, a, bk, c.cBlobRadius, t22);
       if (mask && !loaded) {
         load_brick(ws, a, bk, lane, false);
         loaded = true;
@@ -863,7 +874,7 @@ __global__ __launch_bounds__(64 * kStagedWaves) void fr_insert_staged_kernel(FrJ
         const uint32_t sliceOff =
           (uint32_t)__builtin_amdgcn_readfirstlane(sp.projectionIndex) * sliceBytes;
         // phase 1: the slab test, as in fr_insert_kernel
-        const int cnt = slab_queue(ws, a, bk, sp, lim, stepped, lane);
+        const int cnt = slab_queue(ws, a, bk, sp, lim, lane);
         if (cnt == 0) continue;
         wave_sync();
         const bool inside = brick_inside(bk, sp, cxi, cyi);

@@ -351,17 +351,20 @@ __device__ __forceinline__ bool gather_box(const FrJob &a, int nTable,
   // at box 256 under the exact strategy).
   constexpr int kVecs = (kNB * kPix + 15) / 16;          // 16-byte loads per row
   // Six FP32 columns go row by row: two rows' pixels and weights spilled up to 74 registers (r 2.8,
-  // 500 slices, box 256: exact 5226 -> 1999 us, fast math 1463 -> 1438; r 3.6 13510 -> 8533), while
+  // 500 slices, box 256: exact 5226 -> 1962 us, fast math 1463 -> 1441; r 3.6 13510 -> 8687), while
   // five columns want two (r 2.5, exact 1431 us, 1576 row by row).
   constexpr int kGroup =
     kRows ? kRows : kVecs == 1 ? kNB : kVecs == 2 ? (kNB <= 4 ? kNB : 3) : kNB == 5 ? 2 : 1;
   // wider boxes under the exact strategy mask skipped pixels, whatever their value
   constexpr bool kMask = kNB > 4 && !(kFastMath && kMode == kModeLookup && kTableLds);
   constexpr bool kSkipOutside = kChunk && !kShift;
-#pragma unroll
-  for (int g = 0; g < kNB; g += kGroup) {
-    Pixel<kHalf> px[kGroup][kNB];
-    float wr[kGroup][kNB];
+  // The exact brick kernels' registers (12 wavefronts a CU) hold the next row's pixels beside the one
+  // that is summed, so that a space's chain waits for one row, not six (r 2.8, us: a batch of one box
+  // 176, 1,000 slices 3832 -> 2961, box 256, 500 slices 1962 -> 1661; fast math, with 16, spills: box
+  // 256, 500 1441 -> 1486).
+  constexpr bool kAhead = kGroup == 1 && kNB == 6 && kRows == 0 && !kFastMath && kTableLds;
+  Pixel<kHalf> px[kAhead ? 2 : 1][kGroup][kNB];
+  auto load_group = [&](int g, Pixel<kHalf> (&to)[kGroup][kNB]) {
 #pragma unroll
     for (int i = 0; i < kGroup; ++i) {
       if (g + i >= kNB) continue;
@@ -369,7 +372,18 @@ __device__ __forceinline__ bool gather_box(const FrJob &a, int nTable,
       // from past the slice end instead of its pixels, a quarter of the rows at r = 1.9
       constexpr bool kSkipRows = kFastMath && !kHalf;
       const bool read = kSkipRows ? yz[g + i] <= r2 : !kSkipOutside || yz[g + i] < inf;
-      load_row<kHalf, kNB>(rsrc, read ? base + (g + i) * rowStride : kOutOfRange, px[i]);
+      load_row<kHalf, kNB>(rsrc, read ? base + (g + i) * rowStride : kOutOfRange, to[i]);
+    }
+  };
+  if constexpr (kAhead) load_group(0, px[0]);
+#pragma unroll
+  for (int g = 0; g < kNB; g += kGroup) {
+    const int slot = kAhead ? g & 1 : 0;
+    float wr[kGroup][kNB];
+    if constexpr (kAhead) {
+      load_group(g + 1, px[1 - slot]);
+    } else {
+      load_group(g, px[0]);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -387,7 +401,7 @@ __device__ __forceinline__ bool gather_box(const FrJob &a, int nTable,
       if (g + i >= kNB) continue;
 #pragma unroll
       for (int jj = 0; jj < kNB; ++jj) {
-        float fre = px[i][jj].re(), fim = px[i][jj].im();
+        float fre = px[slot][i][jj].re(), fim = px[slot][i][jj].im();
         if constexpr (kMask) {
           const bool in = xd2[jj] + yz[g + i] <= r2;
           fre = in ? fre : 0.f;

@@ -136,8 +136,7 @@ static int fr_check_init(const umpa_fr_desc &desc, const umpa_fr_settings &s)
   return UMPA_OK;
 }
 
-// Widest blob footprint in pixels: floor(2r) + 1 (plus a margin for rounding at the edge),
-// clamped to the unrolled widths 3..6; wider footprints take the kernel's generic path.
+// Width of the kernels' candidate box in pixels, 3..6; wider footprints take the generic path.
 static int fr_footprint(const umpa_fr_settings &s) { return umpa::host::footprint(s); }
 
 extern "C" {
@@ -442,8 +441,8 @@ int umpa_fr_execute_noalloc(int device, void *stream, const umpa_fr_desc *desc,
     fr_variant_for(*s, fr_footprint(*s), strategy, half, false, umpa::host::SchedParams());
   if (half && v.mode != umpa::kModeLookup) return UMPA_ERR_UNSUPPORTED;
   try {
-    // the schedule a handle would build at Init (default knobs): it must fit the static
-    // scratch, which holds volumes up to 513^3
+    // every brick under the default knobs (a handle also scales their depths by volume and takes the
+    // core as cells): it must fit the static scratch, which holds volumes up to 513^3
     const auto bricks = umpa::host::make_brick_schedule(
       (int)desc->volume.x, (int)desc->volume.y, (int)desc->volume.z, v.fastMath,
       umpa::host::SchedParams());

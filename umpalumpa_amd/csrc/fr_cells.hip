@@ -26,7 +26,7 @@
 // fr_kernels.hip).  What bounds it is the chain of steps, about 1.5 us each, and between VALU
 // busy 0.35 (box 64, 500 spaces) and 0.8.  us per pass, bricks -> cells: box 32, 16 slices
 // 24.7 -> 15.3; box 64, 500, fast math 510 -> 120; box 100, 251, C4, r 1.5, exact 1004 -> 299;
-// box 128, 300, blob evaluated 831 -> 407.
+// box 120, 400, blob evaluated 1224 -> 366.
 #include "fr_cell.hpp"
 
 namespace umpa {
@@ -94,7 +94,8 @@ __global__ __launch_bounds__(kCellThreads, 4) void fr_insert_cell_kernel(FrJob a
 {
   constexpr bool kTableLds = kMode == kModeLookup;
   constexpr int kPix = kHalf ? 4 : 8;
-  // rows of the gather in flight: what 128 registers hold beside two spaces' records
+  // rows of the gather in flight: what 128 registers hold beside two spaces' records (six columns:
+  // two FP32 rows spilled up to 90; box 112, 400 slices, r 2.8, exact 803 -> 464 us with one)
   constexpr int kRows = kHalf ? (kNB <= 4 ? kNB : 3) : kNB <= 3 ? 3 : kNB <= 5 ? 2 : 1;
   extern __shared__ float s_table[];
   __shared__ __align__(16) float s_part[kShared ? 2 : 1][kCellWaves][3 * 64];

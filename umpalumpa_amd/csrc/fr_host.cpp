@@ -234,7 +234,8 @@ namespace {
 // only if both its outermost pixels lie at distance r to the last bit; the 3- and 5-wide boxes
 // test for that and leave such voxels to the general loop, so 2r columns do (9 candidates
 // instead of 16 at r = 1.5, 25 instead of 36 at r = 2.5: box 384, 256 FP16 slices under D2 at
-// r = 2.5, 4.88 -> 3.98 ms; box 100, 251 slices under C4 at r = 1.5, 1.04 -> 0.99 ms).
+// r = 2.5, 4.88 -> 3.98 ms; box 100, 251 slices under C4 at r = 1.5, 1.04 -> 0.99 ms).  Where 2r is
+// even (4 columns would do at r = 2) the box has no such test: it keeps the column more.
 int box_columns(const umpa_fr_settings &s)
 {
   const double d = 2.0 * (double)s.blobRadius;

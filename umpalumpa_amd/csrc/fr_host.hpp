@@ -71,8 +71,9 @@ std::vector<BrickCand> brick_candidates(int vx, int vy, int vz, float depthScale
 float core_radius(int vx, int vy, int vz);
 std::vector<int> core_cells(int vx, int vy, int vz, float core);
 
-// Scale of the brick depths' radii: of a plain operation's launches of up to `spaces` spaces, by
-// the blob (of the settings) and whether heavy bricks are split; of a volume in a batch's launch.
+// Scale of the brick depths' radii: of a plain operation's launches of up to `spaces` spaces (what
+// Init was told, which also decides shared cells: launches of fewer run the same schedule), by the
+// blob (of the settings) and whether heavy bricks are split; of a volume in a batch's launch.
 float plain_depth_scale(int vx, int vy, int vz, uint64_t spaces, const umpa_fr_settings &s,
                         bool split);
 float batch_depth_scale(int vx, int vy, int vz, bool bounded);

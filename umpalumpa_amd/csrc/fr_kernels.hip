@@ -10,8 +10,8 @@
 // scheduled.
 //
 // Per (brick, space) pair the wave
-//   1. tests the reference's slab condition (q.z^2 <= r^2) for its voxels, 4 VALU each, and
-//      compacts the voxels that pass into its LDS queue;
+//   1. tests the reference's slab condition (q.z^2 <= r^2) for its voxels, an addition and a
+//      compare each, and compacts the voxels that pass into its LDS queue;
 //   2. runs the rest of the reference predicate and the gather over the queue with full lanes:
 //      a branch-free NB x NB candidate loop over whole pixel rows in which a candidate the
 //      reference skips reads the zero entry appended to the LDS blob table, adding +-0 (finite
@@ -665,6 +665,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fr_insert_carry_kernel(FrJob j
     const BrickCtx bk = make_brick(a, bo, lane);
     const float usual = bk.colIn ? slab_reach(a.c.cBlobRadius, a.vz, kUsualT22) : -1.f;
     const int bz = bk.z0;
+    // (read before the cull, reached or not; only a brick that a space reaches is written back)
     load_brick(ws, a, bk, lane, split);
     bool loaded = false;
     const uint32_t sliceBytes = (uint32_t)(a.sliceElems * kPix);

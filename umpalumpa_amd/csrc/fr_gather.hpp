@@ -363,27 +363,29 @@ __device__ __forceinline__ bool gather_box(const FrJob &a, int nTable,
   // 176, 1,000 slices 3832 -> 2961, box 256, 500 slices 1962 -> 1661; fast math, with 16, spills: box
   // 256, 500 1441 -> 1486).
   constexpr bool kAhead = kGroup == 1 && kNB == 6 && kRows == 0 && !kFastMath && kTableLds;
-  Pixel<kHalf> px[kAhead ? 2 : 1][kGroup][kNB];
-  auto load_group = [&](int g, Pixel<kHalf> (&to)[kGroup][kNB]) {
-#pragma unroll
-    for (int i = 0; i < kGroup; ++i) {
-      if (g + i >= kNB) continue;
-      // fast-math FP32: a row wholly outside the blob (every candidate weighs 0) reads zeros
-      // from past the slice end instead of its pixels, a quarter of the rows at r = 1.9
-      constexpr bool kSkipRows = kFastMath && !kHalf;
-      const bool read = kSkipRows ? yz[g + i] <= r2 : !kSkipOutside || yz[g + i] < inf;
-      load_row<kHalf, kNB>(rsrc, read ? base + (g + i) * rowStride : kOutOfRange, to[i]);
-    }
+  // fast-math FP32: a row wholly outside the blob (every candidate weighs 0) reads zeros from past
+  // the slice end instead of its pixels, a quarter of the rows at r = 1.9
+  constexpr bool kSkipRows = kFastMath && !kHalf;
+  auto row_offset = [&](int k) {
+    const bool read = kSkipRows ? yz[k] <= r2 : !kSkipOutside || yz[k] < inf;
+    return read ? base + k * rowStride : kOutOfRange;
   };
-  if constexpr (kAhead) load_group(0, px[0]);
+  Pixel<kHalf> ahead[kNB];
+  if constexpr (kAhead) load_row<kHalf, kNB>(rsrc, row_offset(0), ahead);
 #pragma unroll
   for (int g = 0; g < kNB; g += kGroup) {
-    const int slot = kAhead ? g & 1 : 0;
+    Pixel<kHalf> px[kGroup][kNB];
     float wr[kGroup][kNB];
     if constexpr (kAhead) {
-      load_group(g + 1, px[1 - slot]);
+#pragma unroll
+      for (int jj = 0; jj < kNB; ++jj) px[0][jj] = ahead[jj];
+      if (g + 1 < kNB) load_row<kHalf, kNB>(rsrc, row_offset(g + 1), ahead);
     } else {
-      load_group(g, px[0]);
+#pragma unroll
+      for (int i = 0; i < kGroup; ++i) {
+        if (g + i >= kNB) continue;
+        load_row<kHalf, kNB>(rsrc, row_offset(g + i), px[i]);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -401,7 +403,7 @@ __device__ __forceinline__ bool gather_box(const FrJob &a, int nTable,
       if (g + i >= kNB) continue;
 #pragma unroll
       for (int jj = 0; jj < kNB; ++jj) {
-        float fre = px[slot][i][jj].re(), fim = px[slot][i][jj].im();
+        float fre = px[i][jj].re(), fim = px[i][jj].im();
         if constexpr (kMask) {
           const bool in = xd2[jj] + yz[g + i] <= r2;
           fre = in ? fre : 0.f;

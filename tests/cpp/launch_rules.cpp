@@ -6,6 +6,7 @@
 //   op_key key=value ...        the key of an operation's tuning result: Init told of `init` spaces
 //   batch_key key=value ...     ... of a batch of one job
 //   core key=value ...          cells of a volume's core and bricks beside it (exact launches)
+//   depth key=value ...         the depth scale of a batch's launch and of a plain operation's
 #include <dlfcn.h>
 
 #include <cstdio>
@@ -128,6 +129,15 @@ void core()
               umpa::host::make_brick_schedule(side, side, side, false, {}, radius).size());
 }
 
+void depth()
+{
+  const int side = (int)arg("box") + 1;
+  const bool split = arg("fast") != 0;
+  std::printf("%g %g\n",
+              umpa::host::batch_depth_scale(side, side, side, arg("bounded") != 0, split),
+              umpa::host::plain_depth_scale(side, side, side, 1000, settings(), split));
+}
+
 }  // namespace
 
 int main()
@@ -148,6 +158,7 @@ int main()
     else if (command == "op_key") op_key();
     else if (command == "batch_key") batch_key();
     else if (command == "core") core();
+    else if (command == "depth") depth();
     else return 2;
   }
   return 0;

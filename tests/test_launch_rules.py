@@ -125,3 +125,14 @@ def test_lines_of_the_small_problem_kernel(options, box, spaces):
         others += [{**case, "table": 11777}, {**case, "tableGlobal": 1}]
     got = [c[0] for c in L.choices([case, *others])]
     assert got[0] == L.CELLS and L.CELLS not in got[1:]
+
+
+@pytest.mark.parametrize("fast", [0, 1])
+def test_depth_scale_of_large_volumes_in_batches(fast):
+    """Bricks of a batch's volumes above 165^3 are as thick as a plain operation's, whose heaviest
+    brick a launch waits for, too; a bounded launch's are thicker."""
+    for box in (166, 176, 208, 210, 256, 400):
+        (batch, plain), (bounded, _) = L.ask("depth", [{"box": box, "fast": fast},
+                                                       {"box": box, "fast": fast, "bounded": 1}])
+        assert batch == plain and float(bounded) == 0.5
+    assert L.ask("depth", [{"box": 160, "fast": fast}])[0][0] == "1"

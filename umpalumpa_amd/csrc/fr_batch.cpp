@@ -217,7 +217,8 @@ void build_step(umpa_fr_batch *b, const std::vector<JobInfo> &infos,
       recs.push_back(rec);
       const float depth =
         sp.depthScale *
-        umpa::host::batch_depth_scale(rec.vx, rec.vy, rec.vz, b->waveItems > 0);
+        umpa::host::batch_depth_scale(rec.vx, rec.vy, rec.vz, b->waveItems > 0,
+                                      first.v.fastMath);
       work.push_back({ &b->candidates(rec.vx, rec.vy, rec.vz, depth), (int)k,
                        (double)(s1 - s0) });
     }

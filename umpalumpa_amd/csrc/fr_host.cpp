@@ -287,6 +287,15 @@ bool at_most_cube(int vx, int vy, int vz, int64_t n) { return (int64_t)vx * vy *
 
 }  // namespace
 
+namespace {
+
+float large_depth_scale(int vx, int vy, int vz, bool split)
+{
+  return split && !at_most_cube(vx, vy, vz, 209) ? 0.5f : 0.7f;
+}
+
+}  // namespace
+
 // Thin bricks even out the work but fill fewer of a gather's lanes and cost a set-up each.  Volumes
 // up to 165^3 have few bricks for 4,096 wavefronts and want them thinner farther out, if there are
 // enough spaces to pay for the set-up (us at scale 1 / 1.4: box 128, 1,500 slices exact 661 / 579,
@@ -304,17 +313,21 @@ float plain_depth_scale(int vx, int vy, int vz, uint64_t spaces, const umpa_fr_s
   const bool evaluated = !nearest && s.interpolation == UMPA_FR_DYNAMIC;
   if (at_most_cube(vx, vy, vz, 165))
     return !nearest && (evaluated || spaces >= 250) ? 1.4f : 1.f;
-  return split && !at_most_cube(vx, vy, vz, 209) ? 0.5f : 0.7f;
+  return large_depth_scale(vx, vy, vz, split);
 }
 
 // A batch's volumes fill the GPU together, so small ones need no thinner bricks (seven FP16 jobs of
 // boxes 64 to 320 at 1 / 1.4 for boxes up to 165 and 0.5 for the others: 3881 / 3974 us; all at 1:
-// 3930; the small ones at 0.7, 4150, lose a launch's last chunks, where they are alone).  Bounded
+// 3930; the small ones at 0.7, 4150, lose a launch's last chunks, where they are alone); large ones
+// go by the plain rule, since a launch of few jobs waits for its heaviest brick (at 0.5 / 0.7, one
+// job of 1,000 FP32 slices: exact, box 176 1706 / 1414, 256 1778 / 1522, r 3.6 176 12330 / 8871; fast
+// math 176 647 / 558, 192 676 / 648, 224 847 / 855, 256 1085 / 1096).  Bounded
 // launches, whose workgroups turn over, want fewer items (a tick of four jobs, boxes 96 to 256, at
 // 1 / 0.7 / 0.5: FP16 1578 / 1512 / 1463 us, exact 2221 / 2096 / 2103).
-float batch_depth_scale(int vx, int vy, int vz, bool bounded)
+float batch_depth_scale(int vx, int vy, int vz, bool bounded, bool split)
 {
-  return !bounded && at_most_cube(vx, vy, vz, 165) ? 1.f : 0.5f;
+  if (bounded) return 0.5f;
+  return at_most_cube(vx, vy, vz, 165) ? 1.f : large_depth_scale(vx, vy, vz, split);
 }
 
 std::vector<BrickCand> brick_candidates(int vx, int vy, int vz, float depthScale, float core)

@@ -73,10 +73,11 @@ std::vector<int> core_cells(int vx, int vy, int vz, float core);
 
 // Scale of the brick depths' radii: of a plain operation's launches of up to `spaces` spaces (what
 // Init was told, which also decides shared cells: launches of fewer run the same schedule), by the
-// blob (of the settings) and whether heavy bricks are split; of a volume in a batch's launch.
+// blob (of the settings) and whether heavy bricks are split; of a volume in a batch's launch, by
+// whether that is bounded and heavy bricks are split.
 float plain_depth_scale(int vx, int vy, int vz, uint64_t spaces, const umpa_fr_settings &s,
                         bool split);
-float batch_depth_scale(int vx, int vy, int vz, bool bounded);
+float batch_depth_scale(int vx, int vy, int vz, bool bounded, bool split);
 
 // A volume's bricks sorted by estimated cost (heaviest first, ties in brick order) and the
 // costs' sum: what make_schedule needs of a volume, built once per volume shape.

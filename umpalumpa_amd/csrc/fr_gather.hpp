@@ -344,8 +344,9 @@ __device__ __forceinline__ bool gather_box(const FrJob &a, int nTable,
   // values they add +-0, which changes no running sum (the sums start at +0 and are never -0):
   // the result equals the reference's skip-the-pixel loop bit for bit.
   //
-  // The rows go in groups of kGroup (kRows, or what the brick kernels' registers hold): all of a group's pixel loads are issued, then its table
-  // reads, then its sums, each in a scheduling region of its own.  Left to itself this compiler
+  // The rows go in groups of kGroup (kRows, or what the brick kernels' registers hold): all of a
+  // group's pixel loads are issued, then its table reads, then its sums, each in a scheduling region
+  // of its own.  Left to itself this compiler
   // orders the same code by what else the kernel holds in registers: a change elsewhere could
   // make it wait for every row before loading the next (1.42 -> 1.84 ms per 1,000-slice chunk
   // at box 256 under the exact strategy).

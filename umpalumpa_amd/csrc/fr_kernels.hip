@@ -304,7 +304,7 @@ __device__ __forceinline__ bool cull_space(const FrJob &a, const BrickCtx &b, in
 // The column's limit in the slab tests of 64 spaces, `t22` from the lane's: `usual` where each is at
 // most kUsualT22, as a rotation's is, else what the largest needs.  The five- and six-wide kernels
 // (!kHold), which spill where one more register is held, compute it anew, for 4,096 or no limit at
-// all.  (us, the start / held / anew: box 256, 1,000 slices, exact 1220 / 1224 / 1226, FP16 1039 /
+// all.  (us, kUsualT22's only / held / anew: box 256, 1,000 slices, exact 1220 / 1224 / 1226, FP16 1039 /
 // 1038 / 1044; four FP16 jobs, bounded 1306 / 1306 / 1338; box 256, 500, exact in a batch, r 2.5 1448
 // / 1583 / 1461.)
 constexpr float kUsualT22 = 2.f;
